@@ -116,7 +116,7 @@ def measure_traffic(precision="fp64", timeout_s=240):
         for fn in files:
             with open(fn) as f:
                 for row in csv.DictReader(f):
-                    if "rhs_pencil_kernel" in row.get("Kernel_Name", "") and row.get("Counter_Name") == counter:
+                    if "rhs_march_kernel" in row.get("Kernel_Name", "") and row.get("Counter_Name") == counter:
                         kib += float(row["Counter_Value"])
         shutil.rmtree(out, ignore_errors=True)
         if kib <= 0:
@@ -231,7 +231,7 @@ def measure_group(case, args, specs, rounds=5, traffic=None):
                 "bound": "hbm", "achieved": round(achieved, 2), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                 "frac": round(achieved / HBM_PEAK_GBS, 5), "traffic": tr,
                 "traffic_bytes_per_cell_stage": round(tr / case.n_cells, 1) if tr else None,
-                "kernel": "rhs_pencil_kernel (LDS-staged RHS, one launch per face direction)",
+                "kernel": "rhs_march_kernel (all face directions in one launch, marching along k)",
                 "kernel_avg_ms_per_stage": round(rhs_stage_s * 1e3, 4),
                 "launches_per_stage": round(rhs_n / stages, 2), "bytes_per_cell_stage": round(bpc, 2)}
             # the same kernel against the vector ALU: FP64 / FP32 flops per stage

@@ -60,6 +60,10 @@ void fill_thermo(SpeciesT<T> &s) {
       for (int k = 0; k < 5; ++k) v[kThCp + 5 * g + k] = s.cpc[g][l][k];
       for (int k = 0; k < 6; ++k) v[kThH + 6 * g + k] = s.hc[g][l][k];
     }
+    for (int g = 0; g < 2; ++g) {
+      for (int k = 0; k < 6; ++k) s.mix[g][l].v[k] = s.hc[g][l][k];
+      s.mix[g][l].v[6] = s.inv_mw[l];
+    }
     v[kThTmid] = s.t_mid[l];
     v[kThTlow] = s.t_low[l];
     v[kThHtlow] = s.h_tlow[l];
@@ -217,15 +221,80 @@ int build_tables(cfx_ctx *ctx) {
       (rc = upload_table(ctx, ctx->t_dt, dtc)) || (rc = upload_table(ctx, ctx->t_last, last)) ||
       (rc = upload_table(ctx, ctx->t_res, res)) || (rc = upload_table(ctx, ctx->t_tile, til)))
     return rc;
-  for (int d = 0; d < ctx->dim; ++d)
-    for (int v = 0; v < rhs_variants(ctx->dim); ++v) {
+  for (int d = 0; d < 2 && ctx->dim == 2; ++d)
+    for (int v = 0; v < kNVar2; ++v) {
       std::vector<int> tiles(nb);
       for (int b = 0; b < nb; ++b) {
         const int m[3] = {ctx->hb[b].mx, ctx->hb[b].my, ctx->hb[b].mz};
-        tiles[b] = pencil_tiles(m, d, rhs_tile_shape(ctx->dim, d, v));
+        tiles[b] = pencil_tiles(m, d, kTiles2[d][v]);
       }
       if ((rc = upload_table(ctx, ctx->t_rhs[d][v], tiles))) return rc;
     }
+  return 0;
+}
+
+// The marching RHS of a 3-D context: the planes per workgroup of every variant
+// and its workgroup prefix.
+int plan_march(cfx_ctx *ctx) {
+  if (ctx->dim != 3) return 0;
+  const MarchTile t = ctx->mixed ? kMarch32 : kMarch64;
+  const OccFn occ = ctx->mixed ? g_kernels32[ctx->ns].march_occ : g_kernels64[ctx->ns].march_occ;
+  const double word = ctx->mixed ? 4 : 8;
+  const size_t nb = ctx->hb.size();
+  std::vector<int> groups(nb);
+  int top = 0;
+  for (const HostBlock &H : ctx->hb) {
+    ctx->march_big = ctx->march_big || 9.0 * word * (double)H.np >= 4294967296.0;
+    top = std::max(top, H.mz);
+  }
+  auto split = [&](int chunk) {
+    for (size_t b = 0; b < nb; ++b) {
+      const int m[3] = {ctx->hb[b].mx, ctx->hb[b].my, ctx->hb[b].mz};
+      groups[b] = march_groups(m, t, chunk);
+    }
+  };
+  // Variant 0: a chunk of n planes costs about n + kFill planes' time (the
+  // first planes' loads, the last z faces; 256x128x128 with 9 species in
+  // chunks of 8 and of 128 or 64 planes: 1.2 in FP64, 1.4 in FP32).  The
+  // workgroups go to the 8 XCDs in contiguous runs of equal count; a launch
+  // lasts as long as its fullest XCD: whole rounds of one block, an average
+  // load and half of the longest chunk of many (27 blocks of 33..90 points:
+  // planned without the runs 6.98 ms per step in FP64, with them 6.24).
+  constexpr double kFill = 1.3;
+  const double slots = std::max(1.0, (double)std::max(1, occ()) * ctx->n_cu / 8);
+  double best = 1e300;
+  int planned = top;
+  for (int parts = 1; parts <= top; ++parts) {
+    const int chunk = chunks(top, parts);
+    if (parts > 1 && chunk == chunks(top, parts - 1)) continue;
+    split(chunk);
+    long long total = 0;
+    for (size_t b = 0; b < nb; ++b) total += groups[b];
+    const long long run = (total + 7) / 8;
+    double est = 0;
+    size_t b = 0;
+    long long left = groups[0];
+    for (int x = 0; x < 8; ++x) {
+      double work = 0, longest = 0, n = 0;
+      for (long long room = run; room > 0 && b < nb;) {
+        const long long k = std::min(room, left);
+        const double len = chunks(ctx->hb[b].mz, chunks(ctx->hb[b].mz, chunk)) + kFill;
+        work += (double)k * len;
+        n += (double)k;
+        longest = std::max(longest, len);
+        room -= k;
+        left -= k;
+        if (left == 0 && ++b < nb) left = groups[b];
+      }
+      est = std::max(est, nb == 1 ? std::ceil(n / slots) * longest : std::max(longest, work / slots + 0.5 * longest));
+    }
+    if (est < best) best = est, planned = chunk;
+  }
+  for (int v = 0; v < kNVar3; ++v) {
+    ctx->march_chunk[v] = v == 0 ? planned : kMarchChunk[v];
+    split(ctx->march_chunk[v]);
+    if (int rc = upload_table(ctx, ctx->t_march[v], groups)) return rc;
+  }
   return 0;
 }
 
@@ -472,10 +541,10 @@ int run_levels(cfx_ctx *ctx, const Schedule &sc, int l0, int l1) {
 }
 
 // ------------------------------------------------------------ step parts ---
+// 2-D: one face direction
 int rhs_dir(cfx_ctx *ctx, int d, const Batch &b, int accumulate) {
   const int v = ctx->rhs_var[d];
-  const RhsEntry &e = ctx->mixed ? (ctx->dim == 3 ? g_kernels32[ctx->ns].rhs3[d][v] : g_kernels32[ctx->ns].rhs2[d][v])
-                                 : (ctx->dim == 3 ? g_kernels64[ctx->ns].rhs3[d][v] : g_kernels64[ctx->ns].rhs2[d][v]);
+  const RhsEntry &e = ctx->mixed ? g_kernels32[ctx->ns].rhs2[d][v] : g_kernels64[ctx->ns].rhs2[d][v];
   const int padded = (b.total + 7) / 8 * 8;
   int grid = padded;
   const int occ = ctx->occ[ctx->mixed ? 1 : 0][d][v];
@@ -483,14 +552,30 @@ int rhs_dir(cfx_ctx *ctx, int d, const Batch &b, int accumulate) {
   return ctx->timed_launch(K_RHS, [&] { return e.launch(b, grid, ctx->sp_dev, ctx->S, accumulate, ctx->stream); });
 }
 
+// 3-D: all face directions; the march runs along k, so the variant of that direction counts
+int rhs_march(cfx_ctx *ctx, int blk) {
+  const int v = ctx->rhs_var[2];
+  const MarchFn fn = ctx->mixed ? g_kernels32[ctx->ns].march : g_kernels64[ctx->ns].march;
+  const Batch b = blk < 0 ? ctx->all(ctx->t_march[v]) : ctx->one(ctx->t_march[v], blk);
+  return ctx->timed_launch(K_RHS, [&] {
+    return fn(b, ctx->march_chunk[v], ctx->march_big ? 1 : 0, ctx->sp_dev, ctx->S, ctx->stream);
+  });
+}
+
 int do_rhs(cfx_ctx *ctx, int blk) {
-  if (blk < 0 && ctx->batched) {
-    for (int d = 0; d < ctx->dim; ++d) CFX_TRY(rhs_dir(ctx, d, ctx->all(ctx->t_rhs[d][ctx->rhs_var[d]]), d > 0));
+  auto run = [&](int b) {  // b < 0: every block in one launch
+    if (ctx->dim == 3) return rhs_march(ctx, b);
+    for (int d = 0; d < 2; ++d) {
+      const Table &t = ctx->t_rhs[d][ctx->rhs_var[d]];
+      if (int rc = rhs_dir(ctx, d, b < 0 ? ctx->all(t) : ctx->one(t, b), d > 0)) return rc;
+    }
+    return 0;
+  };
+  if (blk >= 0 || ctx->batched) {
+    CFX_TRY(run(blk));
     return 0;
   }
-  const int b0 = blk < 0 ? 0 : blk, b1 = blk < 0 ? (int)ctx->views.size() : blk + 1;
-  for (int b = b0; b < b1; ++b)
-    for (int d = 0; d < ctx->dim; ++d) CFX_TRY(rhs_dir(ctx, d, ctx->one(ctx->t_rhs[d][ctx->rhs_var[d]], b), d > 0));
+  for (int b = 0; b < (int)ctx->views.size(); ++b) CFX_TRY(run(b));
   return 0;
 }
 
@@ -845,15 +930,6 @@ int cfx_create(const cfx_params *params, const cfx_species *species, const cfx_b
   S.lusgs = params->lusgs ? 1 : 0;
   S.omega = params->lusgs_omega > 0 ? params->lusgs_omega : 1.0;
   ctx->rk = S.rk;
-  // default RHS tiles of a 3-D context: shapes among the fastest the
-  // autotuner measures on MI355X for the 256x128x128 9-species block (FP64:
-  // x 32x4x2, y 8x32x1 and z 8x32x1 with c fastest; FP32: x 32x4x2 at 4
-  // waves, y 8x32x1, z 8x64x1 (512 threads) with c fastest); cfx_autotune
-  // re-picks per context
-  if (ctx->dim == 3) {
-    const int d64[3] = {5, 1, 1}, d32[3] = {5, 2, 3};
-    for (int d = 0; d < 3; ++d) ctx->rhs_var[d] = ctx->mixed ? d32[d] : d64[d];
-  }
   ctx->lusgs = S.lusgs != 0;
   if (ctx->lusgs && (S.rk != 1 || ctx->mixed)) {
     ctx->err = "the LU-SGS step needs rk_stages 1 (local time step) and FP64";
@@ -976,16 +1052,13 @@ int cfx_create(const cfx_params *params, const cfx_species *species, const cfx_b
     (void)hipGetDevice(&dev);
     if (hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && ncu > 0)
       ctx->n_cu = ncu;
-    for (int f32 = 0; f32 < 2; ++f32) {
-      if (f32 && !ctx->mixed) continue;
-      for (int d = 0; d < ctx->dim; ++d)
-        for (int v = 0; v < rhs_variants(ctx->dim); ++v) {
-          const RhsEntry &e = f32 ? (ctx->dim == 3 ? g_kernels32[ctx->ns].rhs3[d][v] : g_kernels32[ctx->ns].rhs2[d][v])
-                                  : (ctx->dim == 3 ? g_kernels64[ctx->ns].rhs3[d][v] : g_kernels64[ctx->ns].rhs2[d][v]);
-          ctx->occ[f32][d][v] = e.occupancy();
-        }
-    }
+    if (ctx->dim == 2)
+      for (int f32 = 0; f32 <= (ctx->mixed ? 1 : 0); ++f32)
+        for (int d = 0; d < 2; ++d)
+          for (int v = 0; v < kNVar2; ++v)
+            ctx->occ[f32][d][v] = (f32 ? g_kernels32[ctx->ns].rhs2[d][v] : g_kernels64[ctx->ns].rhs2[d][v]).occupancy();
   }
+  if ((rc = plan_march(ctx))) return bail(ctx->fail(rc, "march table"));
   e = hipDeviceSynchronize();
   if (e != hipSuccess) return bail(ctx->fail((int)e, "device setup"));
   *out = ctx;
@@ -1230,9 +1303,10 @@ int cfx_get_rhs_tiles(cfx_ctx *ctx, int variant[3], int persist[3]) {
   return 0;
 }
 
-// Times every tile shape and persistence factor of each face direction on
-// this context's blocks (reps launches each, after one warm-up launch) and
-// keeps the fastest.  dq holds no result afterwards; the next RHS rewrites it.
+// Times every variant on this context's blocks (reps launches each, after one
+// warm-up launch) and keeps the fastest: in 2-D every tile shape and
+// persistence factor of each face direction, in 3-D every chunk length of the
+// march (direction 2).  dq holds no result afterwards; the next RHS rewrites it.
 int cfx_autotune(cfx_ctx *ctx, int reps, double *best_ms) {
   if (!ctx || reps <= 0) return CFX_E_ARG;
   const bool prof = ctx->profiling;
@@ -1242,17 +1316,25 @@ int cfx_autotune(cfx_ctx *ctx, int reps, double *best_ms) {
   (void)hipEventCreate(&b);
   static const int kPersist[] = {0, 1, 2, 4};
   int rc = 0;
-  for (int d = 0; d < ctx->dim && !rc; ++d) {
+  if (best_ms)
+    for (int d = 0; d < ctx->dim; ++d) best_ms[d] = 0;
+  for (int d = ctx->dim == 3 ? 2 : 0; d < ctx->dim && !rc; ++d) {
     double best = 1e30;
     int bv = 0, bp = 0;
     for (int v = 0; v < rhs_variants(ctx->dim) && !rc; ++v)
       for (int p : kPersist) {
+        if (ctx->dim == 3 && p) break;
         ctx->rhs_var[d] = v;
         ctx->rhs_persist[d] = p;
+        auto one = [&](int k) {
+          if (ctx->dim == 3) return rhs_march(ctx, k);
+          const Table &t = ctx->t_rhs[d][v];
+          return rhs_dir(ctx, d, k < 0 ? ctx->all(t) : ctx->one(t, k), d > 0);
+        };
         auto run = [&] {
-          if (ctx->batched) return rhs_dir(ctx, d, ctx->all(ctx->t_rhs[d][v]), d > 0);
+          if (ctx->batched) return one(-1);
           for (size_t k = 0; k < ctx->views.size(); ++k)
-            if (int r = rhs_dir(ctx, d, ctx->one(ctx->t_rhs[d][v], (int)k), d > 0)) return r;
+            if (int r = one((int)k)) return r;
           return 0;
         };
         if ((rc = run())) break;

@@ -36,9 +36,19 @@ struct alignas(64) ThermoRec {
   T v[kThLen];
 };
 
+
+// The enthalpy coefficients of one species in one range alone, for the sums
+// over species that form a mixture's polynomial: [0..5] as kThH, [6] 1/W.
+// One record is one scalar load (16 dwords in FP64, 8 in FP32).
+template <typename T>
+struct alignas(8 * sizeof(T)) MixRec {
+  T v[8];
+};
+
 template <typename T>
 struct SpeciesT {
   ThermoRec<T> th[kMaxSp];   // the thermo arrays below, regrouped per species
+  MixRec<T> mix[2][kMaxSp];  // range 0 low, 1 high
   int ns;
   T mw[kMaxSp], inv_mw[kMaxSp], r_sp[kMaxSp];  // W, 1/W, R_u/W
   T t_low[kMaxSp], t_mid[kMaxSp];

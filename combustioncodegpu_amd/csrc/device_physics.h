@@ -90,6 +90,83 @@ __device__ __forceinline__ R flog(R a) { return log(a); }
 template <>
 __device__ __forceinline__ float flog<float>(float a) { return __builtin_amdgcn_logf(a) * 0.6931471805599453f; }
 
+// N reciprocals, quotients or square roots at once, each step over all of
+// them before the next: an FP64 chain of dependent operations leaves most
+// issue slots of a wavefront empty (two wavefronts share a SIMD in the FP64
+// kernels), and the compiler keeps the order in which chains are written.
+// The values are those of the single forms.
+template <int N, typename R>
+__device__ __forceinline__ void frcp_n(const R *b, R *r) {
+  if constexpr (sizeof(R) == 8) {
+    R e[N];
+#pragma unroll
+    for (int n = 0; n < N; ++n) r[n] = __builtin_amdgcn_rcp(b[n]);
+#pragma unroll
+    for (int it = 0; it < 2; ++it) {
+#pragma unroll
+      for (int n = 0; n < N; ++n) e[n] = fma(-b[n], r[n], R(1));
+#pragma unroll
+      for (int n = 0; n < N; ++n) r[n] = fma(r[n], e[n], r[n]);
+    }
+  } else {
+#pragma unroll
+    for (int n = 0; n < N; ++n) r[n] = frcp<R>(b[n]);
+  }
+}
+template <int N, typename R>
+__device__ __forceinline__ void fdiv_n(const R *a, const R *b, R *q) {
+  R r[N];
+  frcp_n<N, R>(b, r);
+#pragma unroll
+  for (int n = 0; n < N; ++n) q[n] = a[n] * r[n];
+  if constexpr (sizeof(R) == 8) {
+    R e[N];
+#pragma unroll
+    for (int n = 0; n < N; ++n) e[n] = fma(-b[n], q[n], a[n]);
+#pragma unroll
+    for (int n = 0; n < N; ++n) q[n] = fma(r[n], e[n], q[n]);
+  }
+}
+// sqrt(a) and 1/sqrt(a) of positive, normal operands well inside the exponent
+// range.  FP64: one hardware reciprocal square root, g -> sqrt(a), h ->
+// 1/(2 sqrt(a)) by the coupled Newton iteration e = 1/2 - g h, g += g e,
+// h += h e, and two residual corrections of g (no scaling and special-value
+// steps, as for fdiv).
+template <int N, typename R>
+__device__ __forceinline__ void fsqrt_n(const R *a, R *g, R *rs) {
+  if constexpr (sizeof(R) == 8) {
+    R h[N], e[N];
+#pragma unroll
+    for (int n = 0; n < N; ++n) h[n] = __builtin_amdgcn_rsq(a[n]);
+#pragma unroll
+    for (int n = 0; n < N; ++n) g[n] = a[n] * h[n];
+#pragma unroll
+    for (int n = 0; n < N; ++n) h[n] = R(0.5) * h[n];
+#pragma unroll
+    for (int n = 0; n < N; ++n) e[n] = fma(-h[n], g[n], R(0.5));
+#pragma unroll
+    for (int n = 0; n < N; ++n) g[n] = fma(g[n], e[n], g[n]);
+#pragma unroll
+    for (int n = 0; n < N; ++n) h[n] = fma(h[n], e[n], h[n]);
+#pragma unroll
+    for (int n = 0; n < N; ++n) e[n] = fma(-h[n], g[n], R(0.5));
+#pragma unroll
+    for (int n = 0; n < N; ++n) h[n] = fma(h[n], e[n], h[n]);
+#pragma unroll
+    for (int it = 0; it < 2; ++it) {
+#pragma unroll
+      for (int n = 0; n < N; ++n) e[n] = fma(-g[n], g[n], a[n]);
+#pragma unroll
+      for (int n = 0; n < N; ++n) g[n] = fma(e[n], h[n], g[n]);
+    }
+#pragma unroll
+    for (int n = 0; n < N; ++n) rs[n] = h[n] + h[n];
+  } else {
+#pragma unroll
+    for (int n = 0; n < N; ++n) g[n] = fsqrt<R>(a[n]), rs[n] = frcp<R>(g[n]);
+  }
+}
+
 // ---------------------------------------------------------------- thermo ---
 // h_l(T) and cp_l(T) of one species (Thermo.cu:27-47): NASA-7 polynomial in
 // Horner form with the low/high set chosen at t_mid and the linear enthalpy
@@ -111,15 +188,19 @@ __device__ __forceinline__ R on_all_lanes(R v) {
 
 // The NASA-7 range every lane of the wavefront is in, for every species:
 // kRangeHi (all in the high set), kRangeLo (all in the low set, above
-// t_low), or kRangeMixed.  Smooth fields put most wavefronts on one side of
-// t_mid; those evaluate one polynomial set instead of both (the value is
-// the same bit for bit: the general path selects the same expression).
-constexpr int kRangeMixed = 0, kRangeLo = 1, kRangeHi = 2;
-template <typename R>
+// t_low), kRangeEach (each lane in one of the two; asked for with EACH), or
+// kRangeMixed.  Smooth fields put most wavefronts on one side of t_mid; those
+// evaluate one polynomial set instead of both (the value is the same bit for
+// bit: the general path selects the same expression).
+constexpr int kRangeMixed = 0, kRangeLo = 1, kRangeHi = 2, kRangeEach = 3;
+template <typename R, bool EACH = false>
 __device__ __forceinline__ int thermo_range(SpeciesPtrT<R> sp, R t0, R t1) {
   const R hf = R(sp->hi_from), lf = R(sp->lo_from), lt = R(sp->lo_to);
-  if (__all(t0 >= hf && t1 >= hf)) return kRangeHi;
-  if (__all(t0 >= lf && t0 < lt && t1 >= lf && t1 < lt)) return kRangeLo;
+  const bool h0 = t0 >= hf, h1 = t1 >= hf, l0 = t0 >= lf && t0 < lt, l1 = t1 >= lf && t1 < lt;
+  if (__all(h0 && h1)) return kRangeHi;
+  if (__all(l0 && l1)) return kRangeLo;
+  if constexpr (EACH)
+    if (__all((h0 || l0) && (h1 || l1))) return kRangeEach;
   return kRangeMixed;
 }
 
@@ -170,6 +251,84 @@ __device__ __forceinline__ R species_h(SpeciesPtrT<R> sp, int l, R t) {
   return t < tl ? R(c[kThHtlow]) + R(c[kThCptlow]) * (t - tl) : hp;
 }
 
+// Where a kernel reads the thermo records from: constant memory, or with the
+// mixture coefficients copied into LDS (2 x NS records of 8, range 0 first),
+// where each lane can have a range of its own (kEach).
+template <typename R>
+struct ThermoConst {
+  static constexpr bool kEach = false;
+  SpeciesPtrT<R> sp;
+  typedef R V8 __attribute__((ext_vector_type(8)));
+  __device__ auto rec(int l) const { return sp->th[l].v; }
+  __device__ auto mix(bool hi) const {
+    const auto *tab = (const __attribute__((address_space(4))) V8 *)(hi ? &sp->mix[1][0] : &sp->mix[0][0]);
+    return [tab](int l) { return tab[l]; };
+  }
+};
+template <int NS, typename R>
+struct ThermoLds {
+  static constexpr bool kEach = true;
+  SpeciesPtrT<R> sp;
+  const R *lds;
+  __device__ auto rec(int l) const { return sp->th[l].v; }
+  __device__ auto mix(bool hi) const {
+    const R *tab = lds + (hi ? NS * 8 : 0);
+    return [tab](int l) { return tab + 8 * l; };
+  }
+};
+
+// H_k = sum_l w_l h_{l,k}, k = 0..5, with the coefficients of range rg at
+// temperature t (kRangeLo, kRangeHi, or by lane with kRangeEach), N sums at
+// once over the weights w(n, l).  TH is where the records are read from.
+// Constant memory: the address is formed once and a record read as one vector
+// (a single scalar load); but only a few records fit the scalar registers, so
+// that every one or two species wait for a scalar load.  A copy in LDS
+// (broadcast reads) keeps many reads in flight: an FP64 RHS wavefront's AUSM+
+// phase took 3.4k cycles with scalar loads, of which it issued 1.6k.
+template <int NS, int N, typename R, typename TH, typename W>
+__device__ __forceinline__ void mixture_sum(const TH &th, int rg, const R *t, W w, R (*H)[6]) {
+  auto add = [&](const auto &c, int n, int l) {
+    const R x = w(n, l);
+#pragma unroll
+    for (int k = 0; k < 6; ++k) H[n][k] = l == 0 ? x * c[k] : H[n][k] + x * c[k];
+  };
+  if constexpr (TH::kEach && N > 1) {
+    if (rg == kRangeEach) {
+      const R hf = R(th.sp->hi_from);
+#pragma unroll
+      for (int n = 0; n < N; ++n) {
+        const auto tab = th.mix(t[n] >= hf);
+#pragma unroll
+        for (int l = 0; l < NS; ++l) add(tab(l), n, l);
+      }
+      return;
+    }
+  }
+  const auto tab = th.mix(TH::kEach && N == 1 ? t[0] >= R(th.sp->hi_from) : rg == kRangeHi);
+#pragma unroll
+  for (int l = 0; l < NS; ++l) {
+    const auto c = tab(l);
+#pragma unroll
+    for (int n = 0; n < N; ++n) add(c, n, l);
+  }
+}
+
+// h(T) and cp(T) = dh/dT of a mixture from its summed enthalpy coefficients
+// H_k = sum_l Y_l h_{l,k} (k = 0..5, in the layout of the thermo records, all
+// species in one range): cp's coefficients are (k + 1) H_k.
+// N mixtures in lockstep.
+template <int N, typename R>
+__device__ __forceinline__ void mixture_h_cp(const R (*C)[6], const R *t, R *h, R *cp) {
+#pragma unroll
+  for (int n = 0; n < N; ++n) h[n] = C[n][3] + t[n] * C[n][4], cp[n] = R(4) * C[n][3] + t[n] * (R(5) * C[n][4]);
+#pragma unroll
+  for (int k = 2; k >= 0; --k)
+#pragma unroll
+    for (int n = 0; n < N; ++n) h[n] = C[n][k] + t[n] * h[n], cp[n] = R(k + 1) * C[n][k] + t[n] * cp[n];
+#pragma unroll
+  for (int n = 0; n < N; ++n) h[n] = C[n][5] + t[n] * h[n];
+}
+
 // cp_l(T) only, frozen below t_low (Thermo.cu:49-63).  Loops over species
 // that need only cp read the per-array layout: the cp coefficients of all
 // species are contiguous there and arrive in a few wide loads.
@@ -187,46 +346,73 @@ __device__ __forceinline__ R species_cp(SpeciesPtrT<R> sp, int l, R t) {
   return t < R(sp->t_low[l]) ? R(sp->cp_tlow[l]) : cpp;
 }
 
-// Where a kernel reads the thermo records from: constant memory, or a copy
-// of the species' records in LDS (loaded once per workgroup).
-template <typename R>
-struct ThermoConst {
-  SpeciesPtrT<R> sp;
-  __device__ auto rec(int l) const { return sp->th[l].v; }
-};
-template <typename R>
-struct ThermoShared {
-  const R *p;
-  __device__ const R *rec(int l) const { return p + l * kThLen; }
-};
-
 // -------------------------------------------------------------- limiters ---
-// minmod (Limiter.cuh:13-16) and Van Albada (tag 1)
-template <typename R>
-__device__ __forceinline__ R limiter(int tag, R a, R b) {
-  if (tag == 1) {
-    const R ab = a * b;
-    return ab > R(0) ? fdiv<R>(ab * (a + b), a * a + b * b + Tiny<R>::v) : R(0);
+// N limited slopes in lockstep: minmod (Limiter.cuh:13-16), or Van Albada
+// (MODE 1).  The quotient is formed on every lane and then selected: as a
+// branch, each limiter would be a basic block of its own.
+template <int MODE, int N, typename R>
+__device__ __forceinline__ void limiter_n(const R *a, const R *b, R *s) {
+  if constexpr (MODE == 1) {
+    R ab[N], num[N], den[N];
+#pragma unroll
+    for (int n = 0; n < N; ++n) ab[n] = a[n] * b[n];
+#pragma unroll
+    for (int n = 0; n < N; ++n) num[n] = a[n] + b[n];
+#pragma unroll
+    for (int n = 0; n < N; ++n) den[n] = a[n] * a[n] + b[n] * b[n] + Tiny<R>::v;
+#pragma unroll
+    for (int n = 0; n < N; ++n) num[n] = ab[n] * num[n];
+    fdiv_n<N, R>(num, den, s);
+#pragma unroll
+    for (int n = 0; n < N; ++n) s[n] = on_all_lanes<R>(s[n]);
+    bool up[N];
+#pragma unroll
+    for (int n = 0; n < N; ++n) up[n] = ab[n] > R(0);
+  #pragma unroll
+    for (int n = 0; n < N; ++n) s[n] = on_all_lanes<R>(up[n] ? s[n] : R(0));
+  } else {
+#pragma unroll
+    for (int n = 0; n < N; ++n) {
+      const R m = fmin(fabs(a[n]), fabs(b[n]));
+      const bool up = a[n] > R(0) && b[n] > R(0), down = a[n] < R(0) && b[n] < R(0);
+          s[n] = up ? m : (down ? -m : R(0));
+    }
   }
-  const R m = fmin(fabs(a), fabs(b));
-  return (a > R(0) && b > R(0)) ? m : ((a < R(0) && b < R(0)) ? -m : R(0));
 }
 
 // MUSCL kappa = 1/3 on one variable (Reconstruction.cu:26-44), or first
 // order.  Both limiters are symmetric, lim(a,b) == lim(b,a) bit for bit, so
 // the reference's four calls per face reduce to the two limited slopes of
 // the two cells: (1-kappa)/4 + (1+kappa)/4 = 1/2.
+// N variables in lockstep, q[n][0..3] the four points; MODE: 0 minmod, 1 Van
+// Albada, 2 first order.
+template <int MODE, int N, typename R>
+__device__ __forceinline__ void muscl_n(const R (*q)[4], R *l, R *r) {
+  if constexpr (MODE < 2) {
+    R a[2 * N], b[2 * N], s[2 * N];
+#pragma unroll
+    for (int n = 0; n < N; ++n) {
+      a[2 * n] = q[n][1] - q[n][0];
+      b[2 * n] = a[2 * n + 1] = q[n][2] - q[n][1];
+      b[2 * n + 1] = q[n][3] - q[n][2];
+    }
+    limiter_n<MODE, 2 * N, R>(a, b, s);
+#pragma unroll
+    for (int n = 0; n < N; ++n) {
+      l[n] = q[n][1] + R(0.5) * s[2 * n];
+      r[n] = q[n][2] - R(0.5) * s[2 * n + 1];
+    }
+  } else {
+#pragma unroll
+    for (int n = 0; n < N; ++n) l[n] = q[n][1], r[n] = q[n][2];
+  }
+}
 template <typename R>
 __device__ __forceinline__ void muscl(const SchemeDev &S, R q0, R q1, R q2, R q3, R &l, R &r) {
-  if (S.reconstruction == 2) {
-    const R sl = limiter<R>(S.limiter, q1 - q0, q2 - q1);
-    const R sr = limiter<R>(S.limiter, q2 - q1, q3 - q2);
-    l = q1 + R(0.5) * sl;
-    r = q2 - R(0.5) * sr;
-  } else {
-    l = q1;
-    r = q2;
-  }
+  const R q[1][4] = {{q0, q1, q2, q3}};
+  if (S.reconstruction != 2) muscl_n<2, 1, R>(q, &l, &r);
+  else if (S.limiter == 1) muscl_n<1, 1, R>(q, &l, &r);
+  else muscl_n<0, 1, R>(q, &l, &r);
 }
 
 // AUSM+ flux (InviscidScheme.cu:39-106) from the reconstructed face states
@@ -237,74 +423,78 @@ template <int NS, typename R, typename TH>
 __device__ __forceinline__ void ausm_from_states(SpeciesPtrT<R> sp, const TH &th, const SchemeDev &S, const R *pl,
                                                  const R *pr, R k1, R k2, R k3, R *F) {
   constexpr int NV = 5 + NS;
-  R el = R(0.5) * (pl[1] * pl[1] + pl[2] * pl[2] + pl[3] * pl[3]);
-  R er = R(0.5) * (pr[1] * pr[1] + pr[2] * pr[2] + pr[3] * pr[3]);
-  R gam_l, gam_r, E_l, E_r;
+  // both sides in lockstep (index 0 left, 1 right).  H: specific total
+  // enthalpy (E + p) / rho; c2: gamma p / rho, third entry |k|^2
+  const R *const P[2] = {pl, pr};
+  R H[2], c2[3], x[2], y[2];
+#pragma unroll
+  for (int n = 0; n < 2; ++n) H[n] = R(0.5) * (P[n][1] * P[n][1] + P[n][2] * P[n][2] + P[n][3] * P[n][3]);
   if constexpr (NS > 0) {
-    R wl = R(0), wr = R(0);
+    R w[2] = {R(0), R(0)}, t[2], cp[2] = {R(0), R(0)};
 #pragma unroll
-    for (int l = 0; l < NS; ++l) {
-      wl += pl[5 + l] * R(sp->inv_mw[l]);
-      wr += pr[5 + l] * R(sp->inv_mw[l]);
+    for (int l = 0; l < NS; ++l)
+#pragma unroll
+      for (int n = 0; n < 2; ++n) w[n] += P[n][5 + l] * R(sp->inv_mw[l]);
+#pragma unroll
+    for (int n = 0; n < 2; ++n) w[n] *= R(kRu);  // gas constant of the mixture
+#pragma unroll
+    for (int n = 0; n < 2; ++n) x[n] = P[n][4], y[n] = P[n][0] * w[n];
+    fdiv_n<2, R>(x, y, t);
+    const int rg = thermo_range<R, TH::kEach>(sp, t[0], t[1]);
+    if (rg != kRangeMixed) {
+      // every lane in one range: the mixture's polynomial first
+      // (six coefficients, each summed over the species), evaluated once, in
+      // place of one enthalpy and one cp polynomial per species
+      R C[2][6], h[2];
+      mixture_sum<NS, 2, R>(th, rg, t, [&](int n, int l) { return P[n][5 + l]; }, C);
+      mixture_h_cp<2, R>(C, t, h, cp);
+#pragma unroll
+      for (int n = 0; n < 2; ++n) H[n] += h[n];
+    } else {
+#pragma unroll
+      for (int l = 0; l < NS; ++l)
+#pragma unroll
+        for (int n = 0; n < 2; ++n) {
+          R h, c;
+          thermo_h_cp<R>(th.rec(l), t[n], h, c);
+          H[n] += h * P[n][5 + l];
+          cp[n] += c * P[n][5 + l];
+        }
     }
-    const R Ru = R(kRu);
-    const R t_l = fdiv<R>(pl[4], pl[0] * Ru * wl);
-    const R t_r = fdiv<R>(pr[4], pr[0] * Ru * wr);
-    R cpl = R(0), cpr = R(0);
-    auto species_loop = [&](auto rgc) {
-      constexpr int RG = decltype(rgc)::value;
 #pragma unroll
-      for (int l = 0; l < NS; ++l) {
-        R h, cp;
-        thermo_h_cp<R, RG>(th.rec(l), t_l, h, cp);
-        el += h * pl[5 + l];
-        cpl += cp * pl[5 + l];
-        thermo_h_cp<R, RG>(th.rec(l), t_r, h, cp);
-        er += h * pr[5 + l];
-        cpr += cp * pr[5 + l];
-      }
-    };
-    const int rg = thermo_range<R>(sp, t_l, t_r);
-    if (rg == kRangeHi) species_loop(std::integral_constant<int, kRangeHi>{});
-    else if (rg == kRangeLo) species_loop(std::integral_constant<int, kRangeLo>{});
-    else species_loop(std::integral_constant<int, kRangeMixed>{});
-    E_l = pl[0] * el - pl[4];
-    E_r = pr[0] * er - pr[4];
-    gam_l = fdiv<R>(cpl, cpl - Ru * wl);
-    gam_r = fdiv<R>(cpr, cpr - Ru * wr);
+    for (int n = 0; n < 2; ++n) x[n] = cp[n] * (w[n] * t[n]), y[n] = cp[n] - w[n];
+    fdiv_n<2, R>(x, y, c2);  // gamma R T
   } else {
-    const R g1 = R(1) / R(S.gamma_air - 1);
-    E_l = el * pl[0] + pl[4] * g1;
-    E_r = er * pr[0] + pr[4] * g1;
-    gam_l = gam_r = R(S.gamma_air);
+    R v[2];
+#pragma unroll
+    for (int n = 0; n < 2; ++n) x[n] = P[n][4], y[n] = P[n][0];
+    fdiv_n<2, R>(x, y, v);
+    const R gam = R(S.gamma_air), g1 = R(S.gamma_air / (S.gamma_air - 1));
+#pragma unroll
+    for (int n = 0; n < 2; ++n) H[n] += g1 * v[n], c2[n] = gam * v[n];
   }
-  const R gk = fsqrt<R>(k1 * k1 + k2 * k2 + k3 * k3);
-  const R igk = frcp<R>(gk);
-  const R ul = (k1 * pl[1] + k2 * pl[2] + k3 * pl[3]) * igk;
-  const R ur = (k1 * pr[1] + k2 * pr[2] + k3 * pr[3]) * igk;
-  const R c = R(0.5) * (fsqrt<R>(fdiv<R>(gam_l * pl[4], pl[0])) + fsqrt<R>(fdiv<R>(gam_r * pr[4], pr[0])));
-  const R ic = frcp<R>(c);
-  const R ml = ul * ic, mr = ur * ic;
+  c2[2] = k1 * k1 + k2 * k2 + k3 * k3;
+  R g[3], rs[3];
+  fsqrt_n<3, R>(c2, g, rs);
+  const R gk = g[2], c = R(0.5) * (g[0] + g[1]);
+  const R ic = frcp<R>(c) * rs[2];  // 1 / (c |k|)
+  R m[2], a[2], b[2];
+#pragma unroll
+  for (int n = 0; n < 2; ++n) m[n] = (k1 * P[n][1] + k2 * P[n][2] + k3 * P[n][3]) * ic;
   constexpr double alpha = 3 / 16.0;
-  R mlp, plp, mrn, prn;
-  if (fabs(ml) > R(1)) {
-    mlp = R(0.5) * (ml + fabs(ml));
-    plp = fdiv<R>(mlp, ml);
-  } else {
-    const R a = (ml + R(1)) * (ml + R(1)) * R(0.25);
-    const R b = (ml * ml - R(1)) * (ml * ml - R(1));
-    mlp = a + R(0.125) * b;
-    plp = a * (R(2) - ml) + R(alpha) * ml * b;
+  // split Mach numbers and pressures; beyond |M| = 1 the pressure split
+  // M+-/M is 1 or 0 by the sign of M
+#pragma unroll
+  for (int n = 0; n < 2; ++n) {
+    const R o = n == 0 ? R(1) : R(-1);
+    a[n] = (m[n] + o) * (m[n] + o) * R(0.25);
+    b[n] = (m[n] * m[n] - R(1)) * (m[n] * m[n] - R(1));
   }
-  if (fabs(mr) > R(1)) {
-    mrn = R(0.5) * (mr - fabs(mr));
-    prn = fdiv<R>(mrn, mr);
-  } else {
-    const R a = (mr - R(1)) * (mr - R(1)) * R(0.25);
-    const R b = (mr * mr - R(1)) * (mr * mr - R(1));
-    mrn = -a - R(0.125) * b;
-    prn = a * (R(2) + mr) - R(alpha) * mr * b;
-  }
+  const bool sl = fabs(m[0]) > R(1), sr = fabs(m[1]) > R(1);
+  const R mlp = sl ? fmax(m[0], R(0)) : a[0] + R(0.125) * b[0];
+  const R mrn = sr ? fmin(m[1], R(0)) : -a[1] - R(0.125) * b[1];
+  const R plp = sl ? (m[0] > R(0) ? R(1) : R(0)) : a[0] * (R(2) - m[0]) + R(alpha) * m[0] * b[0];
+  const R prn = sr ? (m[1] < R(0) ? R(1) : R(0)) : a[1] * (R(2) + m[1]) - R(alpha) * m[1] * b[1];
   const R p_coeff = plp * pl[4] + prn * pr[4];
   const R m_half = mlp + mrn;
   const R mpos = R(0.5) * (m_half + fabs(m_half));
@@ -312,12 +502,11 @@ __device__ __forceinline__ void ausm_from_states(SpeciesPtrT<R> sp, const TH &th
   const R mass = c * (pl[0] * mpos + pr[0] * mneg);
   const R coeff = mass * gk;
   const bool left = mass >= R(0);
-  const R rho = left ? pl[0] : pr[0];
   F[0] = coeff;
   F[1] = coeff * (left ? pl[1] : pr[1]) + p_coeff * k1;
   F[2] = coeff * (left ? pl[2] : pr[2]) + p_coeff * k2;
   F[3] = coeff * (left ? pl[3] : pr[3]) + p_coeff * k3;
-  F[4] = fdiv<R>(coeff * ((left ? E_l : E_r) + (left ? pl[4] : pr[4])), rho);
+  F[4] = coeff * (left ? H[0] : H[1]);
 #pragma unroll
   for (int l = 5; l < NV; ++l) F[l] = coeff * (left ? pl[l] : pr[l]);
 }

@@ -33,7 +33,29 @@ struct Batch {
 };
 
 // --------------------------------------------------------- RHS tile shapes ---
-// Per face direction, the pencil tiles (faces along the direction x two
+// 3-D: one launch marches along k (rhs_march.h); a workgroup of nt threads
+// owns tx x ty cells.  A variant is the number of planes a workgroup marches
+// through: variant 0 as planned for the context's blocks, the others at most
+// kMarchChunk[v].
+struct MarchTile {
+  int tx, ty, nt, wpe;
+};
+// 16 x 8 cells have 408 faces, 7 wavefronts, and with the one that moves data
+// fill 2 waves per SIMD; the FP64 planes and fluxes of 9 species then take
+// 158 KB of LDS, FP32 half of it, so that two workgroups share a CU.
+constexpr MarchTile kMarch64 = {16, 8, 512, 2}, kMarch32 = {16, 8, 512, 4};
+constexpr int kNVar3 = 6;
+constexpr int kMarchChunk[kNVar3] = {0, 8, 16, 32, 64, 1 << 30};
+// workgroups of a block of m[3] points marched in chunks of at most `chunk` planes
+inline int march_groups(const int m[3], const MarchTile &t, int chunk) {
+  const int parts = m[2] <= chunk ? 1 : (m[2] + chunk - 1) / chunk;
+  return (m[0] + t.tx - 1) / t.tx * ((m[1] + t.ty - 1) / t.ty) * parts;
+}
+// big: a block's nine metric fields pass 4 GiB
+using MarchFn = int (*)(const Batch &b, int chunk, int big, const SpeciesDev *sp, const SchemeDev &S, hipStream_t st);
+using OccFn = int (*)();  // resident workgroups per CU of the kernel
+
+// 2-D: per face direction, the pencil tiles (faces along the direction x two
 // tangential extents) and the tile-group width G that the autotuner chooses
 // among.  Index v of each list is "variant v" of that direction.
 // w32: target waves per SIMD of the FP32 (mixed-precision) kernel; FP64
@@ -41,15 +63,10 @@ struct Batch {
 struct PencilTile {
   int ta, tb, tc, g, w32;
 };
-constexpr int kNVar3 = 6, kNVar2 = 2;
-constexpr PencilTile kTiles3[3][kNVar3] = {
-    {{32, 4, 2, 1, 3}, {32, 4, 4, 1, 3}, {64, 2, 2, 1, 3}, {32, 8, 1, 1, 3}, {32, 8, 1, 1, 4}, {32, 4, 2, 1, 4}},
-    {{8, 64, 1, 1, 4}, {8, 32, 1, 0, 4}, {8, 32, 1, 1, 4}, {8, 64, 1, 0, 4}, {16, 16, 1, 1, 4}, {16, 8, 2, 1, 4}},
-    {{8, 64, 1, 1, 4}, {8, 32, 1, 0, 4}, {8, 32, 1, 1, 4}, {8, 64, 1, 0, 4}, {16, 16, 1, 1, 4}, {16, 8, 2, 1, 4}}};
+constexpr int kNVar2 = 2;
 constexpr PencilTile kTiles2[2][kNVar2] = {{{32, 8, 1, 1, 3}, {64, 4, 1, 1, 3}}, {{16, 16, 1, 1, 3}, {32, 8, 1, 1, 3}}};
 
 inline int rhs_variants(int dim) { return dim == 3 ? kNVar3 : kNVar2; }
-inline const PencilTile &rhs_tile_shape(int dim, int dir, int v) { return dim == 3 ? kTiles3[dir][v] : kTiles2[dir][v]; }
 
 // Tiles one pencil launch of shape s covers on a block of m[3] points
 // (including the padding tiles of partial G x G groups).
@@ -64,7 +81,6 @@ inline int pencil_tiles(const int m[3], int dir, const PencilTile &s) {
 // grid: workgroups launched (a multiple of 8, at most the padded tile count)
 using RhsFn = int (*)(const Batch &b, int grid, const SpeciesDev *sp, const SchemeDev &S, int accumulate,
                       hipStream_t st);
-using OccFn = int (*)();  // resident workgroups per CU of the kernel
 struct RhsEntry {
   RhsFn launch;
   OccFn occupancy;
@@ -79,8 +95,9 @@ struct KernelSet64 {
   // ops[0..nops) with workgroup prefix off[0..nops], total workgroups
   int (*face_ops)(const BlockView *views, const FaceOp *ops, const int *off, int nops, int total,
                   const SpeciesDev *sp, const SchemeDev &S, const InflowDev *inflow, hipStream_t st);
-  RhsEntry rhs3[3][kNVar3];
   RhsEntry rhs2[2][kNVar2];
+  MarchFn march;
+  OccFn march_occ;
   // surrogate training set: n samples of (T, log p, Y) and log(mu, kappa,
   // rho*D) from the FP64 transport; lim = t_lo, t_hi, log p_lo, log p_hi
   int (*mlp_samples)(const SpeciesDev *sp, const SchemeDev &S, long long n, unsigned long long seed,
@@ -100,8 +117,9 @@ struct KernelSet32 {
   // properties with the surrogate transport (mixed precision)
   int (*props_mlp)(const Batch &b, const SpeciesDev *sp, const SchemeDev &S, const MlpDev *mlp, const void *ops,
                    const float *bias, unsigned long long *counters, hipStream_t st);
-  RhsEntry rhs3[3][kNVar3];
   RhsEntry rhs2[2][kNVar2];
+  MarchFn march;
+  OccFn march_occ;
 };
 
 extern KernelSet64 g_kernels64[kMaxSp + 1];

@@ -10,6 +10,7 @@
 #include "device_physics.h"
 #include "kernels.h"
 #include "mlp.h"
+#include "rhs_march.h"
 #include "rhs_pencil.h"
 
 #ifndef CFX_NS
@@ -26,10 +27,6 @@ namespace {
 constexpr int NS = CFX_NS;
 constexpr int NSA = NS > 0 ? NS : 1;  // extent of the per-species arrays
 static_assert(NS >= 0 && NS <= kMaxSp, "species count out of range");
-
-constexpr PencilTile tile_of(bool d3, int dir, int v) {
-  return d3 ? kTiles3[dir][v] : kTiles2[dir < 2 ? dir : 0][v < kNVar2 ? v : 0];
-}
 
 __device__ __forceinline__ long long pidx(const GView &B, int i, int j, int k) {
   return (long long)(k + kNgg) * B.sz + (long long)(j + kNgg) * B.sy + (i + kNgg);
@@ -188,13 +185,13 @@ int launch_props(const Batch &b, const SpeciesDev *sp, const SchemeDev &S, hipSt
 }
 
 // ------------------------------------------------------------------- RHS ---
-// FP64 pencils at 2 waves per SIMD; FP32 needs half the registers and
+// FP64 pencils (2-D) at 2 waves per SIMD; FP32 needs half the registers and
 // targets 3.
 // grid < padded tile count: the persistent kernel strides through the tiles
-template <int DIR, int V, typename R, bool D3>
+template <int DIR, int V, typename R>
 int launch_rhs_dir(const Batch &b, int grid, const SpeciesDev *sp, const SchemeDev &S, int accumulate,
                    hipStream_t st) {
-  constexpr PencilTile s = tile_of(D3, DIR, V);
+  constexpr PencilTile s = kTiles2[DIR][V];
   constexpr int WPE = sizeof(R) == 8 ? 2 : s.w32;
   if (b.total <= 0) return 0;
   const int padded = (b.total + 7) / 8 * 8;
@@ -207,9 +204,9 @@ int launch_rhs_dir(const Batch &b, int grid, const SpeciesDev *sp, const SchemeD
   return (int)hipGetLastError();
 }
 
-template <int DIR, int V, typename R, bool D3>
+template <int DIR, int V, typename R>
 int occupancy_rhs_dir() {
-  constexpr PencilTile s = tile_of(D3, DIR, V);
+  constexpr PencilTile s = kTiles2[DIR][V];
   constexpr int WPE = sizeof(R) == 8 ? 2 : s.w32;
   int n = 0;
   if (hipOccupancyMaxActiveBlocksPerMultiprocessor(
@@ -218,30 +215,43 @@ int occupancy_rhs_dir() {
   return n;
 }
 
+template <typename R>
+constexpr MarchTile march_tile() {
+  return sizeof(R) == 8 ? kMarch64 : kMarch32;
+}
+
+template <typename R>
+int launch_rhs_march(const Batch &b, int chunk, int big, const SpeciesDev *sp, const SchemeDev &S, hipStream_t st) {
+  constexpr MarchTile t = march_tile<R>();
+  if (b.total <= 0) return 0;
+  const int padded = (b.total + 7) / 8 * 8;
+  if (big)
+    rhs_march_kernel<NS, t.tx, t.ty, t.nt, t.wpe, R, true>
+        <<<padded, t.nt, 0, st>>>(b.views, b.off, b.nb, padded, chunk, sp, S);
+  else
+    rhs_march_kernel<NS, t.tx, t.ty, t.nt, t.wpe, R, false>
+        <<<padded, t.nt, 0, st>>>(b.views, b.off, b.nb, padded, chunk, sp, S);
+  return (int)hipGetLastError();
+}
+
+template <typename R>
+int occupancy_rhs_march() {
+  constexpr MarchTile t = march_tile<R>();
+  int n = 0;
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, rhs_march_kernel<NS, t.tx, t.ty, t.nt, t.wpe, R, false>, t.nt,
+                                                   0) != hipSuccess)
+    return 0;
+  return n;
+}
+
 template <typename R, typename Set>
 void register_rhs(Set &k) {
-  k.rhs3[0][0] = {launch_rhs_dir<0, 0, R, true>, occupancy_rhs_dir<0, 0, R, true>};
-  k.rhs3[0][1] = {launch_rhs_dir<0, 1, R, true>, occupancy_rhs_dir<0, 1, R, true>};
-  k.rhs3[0][2] = {launch_rhs_dir<0, 2, R, true>, occupancy_rhs_dir<0, 2, R, true>};
-  k.rhs3[0][3] = {launch_rhs_dir<0, 3, R, true>, occupancy_rhs_dir<0, 3, R, true>};
-  k.rhs3[0][4] = {launch_rhs_dir<0, 4, R, true>, occupancy_rhs_dir<0, 4, R, true>};
-  k.rhs3[0][5] = {launch_rhs_dir<0, 5, R, true>, occupancy_rhs_dir<0, 5, R, true>};
-  k.rhs3[1][0] = {launch_rhs_dir<1, 0, R, true>, occupancy_rhs_dir<1, 0, R, true>};
-  k.rhs3[1][1] = {launch_rhs_dir<1, 1, R, true>, occupancy_rhs_dir<1, 1, R, true>};
-  k.rhs3[1][2] = {launch_rhs_dir<1, 2, R, true>, occupancy_rhs_dir<1, 2, R, true>};
-  k.rhs3[1][3] = {launch_rhs_dir<1, 3, R, true>, occupancy_rhs_dir<1, 3, R, true>};
-  k.rhs3[1][4] = {launch_rhs_dir<1, 4, R, true>, occupancy_rhs_dir<1, 4, R, true>};
-  k.rhs3[1][5] = {launch_rhs_dir<1, 5, R, true>, occupancy_rhs_dir<1, 5, R, true>};
-  k.rhs3[2][0] = {launch_rhs_dir<2, 0, R, true>, occupancy_rhs_dir<2, 0, R, true>};
-  k.rhs3[2][1] = {launch_rhs_dir<2, 1, R, true>, occupancy_rhs_dir<2, 1, R, true>};
-  k.rhs3[2][2] = {launch_rhs_dir<2, 2, R, true>, occupancy_rhs_dir<2, 2, R, true>};
-  k.rhs3[2][3] = {launch_rhs_dir<2, 3, R, true>, occupancy_rhs_dir<2, 3, R, true>};
-  k.rhs3[2][4] = {launch_rhs_dir<2, 4, R, true>, occupancy_rhs_dir<2, 4, R, true>};
-  k.rhs3[2][5] = {launch_rhs_dir<2, 5, R, true>, occupancy_rhs_dir<2, 5, R, true>};
-  k.rhs2[0][0] = {launch_rhs_dir<0, 0, R, false>, occupancy_rhs_dir<0, 0, R, false>};
-  k.rhs2[0][1] = {launch_rhs_dir<0, 1, R, false>, occupancy_rhs_dir<0, 1, R, false>};
-  k.rhs2[1][0] = {launch_rhs_dir<1, 0, R, false>, occupancy_rhs_dir<1, 0, R, false>};
-  k.rhs2[1][1] = {launch_rhs_dir<1, 1, R, false>, occupancy_rhs_dir<1, 1, R, false>};
+  k.march = launch_rhs_march<R>;
+  k.march_occ = occupancy_rhs_march<R>;
+  k.rhs2[0][0] = {launch_rhs_dir<0, 0, R>, occupancy_rhs_dir<0, 0, R>};
+  k.rhs2[0][1] = {launch_rhs_dir<0, 1, R>, occupancy_rhs_dir<0, 1, R>};
+  k.rhs2[1][0] = {launch_rhs_dir<1, 0, R>, occupancy_rhs_dir<1, 0, R>};
+  k.rhs2[1][1] = {launch_rhs_dir<1, 1, R>, occupancy_rhs_dir<1, 1, R>};
 }
 
 #if CFX_PREC == 64

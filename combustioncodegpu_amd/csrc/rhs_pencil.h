@@ -1,5 +1,6 @@
 // rhs_pencil.h — the RHS of one face direction per launch, with the stencil
-// staged through LDS in batches of variables.
+// staged through LDS in batches of variables (2-D blocks; the 3-D RHS is
+// rhs_march.h).
 //
 // A workgroup owns a tile of TA x TB x TC faces (TA along the face direction
 // "a", TB/TC along the two other directions "b"/"c" in increasing axis
