@@ -210,6 +210,28 @@ struct FaceOp {
   FaceRange r;  // boundary range (wall: shrunk by ngg tangentially)
   InnerDev f;   // exchange mapping
   WallDev wl;
+  int ghosts_only;  // exchange: the shared layer belongs to another op
+};
+
+// The exchange of the points near the edges of inner faces, where the ops of
+// several faces meet: one component per set of stored points that such ops
+// link (copies of one grid point in the blocks around it), with the ops on
+// it in application order.  Component c has slots [slot_off[c], slot_off[c+1])
+// and ops [op_off[c], op_off[c+1]).
+constexpr int kMaxSlots = 16;
+constexpr unsigned kSlotWritten = 0x80000000u;  // or'ed into p: an op writes this slot
+struct ExSlot {
+  int blk;
+  unsigned p;  // padded index
+};
+struct ExOp {
+  unsigned char dst, src, average, pad;  // average: both take (dst + src) / 2, else dst takes src
+};
+struct ExStrips {
+  const ExSlot *slots;
+  const ExOp *ops;
+  const int *slot_off, *op_off;
+  int n;  // components
 };
 
 // Work segments: workgroup w (counted from off[0]) belongs to segment s with

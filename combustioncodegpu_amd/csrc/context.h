@@ -89,6 +89,12 @@ struct cfx_ctx {
   std::vector<FaceOp> ops_step;
   std::vector<int> ops_step_src;  // index of the op in `ops` each step op comes from
   Schedule sched_seq_step, sched_all_step;
+  // batched execution of the exchange in two launches, where the mesh allows
+  // it (split_exchange): the middles of the inner faces, then the strips near
+  // their edges; sched_bc_step holds the boundary conditions of a step
+  bool ex_split = false;
+  Schedule sched_mid, sched_bc_step;
+  ExStrips strips{};
   int n_fused = 0;
   bool batched = true, use_graph = false;
   hipGraph_t graph = nullptr;

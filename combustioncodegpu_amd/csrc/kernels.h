@@ -149,6 +149,8 @@ int launch_ghost_corners(double *xyz, int mx, int my, int mz, hipStream_t st);
 // the full prefix, so a per-block launch and a batched one fill the same slots
 int launch_residual_partial(const Batch &b, double *partial, hipStream_t st);
 int launch_residual_final(const double *partial, int n, double *out, hipStream_t st);
+// every component of the strips, one lane per component, the fields over the wavefronts
+int launch_exchange_strips(const BlockView *views, const ExStrips &x, int ns, int mixed, hipStream_t st);
 int launch_eliminate_k(const BlockView &B, int ns, hipStream_t st);
 
 }  // namespace cfx

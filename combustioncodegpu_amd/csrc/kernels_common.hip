@@ -171,6 +171,59 @@ __global__ void __launch_bounds__(kTpb) residual_final_kernel(const double *part
   }
 }
 
+// inner_communication (Field.cu:213-266) of the strips near the edges of the
+// inner faces.  The exchange of a field reads and writes only that field: a
+// lane takes one component and its wavefront every kStripWaves-th field.  Per
+// field it reads the component's points (all loads in flight at once), applies
+// the component's ops in their order to the values in LDS, and stores the
+// points that an op wrote.  Bound by the latency of its scattered reads; the
+// workgroup turns the slots into addresses once for all fields.
+constexpr int kStripWaves = 4, kStripTpb = 64 * kStripWaves;
+constexpr int kStripFill = 2048;  // workgroups
+__global__ void __launch_bounds__(kStripTpb) exchange_strip_kernel(const BlockView *__restrict__ views, ExStrips x,
+                                                                   int nv, int nf) {
+  static_assert(kMaxSlots % 4 == 0, "slots are read in fours");
+  __shared__ double val[kMaxSlots][kStripTpb];
+  __shared__ ExSlot slot[kMaxSlots][64];
+  const int t = threadIdx.x, lane = t & 63, c = (int)blockIdx.x * 64 + lane;
+  const int wv = __builtin_amdgcn_readfirstlane(t >> 6);
+  const bool in = c < x.n;
+  const int s0 = in ? x.slot_off[c] : 0, ns = in ? x.slot_off[c + 1] - s0 : 0;
+  const int o0 = in ? x.op_off[c] : 0, no = in ? x.op_off[c + 1] - o0 : 0;
+  for (int s = wv; s < ns; s += kStripWaves) slot[s][lane] = x.slots[s0 + s];
+  __syncthreads();
+  for (int f = wv + kStripWaves * (int)blockIdx.y; f < nf; f += kStripWaves * (int)gridDim.y) {
+    auto at = [&](const ExSlot &s) -> gptr<double> {
+      const BlockView &B = views[s.blk];
+      double *a = f < 6 ? B.bv + f * B.np : (f < 6 + nv ? B.cv + (f - 6) * B.np : B.yk + (f - 6 - nv) * B.np);
+      return (gptr<double>)a + (s.p & ~kSlotWritten);
+    };
+    // four loads at a time, the last ones repeating slot 0
+    for (int s = 0; s < ns; s += 4) {
+      double v[4];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) v[q] = *at(slot[s + q < ns ? s + q : 0][lane]);
+#pragma unroll
+      for (int q = 0; q < 4; ++q) val[s + q][t] = v[q];
+    }
+    for (int o = 0; o < no; ++o) {
+      const ExOp op = x.ops[o0 + o];
+      const double y = val[op.src][t];
+      if (op.average) {
+        const double a = 0.5 * (y + val[op.dst][t]);
+        val[op.dst][t] = a;
+        val[op.src][t] = a;
+      } else {
+        val[op.dst][t] = y;
+      }
+    }
+    for (int s = 0; s < ns; ++s) {
+      const ExSlot sl = slot[s][lane];
+      if (sl.p & kSlotWritten) *at(sl) = val[s][t];
+    }
+  }
+}
+
 // eliminate_k_gradient (Field.cu:268-292), 2-D only
 __global__ void eliminate_k_kernel(BlockView view, int ns) {
   const GView B = gview(view);
@@ -471,6 +524,15 @@ int launch_residual_partial(const Batch &b, double *partial, hipStream_t st) {
 
 int launch_residual_final(const double *partial, int n, double *out, hipStream_t st) {
   residual_final_kernel<<<1, kTpb, 0, st>>>(partial, n, out);
+  return (int)hipGetLastError();
+}
+
+int launch_exchange_strips(const BlockView *views, const ExStrips &x, int ns, int mixed, hipStream_t st) {
+  if (x.n <= 0) return 0;
+  const int nf = 6 + 5 + ns + (mixed ? 0 : ns), gx = (x.n + 63) / 64;
+  // few components: the fields over several workgroups, to fill the chip
+  const int gy = std::max(1, std::min((nf + kStripWaves - 1) / kStripWaves, kStripFill / gx));
+  exchange_strip_kernel<<<dim3(gx, gy, 1), kStripTpb, 0, st>>>(views, x, 5 + ns, nf);
   return (int)hipGetLastError();
 }
 

@@ -666,7 +666,7 @@ __device__ __forceinline__ void bc_symmetry_point(const GView &B, const FaceRang
 // Mesh.cpp:905-917 at loop point n: shared-face points are averaged between
 // the two blocks, ghost layers take the neighbour's values.
 __device__ __forceinline__ void exchange_point(const GView &B, const GView &T, const InnerDev &f,
-                                               const int n[3]) {
+                                               const int n[3], bool ghosts_only) {
   int idx[3], d_idx[3], it[3];
   for (int q = 0; q < 3; ++q) {
     d_idx[q] = f.loop_dir[q] * n[q];
@@ -681,6 +681,7 @@ __device__ __forceinline__ void exchange_point(const GView &B, const GView &T, c
   // as far as the compiler knows, so it keeps every store before any later
   // load: field by field, each would cost a memory round trip).
   if (idx[f.face] == face_layer) {
+    if (ghosts_only) return;
     // the shared layer: both sides of a group of fields, then the averages
     auto average = [&](gptr<double> bb, gptr<double> tt, auto kc) {
       constexpr int K = decltype(kc)::value;
@@ -744,7 +745,7 @@ __global__ void __launch_bounds__(kTpb) face_ops_kernel(const BlockView *__restr
     case CFX_BC_SYMMETRY: bc_symmetry_point(B, op.r, i, j, k, sp, S); break;
     case kOpExchange: {
       const GView T = gview(views[op.tgt]);
-      exchange_point(B, T, op.f, nn);
+      exchange_point(B, T, op.f, nn, op.ghosts_only != 0);
       break;
     }
     default: break;
