@@ -221,15 +221,17 @@ int build_tables(cfx_ctx *ctx) {
       (rc = upload_table(ctx, ctx->t_dt, dtc)) || (rc = upload_table(ctx, ctx->t_last, last)) ||
       (rc = upload_table(ctx, ctx->t_res, res)) || (rc = upload_table(ctx, ctx->t_tile, til)))
     return rc;
-  for (int d = 0; d < 2 && ctx->dim == 2; ++d)
-    for (int v = 0; v < kNVar2; ++v) {
-      std::vector<int> tiles(nb);
-      for (int b = 0; b < nb; ++b) {
-        const int m[3] = {ctx->hb[b].mx, ctx->hb[b].my, ctx->hb[b].mz};
-        tiles[b] = pencil_tiles(m, d, kTiles2[d][v]);
-      }
-      if ((rc = upload_table(ctx, ctx->t_rhs[d][v], tiles))) return rc;
+  if (ctx->dim != 2) return 0;
+  std::vector<int> count(nb);
+  for (int b = 0; b < nb; ++b) count[b] = chunks((long long)(ctx->hb[b].mx + 2 * kNgg) * (ctx->hb[b].my + 2 * kNgg), kTpb);
+  if ((rc = upload_table(ctx, ctx->t_plane, count))) return rc;
+  for (int v = 0; v < kNVar2; ++v) {
+    for (int b = 0; b < nb; ++b) {
+      const int m[3] = {ctx->hb[b].mx, ctx->hb[b].my, ctx->hb[b].mz};
+      count[b] = plane_groups(m, kTiles2[v]);
     }
+    if ((rc = upload_table(ctx, ctx->t_rhs[v], count))) return rc;
+  }
   return 0;
 }
 
@@ -786,6 +788,16 @@ int build_ops(cfx_ctx *ctx) {
   if ((rc = build_schedule(ctx, ctx->ops_step, ctx->sched_seq_step, 0, ns, false, &ctx->ops_step_src)) ||
       (rc = build_schedule(ctx, ctx->ops_step, ctx->sched_all_step, 0, ns, true)))
     return rc;
+  ctx->plane_only = ctx->dim == 2;
+  for (const FaceOp &op : ctx->ops) {
+    const HostBlock &H = ctx->hb[op.blk];
+    const int a = op.kind == kOpExchange ? op.f.face : op.r.face;
+    const int end[3] = {H.mx - 1, H.my - 1, H.mz - 1};
+    bool edge = a != 2;
+    if (op.kind == kOpExchange) edge = edge && op.f.src_tar[2] == 2;
+    else edge = edge && op.r.rs[a] == op.r.re[a] && (op.r.rs[a] == 0 || op.r.rs[a] == end[a]);
+    ctx->plane_only = ctx->plane_only && edge;
+  }
   int nbc_step = 0;  // fold_outflow keeps the order: boundary conditions first
   while (nbc_step < ns && ctx->ops_step[nbc_step].kind != kOpExchange) ++nbc_step;
   if ((rc = split_exchange(ctx)) ||
@@ -810,15 +822,12 @@ int run_levels(cfx_ctx *ctx, const Schedule &sc, int l0, int l1) {
 }
 
 // ------------------------------------------------------------ step parts ---
-// 2-D: one face direction
-int rhs_dir(cfx_ctx *ctx, int d, const Batch &b, int accumulate) {
-  const int v = ctx->rhs_var[d];
-  const RhsEntry &e = ctx->mixed ? g_kernels32[ctx->ns].rhs2[d][v] : g_kernels64[ctx->ns].rhs2[d][v];
-  const int padded = (b.total + 7) / 8 * 8;
-  int grid = padded;
-  const int occ = ctx->occ[ctx->mixed ? 1 : 0][d][v];
-  if (ctx->rhs_persist[d] > 0 && occ > 0) grid = std::min(grid, (ctx->rhs_persist[d] * occ * ctx->n_cu + 7) / 8 * 8);
-  return ctx->timed_launch(K_RHS, [&] { return e.launch(b, grid, ctx->sp_dev, ctx->S, accumulate, ctx->stream); });
+// 2-D: both face directions; the variant of direction 1 counts
+int rhs_plane(cfx_ctx *ctx, int blk, bool planar) {
+  const int v = ctx->rhs_var[1];
+  const PlaneFn fn = ctx->mixed ? g_kernels32[ctx->ns].plane[v] : g_kernels64[ctx->ns].plane[v];
+  const Batch b = blk < 0 ? ctx->all(ctx->t_rhs[v]) : ctx->one(ctx->t_rhs[v], blk);
+  return ctx->timed_launch(K_RHS, [&] { return fn(b, planar ? 1 : 0, ctx->sp_dev, ctx->S, ctx->stream); });
 }
 
 // 3-D: all face directions; the march runs along k, so the variant of that direction counts
@@ -831,15 +840,9 @@ int rhs_march(cfx_ctx *ctx, int blk) {
   });
 }
 
-int do_rhs(cfx_ctx *ctx, int blk) {
-  auto run = [&](int b) {  // b < 0: every block in one launch
-    if (ctx->dim == 3) return rhs_march(ctx, b);
-    for (int d = 0; d < 2; ++d) {
-      const Table &t = ctx->t_rhs[d][ctx->rhs_var[d]];
-      if (int rc = rhs_dir(ctx, d, b < 0 ? ctx->all(t) : ctx->one(t, b), d > 0)) return rc;
-    }
-    return 0;
-  };
+// blk < 0: every block; planar: see rhs_plane
+int do_rhs(cfx_ctx *ctx, int blk, bool planar = false) {
+  auto run = [&](int b) { return ctx->dim == 3 ? rhs_march(ctx, b) : rhs_plane(ctx, b, planar); };
   if (blk >= 0 || ctx->batched) {
     CFX_TRY(run(blk));
     return 0;
@@ -929,14 +932,15 @@ int do_ghosts(cfx_ctx *ctx, bool after_update) {
   return run_levels(ctx, seq, 0, seq.levels());
 }
 
-int do_elim(cfx_ctx *ctx) {
+int do_elim(cfx_ctx *ctx, bool ring = false) {
   if (ctx->dim != 2) return 0;
   for (auto &B : ctx->views)
-    CFX_TRY(ctx->timed_launch(K_OTHER, [&] { return launch_eliminate_k(B, ctx->ns, ctx->stream); }));
+    CFX_TRY(ctx->timed_launch(K_OTHER, [&] { return launch_eliminate_k(B, ctx->ns, ring ? 1 : 0, ctx->stream); }));
   return 0;
 }
 
-int do_props(cfx_ctx *ctx) {
+// plane: the plane k = 0 of 2-D blocks alone (not with the surrogate)
+int do_props(cfx_ctx *ctx, bool plane = false) {
   if (ctx->transport == CFX_TRANSPORT_MLP) {
     if (!ctx->mlp_ready) return ctx->fail(CFX_E_SURROGATE, "surrogate transport selected but not trained or loaded");
     auto fn = g_kernels32[ctx->ns].props_mlp;
@@ -949,8 +953,8 @@ int do_props(cfx_ctx *ctx) {
     return 0;
   }
   auto fn = ctx->mixed ? g_kernels32[ctx->ns].props : g_kernels64[ctx->ns].props;
-  CFX_TRY(per_batch(ctx, ctx->t_pad, [&](const Batch &b) {
-    return ctx->timed_launch(K_PROPS, [&] { return fn(b, ctx->sp_dev, ctx->S, ctx->stream); });
+  CFX_TRY(per_batch(ctx, plane ? ctx->t_plane : ctx->t_pad, [&](const Batch &b) {
+    return ctx->timed_launch(K_PROPS, [&] { return fn(b, plane ? 1 : 0, ctx->sp_dev, ctx->S, ctx->stream); });
   }));
   return 0;
 }
@@ -965,12 +969,23 @@ int do_store_last(cfx_ctx *ctx) {
 // Driver::steady_simulation loop body (Driver.cu:135-190): with rk_stages 1
 // the reference's explicit Euler with local dt; with 3 the SSP-RK3 stages
 // with the global CFL dt taken at stage 0.
+// 2-D RK3: the ghost planes along k are read by the RHS, whose differences
+// along k vanish where they are copies of the plane, and near the faces by the
+// ghost fills, which cover their tangential rows too.  The stages within the
+// step therefore work on the plane alone (RHS without k differences, copies of
+// the ring near the faces, properties of the plane); the full copies and the
+// properties of all planes are made once, for the state the step leaves.
+// 1021x509 air, per stage: copies 40 -> 5 us, properties 28 -> 9 us.  (The
+// surrogate counts the points it falls back on, over all planes, and keeps the
+// full stages.)
 int do_step(cfx_ctx *ctx) {
   int rc;
   if ((rc = do_store_last(ctx))) return rc;
   const int stages = ctx->rk == 3 ? 3 : 1;
+  const bool planar = ctx->plane_only && ctx->transport != CFX_TRANSPORT_MLP;
   for (int s = 0; s < stages; ++s) {
-    if ((rc = do_rhs(ctx, -1))) return rc;
+    const bool last = s == stages - 1;
+    if ((rc = do_rhs(ctx, -1, planar && s > 0))) return rc;
     if (ctx->rk == 3) {
       if (s == 0 && (rc = do_dt(ctx, 1, 0))) return rc;
     } else {
@@ -979,8 +994,8 @@ int do_step(cfx_ctx *ctx) {
     if (ctx->lusgs && (rc = do_lusgs(ctx))) return rc;
     if ((rc = do_update(ctx, s))) return rc;
     if ((rc = do_ghosts(ctx, true))) return rc;
-    if ((rc = do_elim(ctx))) return rc;
-    if ((rc = do_props(ctx))) return rc;
+    if ((rc = do_elim(ctx, planar && !last))) return rc;
+    if ((rc = do_props(ctx, planar && !last))) return rc;
   }
   return 0;
 }
@@ -1335,11 +1350,6 @@ int cfx_create(const cfx_params *params, const cfx_species *species, const cfx_b
     (void)hipGetDevice(&dev);
     if (hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && ncu > 0)
       ctx->n_cu = ncu;
-    if (ctx->dim == 2)
-      for (int f32 = 0; f32 <= (ctx->mixed ? 1 : 0); ++f32)
-        for (int d = 0; d < 2; ++d)
-          for (int v = 0; v < kNVar2; ++v)
-            ctx->occ[f32][d][v] = (f32 ? g_kernels32[ctx->ns].rhs2[d][v] : g_kernels64[ctx->ns].rhs2[d][v]).occupancy();
   }
   if ((rc = plan_march(ctx))) return bail(ctx->fail(rc, "march table"));
   e = hipDeviceSynchronize();
@@ -1587,9 +1597,9 @@ int cfx_get_rhs_tiles(cfx_ctx *ctx, int variant[3], int persist[3]) {
 }
 
 // Times every variant on this context's blocks (reps launches each, after one
-// warm-up launch) and keeps the fastest: in 2-D every tile shape and
-// persistence factor of each face direction, in 3-D every chunk length of the
-// march (direction 2).  dq holds no result afterwards; the next RHS rewrites it.
+// warm-up launch) and keeps the fastest: in 2-D every tile shape, in 3-D every
+// chunk length of the march; the choice is the last direction's.  dq holds no
+// result afterwards; the next RHS rewrites it.
 int cfx_autotune(cfx_ctx *ctx, int reps, double *best_ms) {
   if (!ctx || reps <= 0) return CFX_E_ARG;
   const bool prof = ctx->profiling;
@@ -1597,42 +1607,25 @@ int cfx_autotune(cfx_ctx *ctx, int reps, double *best_ms) {
   hipEvent_t a, b;
   (void)hipEventCreate(&a);
   (void)hipEventCreate(&b);
-  static const int kPersist[] = {0, 1, 2, 4};
   int rc = 0;
   if (best_ms)
     for (int d = 0; d < ctx->dim; ++d) best_ms[d] = 0;
-  for (int d = ctx->dim == 3 ? 2 : 0; d < ctx->dim && !rc; ++d) {
-    double best = 1e30;
-    int bv = 0, bp = 0;
-    for (int v = 0; v < rhs_variants(ctx->dim) && !rc; ++v)
-      for (int p : kPersist) {
-        if (ctx->dim == 3 && p) break;
-        ctx->rhs_var[d] = v;
-        ctx->rhs_persist[d] = p;
-        auto one = [&](int k) {
-          if (ctx->dim == 3) return rhs_march(ctx, k);
-          const Table &t = ctx->t_rhs[d][v];
-          return rhs_dir(ctx, d, k < 0 ? ctx->all(t) : ctx->one(t, k), d > 0);
-        };
-        auto run = [&] {
-          if (ctx->batched) return one(-1);
-          for (size_t k = 0; k < ctx->views.size(); ++k)
-            if (int r = one((int)k)) return r;
-          return 0;
-        };
-        if ((rc = run())) break;
-        (void)hipEventRecord(a, ctx->stream);
-        for (int r = 0; r < reps && !rc; ++r) rc = run();
-        (void)hipEventRecord(b, ctx->stream);
-        (void)hipEventSynchronize(b);
-        float ms = 0;
-        (void)hipEventElapsedTime(&ms, a, b);
-        if (ms / reps < best) best = ms / reps, bv = v, bp = p;
-      }
-    ctx->rhs_var[d] = bv;
-    ctx->rhs_persist[d] = bp;
-    if (best_ms) best_ms[d] = best;
+  const int d = ctx->dim - 1;
+  double best = 1e30;
+  int bv = 0;
+  for (int v = 0; v < rhs_variants(ctx->dim) && !rc; ++v) {
+    ctx->rhs_var[d] = v;
+    if ((rc = do_rhs(ctx, -1))) break;
+    (void)hipEventRecord(a, ctx->stream);
+    for (int r = 0; r < reps && !rc; ++r) rc = do_rhs(ctx, -1);
+    (void)hipEventRecord(b, ctx->stream);
+    (void)hipEventSynchronize(b);
+    float ms = 0;
+    (void)hipEventElapsedTime(&ms, a, b);
+    if (ms / reps < best) best = ms / reps, bv = v;
   }
+  ctx->rhs_var[d] = bv;
+  if (best_ms) best_ms[d] = best;
   (void)hipEventDestroy(a);
   (void)hipEventDestroy(b);
   ctx->profiling = prof;

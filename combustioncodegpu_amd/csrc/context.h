@@ -74,11 +74,11 @@ struct cfx_ctx {
   Table t_tile;                                // LU-SGS sweeps: one workgroup per (j, k) tile column
   int n_tplanes = 0;                           // LU-SGS tile hyperplanes of the largest block
   bool lusgs = false;
-  Table t_rhs[2][kNVar2];                      // 2-D: pencil tiles per direction and variant
+  Table t_rhs[kNVar2];                         // 2-D: RHS tiles per variant
+  Table t_plane;                               // 2-D: the points of the plane k = 0 with its ghosts
   Table t_march[kNVar3];                       // 3-D: marching workgroups per variant
   int march_chunk[kNVar3] = {};                // ... and the planes each marches through at most
   bool march_big = false;                      // a block's metric fields pass 4 GiB
-  int occ[2][2][kNVar2] = {};                  // 2-D: resident workgroups per CU [fp32][dir][variant]
   int n_cu = 256;
   int rhs_var[3] = {0, 0, 0}, rhs_persist[3] = {0, 0, 0};
   std::vector<FaceOp> ops;                     // BC ops in application order, then exchange ops
@@ -96,6 +96,7 @@ struct cfx_ctx {
   Schedule sched_mid, sched_bc_step;
   ExStrips strips{};
   int n_fused = 0;
+  bool plane_only = false;  // 2-D: no ghost fill reads more of the planes along k than the ring near the faces
   bool batched = true, use_graph = false;
   hipGraph_t graph = nullptr;
   hipGraphExec_t graph_exec = nullptr;

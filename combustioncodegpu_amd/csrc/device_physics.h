@@ -10,10 +10,21 @@
 #include <hip/hip_runtime.h>
 
 #include <type_traits>
+#include <utility>
 
 #include "cfx_types.h"
 
 namespace cfx {
+
+// f(integral_constant<int, I>) for I = 0..N-1, unrolled at compile time.
+template <class F, int... I>
+__device__ __forceinline__ void static_for_impl(F &&f, std::integer_sequence<int, I...>) {
+  (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, class F>
+__device__ __forceinline__ void static_for(F &&f) {
+  static_for_impl(f, std::make_integer_sequence<int, N>{});
+}
 
 // The species table is read through the constant address space: every index
 // into it is uniform across the wavefront, so the loads become scalar loads
@@ -188,34 +199,24 @@ __device__ __forceinline__ R on_all_lanes(R v) {
 
 // The NASA-7 range every lane of the wavefront is in, for every species:
 // kRangeHi (all in the high set), kRangeLo (all in the low set, above
-// t_low), kRangeEach (each lane in one of the two; asked for with EACH), or
-// kRangeMixed.  Smooth fields put most wavefronts on one side of t_mid; those
+// t_low), kRangeEach (each lane in one of the two), or kRangeMixed.  Smooth fields put most wavefronts on one side of t_mid; those
 // evaluate one polynomial set instead of both (the value is the same bit for
 // bit: the general path selects the same expression).
 constexpr int kRangeMixed = 0, kRangeLo = 1, kRangeHi = 2, kRangeEach = 3;
-template <typename R, bool EACH = false>
+template <typename R>
 __device__ __forceinline__ int thermo_range(SpeciesPtrT<R> sp, R t0, R t1) {
   const R hf = R(sp->hi_from), lf = R(sp->lo_from), lt = R(sp->lo_to);
   const bool h0 = t0 >= hf, h1 = t1 >= hf, l0 = t0 >= lf && t0 < lt, l1 = t1 >= lf && t1 < lt;
   if (__all(h0 && h1)) return kRangeHi;
   if (__all(l0 && l1)) return kRangeLo;
-  if constexpr (EACH)
-    if (__all((h0 || l0) && (h1 || l1))) return kRangeEach;
+  if (__all((h0 || l0) && (h1 || l1))) return kRangeEach;
   return kRangeMixed;
 }
 
-// h and cp of one species from its thermo record c (c[i] = value i of the
-// record: constant memory read with scalar loads, or a copy in LDS).
-// RG: kRangeMixed (per-lane selection), or the wavefront's single range.
-template <typename R, int RG = kRangeMixed, typename C>
+// h and cp of one species from its thermo record c, each lane in its own range
+template <typename R, typename C>
 __device__ __forceinline__ void thermo_h_cp(const C &c, R t, R &h, R &cp) {
   auto p5 = [&](int o) { return R(c[o]) + t * (R(c[o + 1]) + t * (R(c[o + 2]) + t * (R(c[o + 3]) + t * R(c[o + 4])))); };
-  if constexpr (RG != kRangeMixed) {
-    const int r = RG == kRangeHi ? 1 : 0;
-    cp = p5(kThCp + 5 * r);
-    h = t * p5(kThH + 6 * r) + R(c[kThH + 6 * r + 5]);
-    return;
-  }
   const R cp_lo = p5(kThCp), cp_hi = p5(kThCp + 5);
   const R h_lo = t * p5(kThH) + R(c[kThH + 5]);
   const R h_hi = t * p5(kThH + 6) + R(c[kThH + 11]);
@@ -236,14 +237,10 @@ __device__ __forceinline__ void species_h_cp(SpeciesPtrT<R> sp, int l, R t, R &h
 // h_l(T) alone (the same value as thermo_h_cp's h), for loops that need no
 // cp: the marker on the selected cp would otherwise keep both cp
 // polynomials alive.
-template <typename R, int RG = kRangeMixed>
+template <typename R>
 __device__ __forceinline__ R species_h(SpeciesPtrT<R> sp, int l, R t) {
   const auto &c = sp->th[l].v;
   auto p5 = [&](int o) { return R(c[o]) + t * (R(c[o + 1]) + t * (R(c[o + 2]) + t * (R(c[o + 3]) + t * R(c[o + 4])))); };
-  if constexpr (RG != kRangeMixed) {
-    const int r = RG == kRangeHi ? 1 : 0;
-    return t * p5(kThH + 6 * r) + R(c[kThH + 6 * r + 5]);
-  }
   const R h_lo = t * p5(kThH) + R(c[kThH + 5]);
   const R h_hi = t * p5(kThH + 6) + R(c[kThH + 11]);
   const R hp = on_all_lanes<R>(t >= R(c[kThTmid]) ? h_hi : h_lo);
@@ -251,66 +248,45 @@ __device__ __forceinline__ R species_h(SpeciesPtrT<R> sp, int l, R t) {
   return t < tl ? R(c[kThHtlow]) + R(c[kThCptlow]) * (t - tl) : hp;
 }
 
-// Where a kernel reads the thermo records from: constant memory, or with the
-// mixture coefficients copied into LDS (2 x NS records of 8, range 0 first),
-// where each lane can have a range of its own (kEach).
-template <typename R>
-struct ThermoConst {
-  static constexpr bool kEach = false;
-  SpeciesPtrT<R> sp;
-  typedef R V8 __attribute__((ext_vector_type(8)));
-  __device__ auto rec(int l) const { return sp->th[l].v; }
-  __device__ auto mix(bool hi) const {
-    const auto *tab = (const __attribute__((address_space(4))) V8 *)(hi ? &sp->mix[1][0] : &sp->mix[0][0]);
-    return [tab](int l) { return tab[l]; };
-  }
-};
+// The mixture coefficients of a kernel: a copy of the table in LDS (2 x NS
+// records of 8, range 0 first).  Read as constant memory only a few records
+// fit the scalar registers, so that every one or two species wait for a scalar
+// load; the LDS copy (broadcast reads) keeps many reads in flight, and lets
+// each lane have a range of its own: an FP64 RHS wavefront's AUSM+ phase took
+// 3.4k cycles with scalar loads, of which it issued 1.6k.
 template <int NS, typename R>
 struct ThermoLds {
-  static constexpr bool kEach = true;
   SpeciesPtrT<R> sp;
   const R *lds;
   __device__ auto rec(int l) const { return sp->th[l].v; }
-  __device__ auto mix(bool hi) const {
-    const R *tab = lds + (hi ? NS * 8 : 0);
-    return [tab](int l) { return tab + 8 * l; };
-  }
+  __device__ const R *mix(bool hi) const { return lds + (hi ? NS * 8 : 0); }
 };
 
 // H_k = sum_l w_l h_{l,k}, k = 0..5, with the coefficients of range rg at
 // temperature t (kRangeLo, kRangeHi, or by lane with kRangeEach), N sums at
-// once over the weights w(n, l).  TH is where the records are read from.
-// Constant memory: the address is formed once and a record read as one vector
-// (a single scalar load); but only a few records fit the scalar registers, so
-// that every one or two species wait for a scalar load.  A copy in LDS
-// (broadcast reads) keeps many reads in flight: an FP64 RHS wavefront's AUSM+
-// phase took 3.4k cycles with scalar loads, of which it issued 1.6k.
+// once over the weights w(n, l).
 template <int NS, int N, typename R, typename TH, typename W>
 __device__ __forceinline__ void mixture_sum(const TH &th, int rg, const R *t, W w, R (*H)[6]) {
-  auto add = [&](const auto &c, int n, int l) {
+  auto add = [&](const R *c, int n, int l) {
     const R x = w(n, l);
 #pragma unroll
     for (int k = 0; k < 6; ++k) H[n][k] = l == 0 ? x * c[k] : H[n][k] + x * c[k];
   };
-  if constexpr (TH::kEach && N > 1) {
-    if (rg == kRangeEach) {
-      const R hf = R(th.sp->hi_from);
+  const R hf = R(th.sp->hi_from);
+  if (N > 1 && rg == kRangeEach) {
 #pragma unroll
-      for (int n = 0; n < N; ++n) {
-        const auto tab = th.mix(t[n] >= hf);
+    for (int n = 0; n < N; ++n) {
+      const R *tab = th.mix(t[n] >= hf);
 #pragma unroll
-        for (int l = 0; l < NS; ++l) add(tab(l), n, l);
-      }
-      return;
+      for (int l = 0; l < NS; ++l) add(tab + 8 * l, n, l);
     }
+    return;
   }
-  const auto tab = th.mix(TH::kEach && N == 1 ? t[0] >= R(th.sp->hi_from) : rg == kRangeHi);
+  const R *tab = th.mix(N == 1 ? t[0] >= hf : rg == kRangeHi);
 #pragma unroll
-  for (int l = 0; l < NS; ++l) {
-    const auto c = tab(l);
+  for (int l = 0; l < NS; ++l)
 #pragma unroll
-    for (int n = 0; n < N; ++n) add(c, n, l);
-  }
+    for (int n = 0; n < N; ++n) add(tab + 8 * l, n, l);
 }
 
 // h(T) and cp(T) = dh/dT of a mixture from its summed enthalpy coefficients
@@ -407,14 +383,6 @@ __device__ __forceinline__ void muscl_n(const R (*q)[4], R *l, R *r) {
     for (int n = 0; n < N; ++n) l[n] = q[n][1], r[n] = q[n][2];
   }
 }
-template <typename R>
-__device__ __forceinline__ void muscl(const SchemeDev &S, R q0, R q1, R q2, R q3, R &l, R &r) {
-  const R q[1][4] = {{q0, q1, q2, q3}};
-  if (S.reconstruction != 2) muscl_n<2, 1, R>(q, &l, &r);
-  else if (S.limiter == 1) muscl_n<1, 1, R>(q, &l, &r);
-  else muscl_n<0, 1, R>(q, &l, &r);
-}
-
 // AUSM+ flux (InviscidScheme.cu:39-106) from the reconstructed face states
 // pl/pr = (rho,u,v,w,p,Y..) and the face area vector k = 0.5(J_L grad_L +
 // J_R grad_R) of the face direction; the face temperature, energy and gamma
@@ -440,7 +408,7 @@ __device__ __forceinline__ void ausm_from_states(SpeciesPtrT<R> sp, const TH &th
 #pragma unroll
     for (int n = 0; n < 2; ++n) x[n] = P[n][4], y[n] = P[n][0] * w[n];
     fdiv_n<2, R>(x, y, t);
-    const int rg = thermo_range<R, TH::kEach>(sp, t[0], t[1]);
+    const int rg = thermo_range<R>(sp, t[0], t[1]);
     if (rg != kRangeMixed) {
       // every lane in one range: the mixture's polynomial first
       // (six coefficients, each summed over the species), evaluated once, in

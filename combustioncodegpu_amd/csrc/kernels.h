@@ -55,47 +55,32 @@ inline int march_groups(const int m[3], const MarchTile &t, int chunk) {
 using MarchFn = int (*)(const Batch &b, int chunk, int big, const SpeciesDev *sp, const SchemeDev &S, hipStream_t st);
 using OccFn = int (*)();  // resident workgroups per CU of the kernel
 
-// 2-D: per face direction, the pencil tiles (faces along the direction x two
-// tangential extents) and the tile-group width G that the autotuner chooses
-// among.  Index v of each list is "variant v" of that direction.
-// w32: target waves per SIMD of the FP32 (mixed-precision) kernel; FP64
-// kernels target 2.
-struct PencilTile {
-  int ta, tb, tc, g, w32;
+// 2-D: one launch over tiles of tx x ty cells (rhs_plane.h); variant v is
+// shape v.
+struct PlaneTile {
+  int tx, ty;
 };
 constexpr int kNVar2 = 2;
-constexpr PencilTile kTiles2[2][kNVar2] = {{{32, 8, 1, 1, 3}, {64, 4, 1, 1, 3}}, {{16, 16, 1, 1, 3}, {32, 8, 1, 1, 3}}};
+constexpr PlaneTile kTiles2[kNVar2] = {{16, 15}, {32, 7}};
+inline int plane_groups(const int m[3], const PlaneTile &t) {
+  return (m[0] + t.tx - 1) / t.tx * ((m[1] + t.ty - 1) / t.ty);
+}
+// planar: the ghost planes along k equal the plane, and are not read
+using PlaneFn = int (*)(const Batch &b, int planar, const SpeciesDev *sp, const SchemeDev &S, hipStream_t st);
 
 inline int rhs_variants(int dim) { return dim == 3 ? kNVar3 : kNVar2; }
 
-// Tiles one pencil launch of shape s covers on a block of m[3] points
-// (including the padding tiles of partial G x G groups).
-inline int pencil_tiles(const int m[3], int dir, const PencilTile &s) {
-  const int a = dir, b = dir == 0 ? 1 : 0, c = dir == 2 ? 1 : 2;
-  const int nta = (m[a] + s.ta - 2) / (s.ta - 1);
-  const int ntb = (m[b] + s.tb - 1) / s.tb, ntc = (m[c] + s.tc - 1) / s.tc;
-  if (s.g == 0) return nta * ntb * ntc;
-  return nta * s.g * s.g * ((ntb + s.g - 1) / s.g) * ((ntc + s.g - 1) / s.g);
-}
-
-// grid: workgroups launched (a multiple of 8, at most the padded tile count)
-using RhsFn = int (*)(const Batch &b, int grid, const SpeciesDev *sp, const SchemeDev &S, int accumulate,
-                      hipStream_t st);
-struct RhsEntry {
-  RhsFn launch;
-  OccFn occupancy;
-};
-
 struct KernelSet64 {
   int present;
-  int (*props)(const Batch &b, const SpeciesDev *sp, const SchemeDev &S, hipStream_t st);
+  // plane: only the plane k = 0 of 2-D blocks (a batch of their planes)
+  int (*props)(const Batch &b, int plane, const SpeciesDev *sp, const SchemeDev &S, hipStream_t st);
   int (*cv_from_bv)(const Batch &b, const SpeciesDev *sp, const SchemeDev &S, hipStream_t st);
   int (*update)(const Batch &b, const SpeciesDev *sp, const SchemeDev &S, int mixed, int stage, const double *dt,
                 int *flags, unsigned long long *newton_fail, hipStream_t st);
   // ops[0..nops) with workgroup prefix off[0..nops], total workgroups
   int (*face_ops)(const BlockView *views, const FaceOp *ops, const int *off, int nops, int total,
                   const SpeciesDev *sp, const SchemeDev &S, const InflowDev *inflow, hipStream_t st);
-  RhsEntry rhs2[2][kNVar2];
+  PlaneFn plane[kNVar2];
   MarchFn march;
   OccFn march_occ;
   // surrogate training set: n samples of (T, log p, Y) and log(mu, kappa,
@@ -113,11 +98,11 @@ struct KernelSet64 {
 struct MlpDev;
 struct KernelSet32 {
   int present;
-  int (*props)(const Batch &b, const SpeciesDev *sp, const SchemeDev &S, hipStream_t st);
+  int (*props)(const Batch &b, int plane, const SpeciesDev *sp, const SchemeDev &S, hipStream_t st);
   // properties with the surrogate transport (mixed precision)
   int (*props_mlp)(const Batch &b, const SpeciesDev *sp, const SchemeDev &S, const MlpDev *mlp, const void *ops,
                    const float *bias, unsigned long long *counters, hipStream_t st);
-  RhsEntry rhs2[2][kNVar2];
+  PlaneFn plane[kNVar2];
   MarchFn march;
   OccFn march_occ;
 };
@@ -151,6 +136,7 @@ int launch_residual_partial(const Batch &b, double *partial, hipStream_t st);
 int launch_residual_final(const double *partial, int n, double *out, hipStream_t st);
 // every component of the strips, one lane per component, the fields over the wavefronts
 int launch_exchange_strips(const BlockView *views, const ExStrips &x, int ns, int mixed, hipStream_t st);
-int launch_eliminate_k(const BlockView &B, int ns, hipStream_t st);
+// ring: only the points that a ghost fill reads
+int launch_eliminate_k(const BlockView &B, int ns, int ring, hipStream_t st);
 
 }  // namespace cfx

@@ -224,12 +224,14 @@ __global__ void __launch_bounds__(kStripTpb) exchange_strip_kernel(const BlockVi
   }
 }
 
-// eliminate_k_gradient (Field.cu:268-292), 2-D only
-__global__ void eliminate_k_kernel(BlockView view, int ns) {
+// eliminate_k_gradient (Field.cu:268-292), 2-D only; ring: only for the points
+// that a ghost fill reads, the ghosts and ngg + 1 layers behind every face
+__global__ void eliminate_k_kernel(BlockView view, int ns, int ring) {
   const GView B = gview(view);
   const int i = (int)(blockIdx.x * blockDim.x + threadIdx.x) - kNgg;
   const int j = (int)(blockIdx.y * blockDim.y + threadIdx.y) - kNgg;
   if (i >= B.mx + kNgg || j >= B.my + kNgg) return;
+  if (ring && i > kNgg && i < B.mx - 1 - kNgg && j > kNgg && j < B.my - 1 - kNgg) return;
   const long long np = B.np;
   const long long p0 = pidx(B, i, j, 0);
   for (int k = 1; k <= kNgg; ++k) {
@@ -536,10 +538,10 @@ int launch_exchange_strips(const BlockView *views, const ExStrips &x, int ns, in
   return (int)hipGetLastError();
 }
 
-int launch_eliminate_k(const BlockView &B, int ns, hipStream_t st) {
+int launch_eliminate_k(const BlockView &B, int ns, int ring, hipStream_t st) {
   const dim3 tpb(16, 16, 1);
   const dim3 g((B.px + 15) / 16, (B.py + 15) / 16, 1);
-  eliminate_k_kernel<<<g, tpb, 0, st>>>(B, ns);
+  eliminate_k_kernel<<<g, tpb, 0, st>>>(B, ns, ring);
   return (int)hipGetLastError();
 }
 

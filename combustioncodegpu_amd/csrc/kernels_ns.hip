@@ -11,7 +11,7 @@
 #include "kernels.h"
 #include "mlp.h"
 #include "rhs_march.h"
-#include "rhs_pencil.h"
+#include "rhs_plane.h"
 
 #ifndef CFX_NS
 #error "CFX_NS (species count) must be defined"
@@ -123,9 +123,10 @@ __device__ __forceinline__ void wilke_point(SpeciesPtrT<R> sp, const SchemeDev &
     out[2 + l] = fabs(X[l] - R(1)) < R(1e-3) ? mus : fdiv<R>((R(1) - Y[l]) * mu, (R(1) - X[l]) * R(S.sc));
 }
 
-// Properties over the padded range.  In R = float (mixed precision) the
+// Properties over the padded range, or the plane k = 0 of it alone (PLANE, 2-D:
+// its rows are contiguous).  In R = float (mixed precision) the
 // kernel also writes the FP32 copies of the primitives the FP32 RHS reads.
-template <typename R>
+template <typename R, bool PLANE>
 __global__ void __launch_bounds__(kTpb) props_kernel(const BlockView *__restrict__ views, const int *__restrict__ off,
                                                      int nb, const SpeciesDev *__restrict__ spg, SchemeDev S) {
   const SpeciesPtrT<R> sp = const_table<R>(spg);
@@ -133,8 +134,9 @@ __global__ void __launch_bounds__(kTpb) props_kernel(const BlockView *__restrict
   const GView B = gview(views[pw.blk]);
   const long long np = B.np;
   constexpr bool f32 = sizeof(R) == 4;
-  const long long p = pw.base + threadIdx.x;
-  if (p >= np) return;
+  const long long q = pw.base + threadIdx.x;
+  if (q >= (PLANE ? B.sz : np)) return;
+  const long long p = PLANE ? kNgg * B.sz + q : q;
   const R t = R(B.bv[5 * np + p]);
   R out[4 + (NS > 0 ? NS : 0)];
   R Y[NSA];
@@ -178,41 +180,29 @@ __global__ void __launch_bounds__(kTpb) props_kernel(const BlockView *__restrict
 }
 
 template <typename R>
-int launch_props(const Batch &b, const SpeciesDev *sp, const SchemeDev &S, hipStream_t st) {
+int launch_props(const Batch &b, int plane, const SpeciesDev *sp, const SchemeDev &S, hipStream_t st) {
   if (b.total <= 0) return 0;
-  props_kernel<R><<<b.total, kTpb, 0, st>>>(b.views, b.off, b.nb, sp, S);
+  if (plane)
+    props_kernel<R, true><<<b.total, kTpb, 0, st>>>(b.views, b.off, b.nb, sp, S);
+  else
+    props_kernel<R, false><<<b.total, kTpb, 0, st>>>(b.views, b.off, b.nb, sp, S);
   return (int)hipGetLastError();
 }
 
 // ------------------------------------------------------------------- RHS ---
-// FP64 pencils (2-D) at 2 waves per SIMD; FP32 needs half the registers and
-// targets 3.
-// grid < padded tile count: the persistent kernel strides through the tiles
-template <int DIR, int V, typename R>
-int launch_rhs_dir(const Batch &b, int grid, const SpeciesDev *sp, const SchemeDev &S, int accumulate,
-                   hipStream_t st) {
-  constexpr PencilTile s = kTiles2[DIR][V];
-  constexpr int WPE = sizeof(R) == 8 ? 2 : s.w32;
+// 2-D.  FP64 with species takes all the registers of 2 waves per SIMD; air and
+// FP32 fit twice that.
+template <int V, typename R>
+int launch_rhs_plane(const Batch &b, int planar, const SpeciesDev *sp, const SchemeDev &S, hipStream_t st) {
+  constexpr PlaneTile t = kTiles2[V];
+  constexpr int WPE = sizeof(R) == 8 && NS > 0 ? 2 : 4;
   if (b.total <= 0) return 0;
   const int padded = (b.total + 7) / 8 * 8;
-  if (grid < padded)
-    rhs_pencil_kernel<NS, DIR, s.ta, s.tb, s.tc, WPE, R, s.g, true>
-        <<<grid, s.ta * s.tb * s.tc, 0, st>>>(b.views, b.off, b.nb, padded, sp, S, accumulate);
+  if (planar)
+    rhs_plane_kernel<NS, t.tx, t.ty, WPE, R, true><<<padded, 512, 0, st>>>(b.views, b.off, b.nb, padded, sp, S);
   else
-    rhs_pencil_kernel<NS, DIR, s.ta, s.tb, s.tc, WPE, R, s.g, false>
-        <<<padded, s.ta * s.tb * s.tc, 0, st>>>(b.views, b.off, b.nb, padded, sp, S, accumulate);
+    rhs_plane_kernel<NS, t.tx, t.ty, WPE, R, false><<<padded, 512, 0, st>>>(b.views, b.off, b.nb, padded, sp, S);
   return (int)hipGetLastError();
-}
-
-template <int DIR, int V, typename R>
-int occupancy_rhs_dir() {
-  constexpr PencilTile s = kTiles2[DIR][V];
-  constexpr int WPE = sizeof(R) == 8 ? 2 : s.w32;
-  int n = 0;
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(
-          &n, rhs_pencil_kernel<NS, DIR, s.ta, s.tb, s.tc, WPE, R, s.g, true>, s.ta * s.tb * s.tc, 0) != hipSuccess)
-    return 0;
-  return n;
 }
 
 template <typename R>
@@ -248,10 +238,8 @@ template <typename R, typename Set>
 void register_rhs(Set &k) {
   k.march = launch_rhs_march<R>;
   k.march_occ = occupancy_rhs_march<R>;
-  k.rhs2[0][0] = {launch_rhs_dir<0, 0, R>, occupancy_rhs_dir<0, 0, R>};
-  k.rhs2[0][1] = {launch_rhs_dir<0, 1, R>, occupancy_rhs_dir<0, 1, R>};
-  k.rhs2[1][0] = {launch_rhs_dir<1, 0, R>, occupancy_rhs_dir<1, 0, R>};
-  k.rhs2[1][1] = {launch_rhs_dir<1, 1, R>, occupancy_rhs_dir<1, 1, R>};
+  k.plane[0] = launch_rhs_plane<0, R>;
+  k.plane[1] = launch_rhs_plane<1, R>;
 }
 
 #if CFX_PREC == 64

@@ -33,7 +33,7 @@
 // 9 species fill the LDS, so a larger tile does not fit).
 #pragma once
 
-#include "rhs_pencil.h"
+#include "device_physics.h"
 
 namespace cfx {
 
@@ -66,7 +66,8 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(WPE, WP
   __shared__ __attribute__((aligned(16))) R sm[P::TOTAL];
   const SpeciesPtrT<R> sp = const_table<R>(spg);
   const int total = off[nb] - off[0];
-  // contiguous runs of workgroups per XCD (see rhs_pencil_tile)
+  // workgroups are dealt to the 8 XCDs round-robin: each works through a
+  // contiguous run of columns and keeps their halos in its own L2
   const int lid = ((int)blockIdx.x & 7) * (padded >> 3) + ((int)blockIdx.x >> 3);
   if (lid >= total) return;  // uniform per workgroup
   const int wgi = __builtin_amdgcn_readfirstlane(lid + off[0]);
@@ -474,7 +475,7 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(WPE, WP
             __builtin_amdgcn_sched_barrier(0);
           });
           // sum_l dp_l h_l(Ta): as the mixture polynomial where every lane is in one range
-          const int vrg = thermo_range<R, true>(sp, Ta, Ta);
+          const int vrg = thermo_range<R>(sp, Ta, Ta);
           if (vrg != kRangeMixed) {
             R H2[1][6];
             mixture_sum<NS, 1, R>(th, vrg, &Ta, [&](int, int s) { return dp[s]; }, H2);

@@ -301,24 +301,22 @@ int cfx_schedule_info(cfx_ctx *ctx, int *n_ops, int *n_levels);
 /* RHS variants and autotuner (no counterpart in the reference, whose
  * inviscid kernels use fixed 64-point lines, TimeAdvanceFunc.cu:38-154).
  * Results do not depend on the choice.
- * 2-D: the RHS runs one kernel per face direction; each direction has
- * cfx_rhs_variants() tile shapes, and a persistence factor p (0: one
- * workgroup per tile; p > 0: p x resident-workgroups-per-CU x CUs
- * workgroups looping over the tiles).
+ * 2-D: one kernel forms both directions; the variant of direction 1 selects
+ * the tile shape (0: 16 x 15 cells, 1: 32 x 7).
  * 3-D: one kernel forms all directions, each workgroup marching along k;
  * the variant of direction 2 selects how many planes it marches through
  * (0, the default: planned for the context's blocks; 1..4: at most 8, 16, 32,
- * 64; 5: the whole block).  The variants of directions 0 and 1 and the
- * persistence factors are checked and kept, and have no effect. */
+ * 64; 5: the whole block).
+ * The variants of the other directions and the persistence factors are
+ * checked and kept, and have no effect. */
 int cfx_rhs_variants(cfx_ctx *ctx);
 /* Same tile variant in every direction, persistence 0. */
 int cfx_set_rhs_variant(cfx_ctx *ctx, int variant);
 int cfx_set_rhs_tiles(cfx_ctx *ctx, const int variant[3], const int persist[3]);
 int cfx_get_rhs_tiles(cfx_ctx *ctx, int variant[3], int persist[3]);
-/* Times every (variant, persistence) of every direction on the context's
- * blocks, reps launches each, and keeps the fastest; best_ms[3] (may be
- * NULL) receives the per-direction time of the choice (3-D: the one launch's
- * time in best_ms[2], 0 in the others).  Leaves dq undefined. */
+/* Times every variant on the context's blocks, reps launches each, and keeps
+ * the fastest; best_ms[3] (may be NULL) receives the launch's time in the last
+ * direction's place and 0 in the others.  Leaves dq undefined. */
 int cfx_autotune(cfx_ctx *ctx, int reps, double *best_ms);
 
 /* ------------------------------------------------ transport surrogate ---
