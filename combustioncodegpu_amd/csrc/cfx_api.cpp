@@ -1410,13 +1410,13 @@ int cfx_download(cfx_ctx *ctx, int blk, int what, double *dst) {
     const float *s32 = what == CFX_PROPS ? V.props32 : V.dq32;
     const size_t n32 = what == CFX_PROPS ? (4 + ctx->ns) * np : ctx->nv * ni;
     std::vector<float> tmp(n32);
-    CFX_TRY((int)hipMemcpy(tmp.data(), s32, sizeof(float) * n32, hipMemcpyDeviceToHost));
+    CFX_TRY(ctx->to_host.to_host(tmp.data(), s32, sizeof(float) * n32, ctx->stream));
     for (size_t i = 0; i < n32; ++i) dst[i] = tmp[i];
     return 0;
   }
   if (V.mixed && what == CFX_YK) {  // the mixed path keeps Y only as rho*Y / rho
     std::vector<double> cv(ctx->nv * np);
-    CFX_TRY((int)hipMemcpy(cv.data(), V.cv, sizeof(double) * cv.size(), hipMemcpyDeviceToHost));
+    CFX_TRY(ctx->to_host.to_host(cv.data(), V.cv, sizeof(double) * cv.size(), ctx->stream));
     for (size_t p = 0; p < np; ++p) {
       const double ir = 1.0 / cv[p];
       for (int l = 0; l < ctx->ns; ++l) dst[l * np + p] = cv[(5 + l) * np + p] * ir;
@@ -1431,7 +1431,7 @@ int cfx_download(cfx_ctx *ctx, int blk, int what, double *dst) {
     case CFX_DQ: src = V.dq, n = ctx->nv * ni; break;
     case CFX_DTLOCAL: src = V.dt_local, n = ni; break;
     case CFX_METRIC:
-      CFX_TRY((int)hipMemcpy(dst, V.metric, sizeof(double) * 9 * np, hipMemcpyDeviceToHost));
+      CFX_TRY(ctx->to_host.to_host(dst, V.metric, sizeof(double) * 9 * np, ctx->stream));
       CFX_TRY((int)hipMemcpy(dst + 9 * np, V.jac, sizeof(double) * np, hipMemcpyDeviceToHost));
       return 0;
     case CFX_COORD: {
@@ -1445,7 +1445,7 @@ int cfx_download(cfx_ctx *ctx, int blk, int what, double *dst) {
     }
     default: return ctx->fail(CFX_E_ARG, "unknown download selector");
   }
-  if (n) CFX_TRY((int)hipMemcpy(dst, src, sizeof(double) * n, hipMemcpyDeviceToHost));
+  if (n) CFX_TRY(ctx->to_host.to_host(dst, src, sizeof(double) * n, ctx->stream));
   return 0;
 }
 

@@ -9,6 +9,7 @@
 
 #include "../../include/cfx.h"
 #include "cfx_types.h"
+#include "host_copy.h"
 #include "kernels.h"
 #include "mesh.h"
 #include "mlp.h"
@@ -60,6 +61,7 @@ struct cfx_ctx {
   std::vector<WallDev> walls;
   std::vector<BcOp> bc_order;
   hipStream_t stream = nullptr;
+  HostCopy to_host;
   double *d_dt = nullptr;  // device dt; its bits are reduced with atomicMin
   double *d_res = nullptr;
   int *d_flags = nullptr;
