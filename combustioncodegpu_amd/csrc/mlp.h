@@ -29,6 +29,7 @@
 
 namespace cfx {
 
+typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
@@ -165,46 +166,6 @@ __device__ __forceinline__ f32x4 load_bias(const float *__restrict__ bias, int l
 }
 __device__ __forceinline__ f32x4 load_bias(lds_ptr<const f32x4> bias, int layer, int mb, int lane) {
   return bias[(layer * kMlpH + 16 * mb) / 4 + (lane >> 4)];
-}
-
-// Activations of one 16-point tile kept for the backward pass.
-struct MlpTile {
-  f32x4 z1[4], z2[4], z3[4];
-  bf16x8 h0, h1[2], h2[2], h3[2];
-  f32x4 y;
-};
-
-// Forward pass of one tile: x is the B operand of the normalised inputs.
-__device__ __forceinline__ void mlp_forward(const bf16x8 *__restrict__ ops, const float *__restrict__ bias,
-                                            bf16x8 x, MlpTile &t) {
-  const int lane = threadIdx.x & 63;
-  t.h0 = x;
-#pragma unroll
-  for (int mb = 0; mb < 4; ++mb) t.z1[mb] = mfma_bf16(load_op(ops, kF1 + mb, lane), x, load_bias(bias, 0, mb, lane));
-#pragma unroll
-  for (int kb = 0; kb < 2; ++kb) t.h1[kb] = pack_pair(silu4(t.z1[2 * kb]), silu4(t.z1[2 * kb + 1]));
-#pragma unroll
-  for (int mb = 0; mb < 4; ++mb) {
-    f32x4 a = load_bias(bias, 1, mb, lane);
-#pragma unroll
-    for (int kb = 0; kb < 2; ++kb) a = mfma_bf16(load_op(ops, kF2 + 2 * mb + kb, lane), t.h1[kb], a);
-    t.z2[mb] = a;
-  }
-#pragma unroll
-  for (int kb = 0; kb < 2; ++kb) t.h2[kb] = pack_pair(silu4(t.z2[2 * kb]), silu4(t.z2[2 * kb + 1]));
-#pragma unroll
-  for (int mb = 0; mb < 4; ++mb) {
-    f32x4 a = load_bias(bias, 2, mb, lane);
-#pragma unroll
-    for (int kb = 0; kb < 2; ++kb) a = mfma_bf16(load_op(ops, kF3 + 2 * mb + kb, lane), t.h2[kb], a);
-    t.z3[mb] = a;
-  }
-#pragma unroll
-  for (int kb = 0; kb < 2; ++kb) t.h3[kb] = pack_pair(silu4(t.z3[2 * kb]), silu4(t.z3[2 * kb + 1]));
-  f32x4 y = load_bias(bias, 3, 0, lane);
-#pragma unroll
-  for (int kb = 0; kb < 2; ++kb) y = mfma_bf16(load_op(ops, kF4 + kb, lane), t.h3[kb], y);
-  t.y = y;
 }
 
 // Forward pass for inference only (no activations kept), on the folded

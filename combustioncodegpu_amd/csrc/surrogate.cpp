@@ -263,22 +263,18 @@ int cfx_mlp_train(cfx_ctx *ctx, const cfx_mlp_config *cfg_in, cfx_mlp_report *re
     }
     return d2;
   };
+  // the training inputs' distances, for the envelope's radius
+  std::vector<double> d2s((size_t)n_train);
   {
-    // the envelope's radius: the envelope_quantile of the training inputs'
-    // distances (the network's largest held-out errors sit in the sparse
-    // tail of the input distribution, at the dominant species' rho*D)
-    std::vector<float> hxs((size_t)n_train * kMlpIO);
-    CFX_TRY((int)hipMemcpyAsync(hxs.data(), xs, sizeof(float) * hxs.size(), hipMemcpyDeviceToHost, ctx->stream));
+    MlpAxes ax;
+    ax.n = nin;
+    std::memcpy(ax.axis, m.pca, sizeof(ax.axis));
+    std::memcpy(ax.inv_var, m.pca_inv_var, sizeof(ax.inv_var));
+    double *d2 = sc.get<double>((size_t)n_train, rc);
+    if (rc) return ctx->fail(rc, "hipMalloc training distances");
+    CFX_TRY(launch_mlp_dist2(xs, n_train, ax, d2, ctx->stream));
+    CFX_TRY((int)hipMemcpyAsync(d2s.data(), d2, sizeof(double) * d2s.size(), hipMemcpyDeviceToHost, ctx->stream));
     CFX_TRY((int)hipStreamSynchronize(ctx->stream));
-    std::vector<double> d2s((size_t)n_train);
-    for (long long s = 0; s < n_train; ++s) d2s[(size_t)s] = dist2(hxs.data() + s * kMlpIO);
-    if (cfg.envelope_quantile >= 1.0) {
-      m.d2_max = (float)(*std::max_element(d2s.begin(), d2s.end()) * 1.0001);
-    } else {
-      const size_t r = (size_t)(cfg.envelope_quantile * (double)(n_train - 1));
-      std::nth_element(d2s.begin(), d2s.begin() + (long long)r, d2s.end());
-      m.d2_max = (float)d2s[r];
-    }
   }
   m.x_pure = kMlpPureX;
   m.check_tol = (float)cfg.check_tol;
@@ -309,8 +305,17 @@ int cfx_mlp_train(cfx_ctx *ctx, const cfx_mlp_config *cfg_in, cfx_mlp_report *re
   const double b1 = 0.9, b2 = 0.999;
   static const long long kPrimes[] = {1000003, 1000033, 1000037, 1000039, 1000081, 1000099, 1000117, 1000121,
                                       1000133, 1000151, 1000159, 1000171, 1000183, 1000187, 1000193, 1000199};
+  // every step leaves its parameters in the operands too
+  CFX_TRY(launch_mlp_pack(ctx->mlp_params, shp, ctx->mlp_ops, ctx->mlp_bias, 0, ctx->stream));
   std::vector<float> hloss(waves);
   double loss_first = -1.0, loss_last = -1.0;
+  auto read_loss = [&](double &l) {  // of the step queued last
+    int e = (int)hipMemcpyAsync(hloss.data(), loss, sizeof(float) * waves, hipMemcpyDeviceToHost, ctx->stream);
+    if (!e) e = (int)hipStreamSynchronize(ctx->stream);
+    l = 0.0;
+    for (float v : hloss) l += v;
+    return e;
+  };
   long long step = 0;
   for (int ep = 0; ep < cfg.epochs; ++ep) {
     long long mult = 1;
@@ -327,22 +332,26 @@ int cfx_mlp_train(cfx_ctx *ctx, const cfx_mlp_config *cfg_in, cfx_mlp_report *re
       const double lr = cfg.lr_final + 0.5 * (cfg.lr - cfg.lr_final) * (1.0 + std::cos(M_PI * frac));
       const double c1 = 1.0 / (1.0 - std::pow(b1, (double)(step + 1)));
       const double c2 = 1.0 / (1.0 - std::pow(b2, (double)(step + 1)));
-      CFX_TRY(launch_mlp_pack(ctx->mlp_params, shp, ctx->mlp_ops, ctx->mlp_bias, 0, ctx->stream));
       CFX_TRY(launch_mlp_train(xs, ts, n_train, b * cfg.batch, offset, mult, waves, ctx->mlp_ops, ctx->mlp_bias,
                                shp, scale, partial, loss, ctx->stream));
       CFX_TRY(launch_mlp_adam(ctx->mlp_params, ctx->mlp_m, ctx->mlp_v, partial, waves, P, (float)lr, (float)b1,
-                              (float)b2, 1e-8f, (float)c1, (float)c2, nullptr, ctx->stream));
-      if (b == 0 || b == steps_per_epoch - 1) {
-        CFX_TRY((int)hipMemcpyAsync(hloss.data(), loss, sizeof(float) * waves, hipMemcpyDeviceToHost, ctx->stream));
-        CFX_TRY((int)hipStreamSynchronize(ctx->stream));
-        double l = 0.0;
-        for (float v : hloss) l += v;
-        if (loss_first < 0) loss_first = l;
-        loss_last = l;
-      }
+                              (float)b2, 1e-8f, (float)c1, (float)c2, nullptr, shp, ctx->mlp_ops, ctx->mlp_bias,
+                              ctx->stream));
+      if (step == 0) CFX_TRY(read_loss(loss_first));
     }
   }
-  CFX_TRY(launch_mlp_pack(ctx->mlp_params, shp, ctx->mlp_ops, ctx->mlp_bias, 0, ctx->stream));
+  // the envelope's radius, while the GPU works through the queued steps: the
+  // envelope_quantile of the training inputs' distances (the network's largest
+  // held-out errors sit in the sparse tail of the input distribution, at the
+  // dominant species' rho*D)
+  if (cfg.envelope_quantile >= 1.0) {
+    m.d2_max = (float)(*std::max_element(d2s.begin(), d2s.end()) * 1.0001);
+  } else {
+    const size_t r = (size_t)(cfg.envelope_quantile * (double)(n_train - 1));
+    std::nth_element(d2s.begin(), d2s.begin() + (long long)r, d2s.end());
+    m.d2_max = (float)d2s[r];
+  }
+  if (step > 0) CFX_TRY(read_loss(loss_last));
   CFX_TRY(launch_mlp_pack(ctx->mlp_params, shp, ctx->mlp_ops_inf, ctx->mlp_bias_inf, 1, ctx->stream));
   (void)hipEventRecord(e2, ctx->stream);
   // ---- validation on the held-out samples
@@ -498,7 +507,7 @@ int cfx_mlp_gradient(cfx_ctx *ctx, const float *x, const float *t, int n, float 
   CFX_TRY(launch_mlp_train(dx, dt, n, 0, 0, 1, waves, ctx->mlp_ops, ctx->mlp_bias, shp, scale, partial, loss,
                            ctx->stream));
   CFX_TRY(launch_mlp_adam(ctx->mlp_params, ctx->mlp_m, ctx->mlp_v, partial, waves, P, 0.0f, 0.9f, 0.999f, 1e-8f, 1.0f,
-                          1.0f, g, ctx->stream));
+                          1.0f, g, shp, nullptr, nullptr, ctx->stream));
   std::vector<float> hl(waves);
   CFX_TRY((int)hipMemcpyAsync(grad, g, sizeof(float) * P, hipMemcpyDeviceToHost, ctx->stream));
   CFX_TRY((int)hipMemcpyAsync(hl.data(), loss, sizeof(float) * waves, hipMemcpyDeviceToHost, ctx->stream));
