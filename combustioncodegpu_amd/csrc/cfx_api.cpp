@@ -203,13 +203,9 @@ int chunks(long long n, int per) { return (int)((n + per - 1) / per); }
 
 int build_tables(cfx_ctx *ctx) {
   const int nb = (int)ctx->hb.size();
-  std::vector<int> pad(nb), in1(nb), dtc(nb), last(nb), res(nb), til(nb);
-  ctx->n_tplanes = 0;
+  std::vector<int> pad(nb), in1(nb), dtc(nb), last(nb), res(nb);
   for (int b = 0; b < nb; ++b) {
     const HostBlock &H = ctx->hb[b];
-    const int nt[3] = {chunks(H.mx, kLuTi), chunks(H.my, kLuTj), chunks(H.mz, kLuTk)};
-    til[b] = nt[1] * nt[2];
-    ctx->n_tplanes = std::max(ctx->n_tplanes, nt[0] + nt[1] + nt[2] - 2);
     pad[b] = chunks(H.np, kTpb);
     in1[b] = chunks(H.ni, kTpb);
     dtc[b] = chunks(H.ni, kTpb * kDtIter);
@@ -219,7 +215,7 @@ int build_tables(cfx_ctx *ctx) {
   int rc;
   if ((rc = upload_table(ctx, ctx->t_pad, pad)) || (rc = upload_table(ctx, ctx->t_int, in1)) ||
       (rc = upload_table(ctx, ctx->t_dt, dtc)) || (rc = upload_table(ctx, ctx->t_last, last)) ||
-      (rc = upload_table(ctx, ctx->t_res, res)) || (rc = upload_table(ctx, ctx->t_tile, til)))
+      (rc = upload_table(ctx, ctx->t_res, res)))
     return rc;
   if (ctx->dim != 2) return 0;
   std::vector<int> count(nb);
@@ -233,6 +229,32 @@ int build_tables(cfx_ctx *ctx) {
     if ((rc = upload_table(ctx, ctx->t_rhs[v], count))) return rc;
   }
   return 0;
+}
+
+// The order in which the sweeps of LU-SGS take the patches: by J + K, so that
+// the two patches a patch waits for stand before it.
+int plan_sweeps(cfx_ctx *ctx) {
+  if (!ctx->lusgs) return 0;
+  std::vector<LuPatch> all, own;
+  std::vector<int> count;
+  for (size_t b = 0; b < ctx->hb.size(); ++b) {
+    const int nj = chunks(ctx->hb[b].my, kLuP), nk = chunks(ctx->hb[b].mz, kLuP);
+    for (int d = 0; d <= nj + nk - 2; ++d)
+      for (int K = std::max(0, d - nj + 1); K <= std::min(d, nk - 1); ++K) {
+        all.push_back(LuPatch{(int)b, d - K, K});
+        own.push_back(LuPatch{0, d - K, K});
+      }
+    count.push_back(nj * nk);
+  }
+  std::stable_sort(all.begin(), all.end(), [](const LuPatch &x, const LuPatch &y) { return x.J + x.K < y.J + y.K; });
+  ctx->lu_off.assign(1, (int)all.size());
+  for (int c : count) ctx->lu_off.push_back(ctx->lu_off.back() + c);
+  all.insert(all.end(), own.begin(), own.end());
+  int rc = 0;
+  ctx->lu_order = ctx->dalloc<LuPatch>(all.size(), rc);
+  ctx->lu_ticket = ctx->dalloc<int>(1, rc);
+  if (rc) return rc;
+  return (int)hipMemcpy(ctx->lu_order, all.data(), sizeof(LuPatch) * all.size(), hipMemcpyHostToDevice);
 }
 
 // The marching RHS of a 3-D context: the planes per workgroup of every variant
@@ -883,19 +905,31 @@ int do_update(cfx_ctx *ctx, int stage) {
 }
 
 // LU-SGS solve (the implicit treatment of Driver.cu:156): coefficients, then
-// the forward and backward sweeps tile hyperplane by tile hyperplane; dq <- dQ
+// the forward and the backward sweep; dq <- dQ
 int do_lusgs(cfx_ctx *ctx) {
   const KernelSet64 &k = g_kernels64[ctx->ns];
   CFX_TRY(per_batch(ctx, ctx->t_int, [&](const Batch &b) {
     return ctx->timed_launch(K_UPDATE, [&] { return k.lusgs_coef(b, ctx->S, ctx->stream); });
   }));
-  for (int pass = 0; pass < 2; ++pass)
-    for (int n = 0; n < ctx->n_tplanes; ++n) {
-      const int tplane = pass == 0 ? n : ctx->n_tplanes - 1 - n;
-      CFX_TRY(per_batch(ctx, ctx->t_tile, [&](const Batch &b) {
-        return ctx->timed_launch(K_UPDATE, [&] { return k.lusgs_sweep(b, ctx->S, tplane, pass == 0, ctx->stream); });
-      }));
+  // blk < 0: every block in one launch
+  auto sweep = [&](int blk, int fwd) {
+    const Batch pts = blk < 0 ? ctx->all(ctx->t_int) : ctx->one(ctx->t_int, blk);
+    const int first = blk < 0 ? 0 : ctx->lu_off[blk], n = (blk < 0 ? ctx->lu_off[0] : ctx->lu_off[blk + 1]) - first;
+    const BlockView *views = blk < 0 ? ctx->views_dev : ctx->views_dev + blk;
+    CFX_TRY(ctx->timed_launch(K_UPDATE, [&] { return k.lusgs_reset(pts, ctx->lu_ticket, ctx->stream); }));
+    CFX_TRY(ctx->timed_launch(K_UPDATE, [&] {
+      return k.lusgs_sweep(views, ctx->lu_order + first, n, ctx->lu_ticket, ctx->S, fwd, ctx->d_flags, ctx->stream);
+    }));
+    return 0;
+  };
+  for (int fwd = 1; fwd >= 0; --fwd) {
+    if (ctx->batched) {
+      if (int rc = sweep(-1, fwd)) return rc;
+      continue;
     }
+    for (int b = 0; b < (int)ctx->views.size(); ++b)
+      if (int rc = sweep(b, fwd)) return rc;
+  }
   return 0;
 }
 
@@ -1312,7 +1346,14 @@ int cfx_create(const cfx_params *params, const cfx_species *species, const cfx_b
     V.qn = ctx->dalloc<double>(ctx->nv * ni, rc);
     V.dt_local = ctx->dalloc<double>(ni, rc);
     V.bv_last = ctx->dalloc<double>(4 * ni, rc);
-    if (ctx->lusgs) V.lus = ctx->dalloc<double>(4 * ni, rc);
+    if (ctx->lusgs) {
+      V.lus = ctx->dalloc<double>(4 * ni, rc);
+      // the implicit step has no stage base: its array takes the hand-over,
+      // unless the block is so thin that the patches' edges need more
+      const int m[3] = {H.mx, H.my, H.mz};
+      const size_t n = (size_t)lu_hand_over(m, ctx->ns);
+      V.luf = n <= ctx->nv * ni ? V.qn : ctx->dalloc<double>(n, rc);
+    }
     if (rc) return bail(ctx->fail(rc, "hipMalloc block arrays"));
     V.mixed = ctx->mixed ? 1 : 0;
     if (ctx->mixed) {
@@ -1352,6 +1393,7 @@ int cfx_create(const cfx_params *params, const cfx_species *species, const cfx_b
       ctx->n_cu = ncu;
   }
   if ((rc = plan_march(ctx))) return bail(ctx->fail(rc, "march table"));
+  if ((rc = plan_sweeps(ctx))) return bail(ctx->fail(rc, "sweep order"));
   e = hipDeviceSynchronize();
   if (e != hipSuccess) return bail(ctx->fail((int)e, "device setup"));
   *out = ctx;
@@ -1528,6 +1570,7 @@ int cfx_check(cfx_ctx *ctx, long long *n_newton_fail) {
   CFX_TRY((int)hipMemcpy(&flags, ctx->d_flags, sizeof(int), hipMemcpyDeviceToHost));
   CFX_TRY((int)hipMemcpy(&nf, ctx->d_newton, sizeof(nf), hipMemcpyDeviceToHost));
   if (n_newton_fail) *n_newton_fail = (long long)nf;
+  if (flags & 2) return ctx->fail((int)hipErrorLaunchTimeOut, "an LU-SGS sweep gave up waiting for a patch");
   if (flags) return ctx->fail(CFX_E_NONFINITE, "non-finite or non-positive rho/T/p in the update");
   if (nf) return ctx->fail(CFX_E_NEWTON, std::to_string(nf) + " Newton temperature inversions did not converge");
   return 0;

@@ -91,6 +91,7 @@ struct BlockView {
   double *metric, *jac;          // metric: 9 x np (xi_x..zeta_z), jac: np
   double *dq, *qn, *dt_local, *bv_last;
   double *lus;  // LU-SGS: D, then a_d for d = 0..2, each over the interior (null otherwise)
+  double *luf;  // LU-SGS: the hand-over between the patches of a sweep (lu_hand_over values; null otherwise)
   // mixed precision: FP32 copies of the RHS inputs (refreshed by the
   // properties kernel over the padded range) and the FP32 dq; null in FP64 mode
   int mixed;
@@ -101,6 +102,23 @@ struct BlockView {
   int fuse[6];
   int fuse_any;
 };
+
+// LU-SGS sweeps: patches of kLuP x kLuP columns along i; the patch (J, K) of a
+// block, in the order in which wavefronts take them (any patch behind (J-1, K)
+// and (J, K-1)); and the values a sweep hands from patch to patch.
+constexpr int kLuP = 4;
+struct LuPatch {
+  int blk, J, K;
+};
+// a third of the species, and the places of a cell's variables: (rho, rho V, E)
+// and three groups of species
+__host__ __device__ constexpr int lu_third(int ns) { return (ns + 2) / 3; }
+__host__ __device__ constexpr int lu_places(int ns) { return 5 + 3 * lu_third(ns); }
+__host__ __device__ inline long long lu_hand_over(const int m[3], int ns) {
+  const long long nj = (m[1] + kLuP - 1) / kLuP, nk = (m[2] + kLuP - 1) / kLuP;
+  const long long wj = m[1] < kLuP ? m[1] : kLuP, wk = m[2] < kLuP ? m[2] : kLuP;
+  return nj * nk * (m[0] + wj + wk - 2) * lu_places(ns) * kLuP * ((nj > 1 ? 1 : 0) + (nk > 1 ? 1 : 0));
+}
 
 // Pointers in the global address space.  A view loaded from device memory
 // (the block table) hands out generic pointers, for which the compiler emits
@@ -128,7 +146,7 @@ struct GView {
   int mx, my, mz;
   int px, py, pz;
   long long np, ni, sy, sz;
-  gptr<double> cv, bv, yk, props, metric, jac, dq, qn, dt_local, bv_last, lus;
+  gptr<double> cv, bv, yk, props, metric, jac, dq, qn, dt_local, bv_last, lus, luf;
   int mixed;
   gptr<float> bv32, yk32, props32, metric32, jac32, dq32;
   int fuse[6];
@@ -142,7 +160,7 @@ __device__ __forceinline__ GView gview(const BlockView &B) {
   g.cv = (gptr<double>)B.cv, g.bv = (gptr<double>)B.bv, g.yk = (gptr<double>)B.yk;
   g.props = (gptr<double>)B.props, g.metric = (gptr<double>)B.metric, g.jac = (gptr<double>)B.jac;
   g.dq = (gptr<double>)B.dq, g.qn = (gptr<double>)B.qn, g.dt_local = (gptr<double>)B.dt_local;
-  g.bv_last = (gptr<double>)B.bv_last, g.lus = (gptr<double>)B.lus;
+  g.bv_last = (gptr<double>)B.bv_last, g.lus = (gptr<double>)B.lus, g.luf = (gptr<double>)B.luf;
   g.mixed = B.mixed;
   g.bv32 = (gptr<float>)B.bv32, g.yk32 = (gptr<float>)B.yk32, g.props32 = (gptr<float>)B.props32;
   g.metric32 = (gptr<float>)B.metric32, g.jac32 = (gptr<float>)B.jac32, g.dq32 = (gptr<float>)B.dq32;

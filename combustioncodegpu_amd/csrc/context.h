@@ -73,8 +73,11 @@ struct cfx_ctx {
   BlockView *views_dev = nullptr;
   std::vector<double *> coords;  // per block: the (ngg+1)-layer coordinates built on the device
   Table t_pad, t_int, t_dt, t_last, t_res;     // point-kernel workgroup prefixes
-  Table t_tile;                                // LU-SGS sweeps: one workgroup per (j, k) tile column
-  int n_tplanes = 0;                           // LU-SGS tile hyperplanes of the largest block
+  // LU-SGS sweeps: the patches of all blocks (block index), then those of each
+  // block (index 0), in the order of their tickets
+  LuPatch *lu_order = nullptr;
+  std::vector<int> lu_off;                     // first entry of each block's own list, and the end
+  int *lu_ticket = nullptr;
   bool lusgs = false;
   Table t_rhs[kNVar2];                         // 2-D: RHS tiles per variant
   Table t_plane;                               // 2-D: the points of the plane k = 0 with its ghosts

@@ -19,9 +19,6 @@ constexpr int kTpb = 256;        // threads per workgroup of the point kernels
 constexpr int kDtIter = 8;       // points per thread of the time-step reduction
 constexpr int kLastIter = 4;     // points per thread of the last-step snapshot
 constexpr int kResIter = 8;      // points per thread of the residual partials
-// LU-SGS sweep tiles: kLuTi x kLuTj x kLuTk cells (i, j, k), one workgroup
-// each, whose first wavefront's lanes own the (j, k) columns
-constexpr int kLuTi = 4, kLuTj = 8, kLuTk = 8;
 
 // A batch of blocks: views[0..nb) with workgroup prefix off[0..nb] (device
 // pointers, off[0] need not be 0) and total = off[nb] - off[0] workgroups.
@@ -88,11 +85,12 @@ struct KernelSet64 {
   int (*mlp_samples)(const SpeciesDev *sp, const SchemeDev &S, long long n, unsigned long long seed,
                      const double lim[4], double alpha, double *x, double *y, hipStream_t st);
   // LU-SGS: the diagonal and neighbour coefficients over the interior (point
-  // batch), and the tiles of one tile hyperplane I + J + K = tplane of the
-  // forward (fwd = 1) or backward sweep (batch of one workgroup per (J, K)
-  // tile column of each block)
+  // batch); what a sweep expects of its hand-over and its ticket counter (point
+  // batch); and the forward (fwd = 1) or backward sweep of n patches
   int (*lusgs_coef)(const Batch &b, const SchemeDev &S, hipStream_t st);
-  int (*lusgs_sweep)(const Batch &b, const SchemeDev &S, int tplane, int fwd, hipStream_t st);
+  int (*lusgs_reset)(const Batch &b, int *ticket, hipStream_t st);
+  int (*lusgs_sweep)(const BlockView *views, const LuPatch *order, int n, int *ticket, const SchemeDev &S, int fwd,
+                     int *flags, hipStream_t st);
 };
 
 struct MlpDev;

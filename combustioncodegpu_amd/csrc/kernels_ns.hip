@@ -789,159 +789,361 @@ __global__ void __launch_bounds__(kTpb) lusgs_coef_kernel(const BlockView *__res
   B.lus[q] = diag;
 }
 
-// The sweeps in tiles of kLuTi x kLuTj x kLuTk cells.  Tiles (I, J, K) on
-// one tile hyperplane I + J + K = tplane depend only on tiles of the
-// previous one, so one launch runs a tile hyperplane, one workgroup per
-// tile.  The workgroup first stages in LDS, for its tile and the upstream
-// face layers around it (the cells at i0-1, j0-1, k0-1 for the forward
-// sweep, past the far faces for the backward one, final since an earlier
-// launch), each cell's dQ slot (R or dQ* on entry), conserved state,
-// pressure, gamma, J grad xi_d, a_d and D.  Lane (jl, kl) of a wavefront
-// then stands for the cell column (j, k), marching along i: at local step s
-// the cell il = s - jl - kl is updated, whose upstream neighbours were
-// updated at step s-1 or
-// are staged; every read of the dependent steps is an LDS read, and a
-// cell's slot is written once, after every read of its input.  The tile's
-// increments go back to dq at the end.  The divisions share a
-// Newton-refined reciprocal per denominator; the three neighbour terms of a
-// cell are formed by three wavefronts at once and added in a fixed order.
-constexpr int kLuEi = kLuTi + 1, kLuEj = kLuTj + 1, kLuEk = kLuTk + 1, kLuExt = kLuEi * kLuEj * kLuEk;
-// LDS slot of staged cell (i, j, k): i + kLuEi j + kLuSk k, the k planes one
-// slot apart so that the lanes of a step, which differ in j and k, spread
-// over the LDS banks (measured: bank-conflict cycles 40% of the LDS-active
-// cycles with kLuSk = 45, 7% with 46); kLuSlots slots per staged variable
-constexpr int kLuSk = kLuEi * kLuEj + 1, kLuSlots = (kLuEk - 1) * kLuSk + kLuEi * kLuEj;
-__device__ __forceinline__ int lu_slot(int i, int j, int k) { return (k * kLuSk + j * kLuEi) + i; }
-// a / b with r = frcp(b) shared by the quotients over one b: one residual
-// correction of a r (within an ulp of the IEEE quotient)
-__device__ __forceinline__ double lu_div(double a, double b, double r) {
-  const double q = a * r;
-  return fma(r, fma(-b, q, a), q);
+// The sweeps.  A workgroup owns a patch of kLuP x kLuP columns along i and
+// marches through them.  In its first wavefront lane (vg, c) updates group vg
+// of the variables of column c = jl + kLuP kl, at step s the cell
+// i = s - jl - kl, whose upstream neighbours are the same column's last cell
+// and the cells that the columns jl - 1 and kl - 1 updated in the step before.
+// Group 0 is (rho, rho V, E), the others are a third of the species each.
+// Having updated its cell, a lane forms the terms that the downstream
+// neighbours along each direction d add (dG_d / 2 + a_d dQ, in the forward
+// sweep): the one along i stays in its registers, the others move by DPP row
+// shifts (the 16 columns of a group are a DPP row), and those of the patch's
+// last columns go to the patches after it through memory.  The second wavefront
+// moves the cells between memory and LDS, kLuG steps at a time.
+//
+// Patches hand over terms while they run.  The places of the terms hold kLuNone
+// until they are written, so a lane that needs one loads it (two steps ahead)
+// and loads it again until it is there; every value is one 64-bit atomic store
+// and load of agent scope and says by itself whether it is valid.  No wait can
+// last: a workgroup takes its patch from a ticket counter whose order holds
+// every patch behind the two that it waits for, so these are done or running.
+// (A wait beyond kLuWait, which none of this allows, is given up with an error
+// flag that ends every other wait as well.)
+//
+// The backward sweep is the forward one in mirrored indices, with the other
+// sign of dG.
+//
+// What bounds it is the chain of dependent steps, mx + my + mz of them at 0.7
+// us, and the hand-overs, 3 us each beyond the steps.  The form before it ran
+// tiles of 4 x 8 x 8 cells, one launch per tile hyperplane, with two barriers per
+// step and the neighbours' terms formed by the consumer: 96x80x64 cells with 9
+// species took 80 launches of 39 us per solve, now two of 0.39 ms.  Measured on
+// the way: one wavefront that also moves the cells 1.1 us per step; hand-over
+// records by cell instead of by step (scattered stores) 0.47 ms per sweep;
+// chunks of 4 steps, with three workgroups per CU, 0.42 (the workgroups of a CU
+// meet on one SIMD), with one 0.35, and 7% slower than 8 on larger blocks.
+constexpr int kLuCols = kLuP * kLuP, kLuG = 8;
+constexpr int kLuHeld = kLuCols * kLuG / 64;  // cells of a chunk per lane of the second wavefront
+static_assert(kLuCols == 16, "the columns of a variable group are one DPP row");
+constexpr unsigned long long kLuNone = 0x7FF4DEADBEEF5AA5ull;  // a signalling NaN: no result of arithmetic is one
+constexpr long long kLuWait = 1000000000ll;                    // of the 100 MHz clock: 10 s
+constexpr int kLuFlag = 2;                                     // in the context's error flags
+
+// v of the lane N before this one in its row of 16, or in the row's first N lanes
+// `first`
+template <int N>
+__device__ __forceinline__ double row_up(double first, double v) {
+  const int lo = __builtin_amdgcn_update_dpp(__double2loint(first), __double2loint(v), 0x110 | N, 0xf, 0xf, false);
+  const int hi = __builtin_amdgcn_update_dpp(__double2hiint(first), __double2hiint(v), 0x110 | N, 0xf, 0xf, false);
+  return __hiloint2double(hi, lo);
 }
-// staged values per cell: dQ (NV), state (NV), p, gamma, S_d (3 x 3), a_d (3), D
-constexpr int kLuVars = 2 * (5 + NS) + 15;
-// four wavefronts stage the tile and write it back; in the dependent steps
-// wavefronts 0-2 form one upstream direction's terms each
-constexpr int kLuThreads = 256;
+
+// the first row's v in every row (the odd rows swapped with the even ones of a
+// copy, then the halves of the wavefront)
+__device__ __forceinline__ double first_row(double v) {
+  auto word = [](unsigned x) {
+    const unsigned y = __builtin_amdgcn_permlane16_swap(x, x, false, false)[0];
+    return __builtin_amdgcn_permlane32_swap(y, y, false, false)[0];
+  };
+  return __hiloint2double((int)word((unsigned)__double2hiint(v)), (int)word((unsigned)__double2loint(v)));
+}
+
+// every place of a hand-over empty, the ticket counter back to 0
+__global__ void __launch_bounds__(kTpb) lusgs_reset_kernel(const BlockView *__restrict__ views,
+                                                           const int *__restrict__ off, int nb, int *ticket) {
+  const PointWork pw = point_work(off, nb);
+  const GView B = gview(views[pw.blk]);
+  const long long q = pw.base + threadIdx.x;
+  if (blockIdx.x == 0 && threadIdx.x == 0) *ticket = 0;
+  if (q >= B.ni) return;
+  const int m[3] = {B.mx, B.my, B.mz};
+  const long long n = lu_hand_over(m, NS);
+  gptr<unsigned long long> f = (gptr<unsigned long long>)B.luf;
+  for (long long x = q; x < n; x += B.ni) f[x] = kLuNone;
+}
 
 template <bool FWD>
-__global__ void __launch_bounds__(kLuThreads) lusgs_tile_kernel(const BlockView *__restrict__ views,
-                                                        const int *__restrict__ off, int nb, SchemeDev S,
-                                                        int tplane) {
-  constexpr int NV = 5 + NS, STEPS = kLuTi + kLuTj + kLuTk - 2;
-  constexpr int XQ = 0, XC = NV, XP = 2 * NV, XG = 2 * NV + 1, XS = 2 * NV + 2, XA = 2 * NV + 11, XD = 2 * NV + 14;
-  static_assert(kLuTj * kLuTk == 64, "one lane per (j, k) column of a tile");
-  static_assert((kLuVars * kLuSlots + 3 * NV * 64) * 8 <= 160 * 1024, "the staged tile fits in LDS");
-  __shared__ double ext[kLuVars][kLuSlots];
-  __shared__ double term[3][NV][64];  // the step's neighbour terms, by direction
-  const int w = blockIdx.x + off[0];
-  const int blk = find_seg(off, nb, w);
-  const GView B = gview(views[blk]);
-  const int m[3] = {B.mx, B.my, B.mz};
-  const int nt0 = (m[0] + kLuTi - 1) / kLuTi, nt1 = (m[1] + kLuTj - 1) / kLuTj, nt2 = (m[2] + kLuTk - 1) / kLuTk;
-  const int t = w - off[blk];
-  const int T1 = t % nt1, T2 = t / nt1, T0 = tplane - T1 - T2;
-  if (T2 >= nt2 || T0 < 0 || T0 >= nt0) return;  // uniform over the workgroup
-  const int lane = threadIdx.x;
-  const int org[3] = {T0 * kLuTi - (FWD ? 1 : 0), T1 * kLuTj - (FWD ? 1 : 0), T2 * kLuTk - (FWD ? 1 : 0)};
-  const long long np = B.np, ni = B.ni;
-  // ---- stage the tile and its upstream faces
-  for (int n = lane; n < kLuExt; n += kLuThreads) {
-    const int li = n % kLuEi, lj = (n / kLuEi) % kLuEj, lk = n / (kLuEi * kLuEj);
-    const int e = lu_slot(li, lj, lk);
-    const int c[3] = {org[0] + li, org[1] + lj, org[2] + lk};
-    if (c[0] < 0 || c[0] >= m[0] || c[1] < 0 || c[1] >= m[1] || c[2] < 0 || c[2] >= m[2]) continue;
-    const long long q = ((long long)c[2] * m[1] + c[1]) * m[0] + c[0];
-    const long long p = pidx(B, c[0], c[1], c[2]);
-#pragma unroll
-    for (int l = 0; l < NV; ++l) {
-      ext[XQ + l][e] = B.dq[l * ni + q];
-      ext[XC + l][e] = B.cv[l * np + p];
-    }
-    ext[XP][e] = B.bv[4 * np + p];
-    ext[XG][e] = B.props[p];
-    const double J = B.jac[p];
-#pragma unroll
-    for (int v = 0; v < 9; ++v) ext[XS + v][e] = J * B.metric[v * np + p];
-#pragma unroll
-    for (int d = 0; d < 3; ++d) ext[XA + d][e] = B.lus[(1 + d) * ni + q];
-    ext[XD][e] = B.lus[q];
-  }
+__global__ void __launch_bounds__(128, 1) lusgs_sweep_kernel(const BlockView *__restrict__ views,
+                                                            const LuPatch *__restrict__ order, int n_patch,
+                                                            int *ticket, SchemeDev S, int *flags) {
+  // variables of a lane (group 0 has 5); places of a cell's variables, group by group
+  constexpr int NV = 5 + NS, N3 = lu_third(NS), NSL = N3 > 5 ? N3 : 5, NP = lu_places(NS);
+  static_assert(N3 <= 5, "the groups after the first hold at most its 5 variables");
+  // a staged cell: dQ (R or dQ* until it is updated), state (the energy's place
+  // holds E + p), S_d = J grad xi_d (3 x 3), a_d, U_d / 2 (its sign as in the
+  // sweep's terms), 1/D, gamma - 1, kinetic energy
+  constexpr int XC = NP, XS = 2 * NP, XA = XS + 9, XU = XA + 3, XI = XU + 3, XG = XI + 1, XK = XG + 1, RS = (XK + 1) | 1;
+  constexpr double SG = FWD ? 0.5 : -0.5;
+  constexpr int CHUNK = kLuG * kLuCols * RS;
+  __shared__ double rec[2 * CHUNK];
+  __shared__ int mine;
+  const int lane = threadIdx.x & 63;
+  const bool mover = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) == 1;
+  if (threadIdx.x == 0) mine = atomicAdd(ticket, 1);
   __syncthreads();
-  // ---- the dependent steps, in LDS: wavefront d (0..2) forms the term of
-  // the upstream neighbour along d for every column of the step, wavefront 0
-  // then adds them in the order d = 0, 1, 2 and updates the cells
-  const int wv = lane >> 6, cl = lane & 63;
-  const int jl = cl % kLuTj, kl = cl / kLuTj;
-  const int j = T1 * kLuTj + jl, k = T2 * kLuTk + kl;
-  const bool col = j < m[1] && k < m[2];
-  const int o = FWD ? 1 : 0;  // position of the tile's first cell in the staged box
-  const int es[3] = {1, kLuEi, kLuSk};
-  for (int step = 0; step < STEPS; ++step) {
-    const int il = (FWD ? step : STEPS - 1 - step) - jl - kl;
-    const int i = T0 * kLuTi + il;
-    const bool act = col && il >= 0 && il < kLuTi && i < m[0];
-    const int ijk[3] = {i, j, k};
-    const int e = lu_slot(il + o, jl + o, kl + o);
-    if (act && wv < S.dim && (FWD ? ijk[wv] > 0 : ijk[wv] < m[wv] - 1)) {
-      const int d = wv;
-      const int en = FWD ? e - es[d] : e + es[d];
-      // dG_d = G_d(Q + dQ) - G_d(Q) of the neighbour, pressure change at its
-      // frozen gamma
-      double dn[NV], q0[NV], q1[NV], dG[NV];
+  const int tk = __builtin_amdgcn_readfirstlane(mine);
+  if (tk >= n_patch) return;  // uniform over the workgroup
+  const LuPatch pt = order[tk];
+  const GView B = gview(views[pt.blk]);
+  const int mx = B.mx, my = B.my, mz = B.mz;
+  const long long np = B.np, ni = B.ni;
+  const bool dim3_ = S.dim == 3;
+
+  const int c = lane & 15, vg = lane >> 4, jl = c % kLuP, kl = c / kLuP;
+  const int jj = pt.J * kLuP + jl, kk = pt.K * kLuP + kl;
+  const bool col = jj < my && kk < mz;
+  const int h0 = vg == 0 ? 0 : 5 + (vg - 1) * N3;  // this lane's places
+  // hand-over to the next patch along j (then along k): [patch][step][variable of
+  // a group][group][kl], so that a step's values are a few whole lines
+  const int nJ = (my + kLuP - 1) / kLuP, nK = (mz + kLuP - 1) / kLuP, wj = min(kLuP, my), wk = min(kLuP, mz);
+  const int steps = mx + wj + wk - 2, n_chunk = (steps + kLuG - 1) / kLuG;
+  constexpr int ST = kLuP * NP;
+  const long long fs = (long long)steps * ST;
+  const long long at = (long long)pt.K * nJ + pt.J;
+  typedef unsigned long long u64;
+  const gptr<u64> F = (gptr<u64>)B.luf;
+  const gptr<u64> FK = F + (nJ > 1 ? (long long)nJ * nK * fs : 0);
+  const bool need_j = col && jl == 0 && jj > 0, need_k = col && kl == 0 && kk > 0;
+  const bool give_j = col && jl == kLuP - 1 && jj + 1 < my, give_k = col && kl == kLuP - 1 && kk + 1 < mz;
+  // a cell that the patch before updates in its step s + kLuP - 1 is the upstream
+  // neighbour of one of step s here
+  gptr<u64> in_j = F + (at - 1) * fs + (kLuP - 1) * ST + kLuP * vg + kl;
+  gptr<u64> in_k = FK + (at - nJ) * fs + (kLuP - 1) * ST + kLuP * vg + jl;
+  gptr<u64> out_j = F + at * fs + kLuP * vg + kl, out_k = FK + at * fs + kLuP * vg + jl;
+  // this lane's value q in a step's record (from N3 on group 0's alone)
+  auto place = [](int q) { return q < N3 ? 4 * kLuP * q : (3 * N3 + q) * kLuP; };
+
+  if (mover) {
+    // ---- the second wavefront moves the cells: lane e + kLuG (column % 8) holds
+    // cell e of a chunk, of one column in each half.  While chunk n is worked on
+    // it takes chunk n - 1 out of LDS, puts chunk n + 1 there and loads chunk n + 2.
+    const int e = lane % kLuG;
+    long long row[kLuHeld], prow[kLuHeld];
+    int i00[kLuHeld];
+    bool real[kLuHeld];
+    double *own[kLuHeld];
 #pragma unroll
-      for (int l = 0; l < NV; ++l) {
-        dn[l] = ext[XQ + l][en];
-        q0[l] = ext[XC + l][en];
-        q1[l] = q0[l] + dn[l];
+    for (int h = 0; h < kLuHeld; ++h) {
+      const int cr = lane / kLuG + 64 / kLuG * h, j0 = pt.J * kLuP + cr % kLuP, k0 = pt.K * kLuP + cr / kLuP;
+      const int jc = min(j0, my - 1), kc = min(k0, mz - 1), j = FWD ? jc : my - 1 - jc, k = FWD ? kc : mz - 1 - kc;
+      row[h] = ((long long)k * my + j) * mx;
+      prow[h] = pidx(B, 0, j, k);
+      i00[h] = e - cr % kLuP - cr / kLuP;
+      real[h] = j0 == jc && k0 == kc;
+      own[h] = rec + (e * kLuCols + cr) * RS;
+    }
+    auto cell = [&](int n, int h, int &i) {  // of chunk n, whether it is on the block
+      const int im = n * kLuG + i00[h], ic = min(max(im, 0), mx - 1);
+      i = FWD ? ic : mx - 1 - ic;
+      return im == ic && real[h];
+    };
+    double xx[kLuHeld][2 * NV], mm[kLuHeld][16];
+    auto load = [&](int n) {
+#pragma unroll
+      for (int h = 0; h < kLuHeld; ++h) {
+        int i;
+        cell(n, h, i);
+        const long long q = row[h] + i, p = prow[h] + i;
+        double *x = xx[h], *m = mm[h];
+#pragma unroll
+        for (int l = 0; l < NV; ++l) x[l] = B.dq[l * ni + q], x[NV + l] = B.cv[l * np + p];
+#pragma unroll
+        for (int v = 0; v < 9; ++v) m[v] = B.metric[v * np + p];
+#pragma unroll
+        for (int v = 0; v < 4; ++v) m[9 + v] = B.lus[v * ni + q];
+        m[13] = B.jac[p];
+        m[14] = B.bv[4 * np + p];
+        m[15] = B.props[p];
       }
-      const double Sx = ext[XS + 3 * d][en], Sy = ext[XS + 3 * d + 1][en], Sz = ext[XS + 3 * d + 2][en];
-      const double gam = ext[XG][en], p0 = ext[XP][en];
-      const double r0 = frcp<double>(q0[0]), r1 = frcp<double>(q1[0]);
-      const double ke0 = lu_div(0.5 * (q0[1] * q0[1] + q0[2] * q0[2] + q0[3] * q0[3]), q0[0], r0);
-      const double ke1 = lu_div(0.5 * (q1[1] * q1[1] + q1[2] * q1[2] + q1[3] * q1[3]), q1[0], r1);
-      const double p1 = p0 + (gam - 1) * (dn[4] - (ke1 - ke0));
-      const double U0 = lu_div(Sx * q0[1] + Sy * q0[2] + Sz * q0[3], q0[0], r0);
-      const double U1 = lu_div(Sx * q1[1] + Sy * q1[2] + Sz * q1[3], q1[0], r1);
-      dG[0] = q1[0] * U1 - q0[0] * U0;
-      dG[1] = (q1[1] * U1 + Sx * p1) - (q0[1] * U0 + Sx * p0);
-      dG[2] = (q1[2] * U1 + Sy * p1) - (q0[2] * U0 + Sy * p0);
-      dG[3] = (q1[3] * U1 + Sz * p1) - (q0[3] * U0 + Sz * p0);
-      dG[4] = (q1[4] + p1) * U1 - (q0[4] + p0) * U0;
+    };
+    auto stage = [&](int n) {
 #pragma unroll
-      for (int l = 5; l < NV; ++l) dG[l] = q1[l] * U1 - q0[l] * U0;
-      const double an = ext[XA + d][en];
+      for (int h = 0; h < kLuHeld; ++h) {
+        int i;
+        const bool in = cell(n, h, i);
+        double *r = own[h] + (n & 1) * CHUNK;
+        const double *x = xx[h], *m = mm[h], *q0 = x + NV;
+        const double J = in ? m[13] : 0.0;  // cells off the block: no terms
+        const double r0 = frcp<double>(q0[0]);
 #pragma unroll
-      for (int l = 0; l < NV; ++l) term[d][l][cl] = FWD ? 0.5 * dG[l] + an * dn[l] : an * dn[l] - 0.5 * dG[l];
+        for (int l = 0; l < NP; ++l) {
+          r[l] = l < NV && in ? x[l < NV ? l : 0] : 0.0;
+          r[XC + l] = l == 4 ? q0[4] + m[14] : (l < NV ? q0[l < NV ? l : 0] : 0.0);
+        }
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+          const double Sx = J * m[3 * d], Sy = J * m[3 * d + 1], Sz = J * m[3 * d + 2];
+          r[XS + 3 * d] = Sx, r[XS + 3 * d + 1] = Sy, r[XS + 3 * d + 2] = Sz;
+          r[XU + d] = SG * ((Sx * q0[1] + Sy * q0[2] + Sz * q0[3]) * r0);
+          r[XA + d] = in ? m[10 + d] : 0.0;
+        }
+        r[XI] = frcp<double>(m[9]);
+        r[XG] = m[15] - 1;
+        r[XK] = (0.5 * (q0[1] * q0[1] + q0[2] * q0[2] + q0[3] * q0[3])) * r0;
+      }
+    };
+    auto take = [&](int n) {
+#pragma unroll
+      for (int h = 0; h < kLuHeld; ++h) {
+        int i;
+        if (!cell(n, h, i)) continue;
+        const double *r = own[h] + (n & 1) * CHUNK;
+#pragma unroll
+        for (int l = 0; l < NV; ++l) B.dq[l * ni + row[h] + i] = r[l];
+      }
+    };
+    load(0);
+    stage(0);
+    if (n_chunk > 1) load(1);
+    for (int n = 0; n < n_chunk; ++n) {
+      __syncthreads();
+      if (n > 0) take(n - 1);
+      if (n + 1 < n_chunk) stage(n + 1);
+      if (n + 2 < n_chunk) load(n + 2);
     }
     __syncthreads();
-    if (act && wv == 0) {
-      double acc[NV];
+    take(n_chunk - 1);
+    return;
+  }
+
+  struct Cell {
+    double R[NSL], q0[NSL], S[9], a[3], U[3], rD, gm, ke;
+  };
+  auto read = [&](const double *chunk, int t, Cell &x) {
+    const double *r = chunk + (t * kLuCols + c) * RS;
 #pragma unroll
-      for (int l = 0; l < NV; ++l) acc[l] = FWD ? ext[XQ + l][e] : 0.0;
-#pragma unroll
-      for (int d = 0; d < 3; ++d) {
-        if (!(d < S.dim && (FWD ? ijk[d] > 0 : ijk[d] < m[d] - 1))) continue;
-#pragma unroll
-        for (int l = 0; l < NV; ++l) acc[l] += term[d][l][cl];
-      }
-      const double D = ext[XD][e], rD = frcp<double>(D);
-#pragma unroll
-      for (int l = 0; l < NV; ++l)
-        ext[XQ + l][e] = FWD ? lu_div(acc[l], D, rD) : ext[XQ + l][e] + lu_div(acc[l], D, rD);
+    for (int q = 0; q < NSL; ++q) {
+      const int v = q < N3 ? h0 + q : q;
+      x.R[q] = r[v], x.q0[q] = r[XC + v];
     }
-    __syncthreads();
-  }
-  // ---- the tile's increments back to dq
-  for (int c = lane; c < kLuTi * kLuTj * kLuTk; c += kLuThreads) {
-    const int il = c % kLuTi, jc = (c / kLuTi) % kLuTj, kc = c / (kLuTi * kLuTj);
-    const int i = T0 * kLuTi + il, jg = T1 * kLuTj + jc, kg = T2 * kLuTk + kc;
-    if (i >= m[0] || jg >= m[1] || kg >= m[2]) continue;
-    const int e = lu_slot(il + o, jc + o, kc + o);
-    const long long q = ((long long)kg * m[1] + jg) * m[0] + i;
 #pragma unroll
-    for (int l = 0; l < NV; ++l) B.dq[l * ni + q] = ext[XQ + l][e];
+    for (int v = 0; v < 9; ++v) x.S[v] = r[XS + v];
+#pragma unroll
+    for (int v = 0; v < 3; ++v) x.a[v] = r[XA + v], x.U[v] = r[XU + v];
+    x.rD = r[XI], x.gm = r[XG], x.ke = r[XK];
+  };
+
+  // ---- terms from the patches before this one and to those after it; a place
+  // past a lane's N3 is one of group 0
+  // and a lane that needs no term keeps the zeros
+  u64 ij[2][NSL] = {}, ik[2][NSL] = {};
+  auto fetch = [&](bool now, gptr<u64> from, u64 *in) {
+    if (now) {
+#pragma unroll
+      for (int q = 0; q < N3; ++q)
+        in[q] = __hip_atomic_load((u64 *)(from + place(q)), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (vg == 0) {
+#pragma unroll
+        for (int q = N3; q < NSL; ++q)
+          in[q] = __hip_atomic_load((u64 *)(from + place(q)), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+    }
+  };
+  auto give = [&](bool on, gptr<u64> to, const double *T) {
+    if (on) {
+#pragma unroll
+      for (int q = 0; q < N3; ++q)
+        __hip_atomic_store((u64 *)(to + place(q)), (u64)__double_as_longlong(T[q]), __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
+      if (vg == 0) {
+#pragma unroll
+        for (int q = N3; q < NSL; ++q)
+          __hip_atomic_store((u64 *)(to + place(q)), (u64)__double_as_longlong(T[q]), __ATOMIC_RELAXED,
+                             __HIP_MEMORY_SCOPE_AGENT);
+      }
+    }
+  };
+  auto missing = [&](const u64 *x, const u64 *y) {  // by the high words
+    unsigned m = ~0u;
+#pragma unroll
+    for (int q = 0; q < NSL; ++q)
+      m = min(min(m, (unsigned)(x[q] >> 32) ^ (unsigned)(kLuNone >> 32)), (unsigned)(y[q] >> 32) ^ (unsigned)(kLuNone >> 32));
+    return m == 0;
+  };
+
+  double T0[NSL], T1[NSL], T2[NSL];
+#pragma unroll
+  for (int q = 0; q < NSL; ++q) T0[q] = T1[q] = T2[q] = 0.0;
+  auto now = [&](bool need, int s) { return need && s >= jl + kl && s < mx + jl + kl; };
+#pragma unroll
+  for (int s = 0; s < 2; ++s) {
+    fetch(now(need_j, s), in_j + s * ST, ij[s]);
+    fetch(now(need_k, s), in_k + s * ST, ik[s]);
   }
+  for (int n = 0; n < n_chunk; ++n) {
+    __syncthreads();
+    double *const chunk = rec + (n & 1) * CHUNK;
+    Cell cell[2];
+    read(chunk, 0, cell[0]);
+#pragma unroll 2
+    for (int t = 0; t < kLuG; ++t) {
+      const int s = n * kLuG + t;
+      const bool act = col && s >= jl + kl && s < mx + jl + kl;
+      const Cell &x = cell[t & 1];
+      read(chunk, min(t + 1, kLuG - 1), cell[(t + 1) & 1]);
+      u64 *aj = ij[t & 1], *ak = ik[t & 1];
+      if (__any(missing(aj, ak))) {
+        // (a patch that waits for its first terms leaves the memory to the others)
+        const long long until = (long long)wall_clock64() + kLuWait;
+        for (int spin = 1; __any(missing(aj, ak)); ++spin) {
+          if (s < kLuP) __builtin_amdgcn_s_sleep(16);
+          if (missing(aj, ak)) {
+            fetch(now(need_j, s), in_j, aj);
+            fetch(now(need_k, s), in_k, ak);
+          }
+          if (spin % 256) continue;
+          if ((long long)wall_clock64() > until) atomicOr(flags, kLuFlag);
+          if (__hip_atomic_load(flags, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & kLuFlag) break;
+        }
+      }
+      double dn[NSL];
+#pragma unroll
+      for (int q = 0; q < NSL; ++q) {
+        const double uj = row_up<1>(0.0, T1[q]), uk = row_up<kLuP>(__longlong_as_double((long long)ak[q]), T2[q]);
+        const double acc = (FWD ? x.R[q] + T0[q] : T0[q]) + (jl == 0 ? __longlong_as_double((long long)aj[q]) : uj) + uk;
+        dn[q] = FWD ? acc * x.rD : x.R[q] + acc * x.rD;
+      }
+      in_j += ST, in_k += ST;
+      fetch(now(need_j, s + 2), in_j + ST, aj);
+      fetch(now(need_k, s + 2), in_k + ST, ak);
+      double *r = chunk + (t * kLuCols + c) * RS + h0;
+#pragma unroll
+      for (int q = 0; q < N3; ++q) r[q] = dn[q];
+      if (vg == 0) {
+#pragma unroll
+        for (int q = N3; q < NSL; ++q) r[q] = dn[q];
+      }
+      // velocities and pressure change of the new state: group 0's, for all groups
+      const double m0 = x.q0[0] + dn[0], m1 = x.q0[1] + dn[1], m2 = x.q0[2] + dn[2], m3 = x.q0[3] + dn[3];
+      const double r1 = frcp<double>(m0);
+      double U1[3];
+#pragma unroll
+      for (int d = 0; d < 3; ++d)
+        U1[d] = first_row((x.S[3 * d] * m1 + x.S[3 * d + 1] * m2 + x.S[3 * d + 2] * m3) * r1);
+      const double dp = x.gm * (dn[4] - ((0.5 * (m1 * m1 + m2 * m2 + m3 * m3)) * r1 - x.ke));
+      const double hp = vg == 0 ? SG * dp : 0.0;
+      // +-dG_d / 2 + a_d dQ with dG = dQ U1 + Q (U1 - U) (+ p terms)
+      auto terms = [&](int d, double *T) {
+        const double h1 = x.a[d] + SG * U1[d], h2 = SG * U1[d] - x.U[d];
+#pragma unroll
+        for (int q = 0; q < NSL; ++q) {
+          T[q] = dn[q] * h1 + x.q0[q] * h2;
+          if (q >= 1 && q <= 3) T[q] += x.S[3 * d + q - 1] * hp;
+          if (q == 4) T[q] += U1[d] * hp;
+        }
+      };
+      terms(1, T1);
+      give(act && give_j, out_j, T1);
+      if (dim3_) {
+        terms(2, T2);
+        give(act && give_k, out_k, T2);
+      }
+      terms(0, T0);
+      out_j += ST, out_k += ST;
+    }
+  }
+  __syncthreads();  // the last chunk is done
 }
 
 int launch_lusgs_coef(const Batch &b, const SchemeDev &S, hipStream_t st) {
@@ -950,12 +1152,19 @@ int launch_lusgs_coef(const Batch &b, const SchemeDev &S, hipStream_t st) {
   return (int)hipGetLastError();
 }
 
-int launch_lusgs_sweep(const Batch &b, const SchemeDev &S, int tplane, int fwd, hipStream_t st) {
+int launch_lusgs_reset(const Batch &b, int *ticket, hipStream_t st) {
   if (b.total <= 0) return 0;
+  lusgs_reset_kernel<<<b.total, kTpb, 0, st>>>(b.views, b.off, b.nb, ticket);
+  return (int)hipGetLastError();
+}
+
+int launch_lusgs_sweep(const BlockView *views, const LuPatch *order, int n, int *ticket, const SchemeDev &S, int fwd,
+                       int *flags, hipStream_t st) {
+  if (n <= 0) return 0;
   if (fwd)
-    lusgs_tile_kernel<true><<<b.total, kLuThreads, 0, st>>>(b.views, b.off, b.nb, S, tplane);
+    lusgs_sweep_kernel<true><<<n, 128, 0, st>>>(views, order, n, ticket, S, flags);
   else
-    lusgs_tile_kernel<false><<<b.total, kLuThreads, 0, st>>>(b.views, b.off, b.nb, S, tplane);
+    lusgs_sweep_kernel<false><<<n, 128, 0, st>>>(views, order, n, ticket, S, flags);
   return (int)hipGetLastError();
 }
 
@@ -1061,6 +1270,7 @@ struct Register64 {
     k.update = launch_update;
     k.face_ops = launch_face_ops;
     k.lusgs_coef = launch_lusgs_coef;
+    k.lusgs_reset = launch_lusgs_reset;
     k.lusgs_sweep = launch_lusgs_sweep;
     register_rhs<double>(k);
     k.present = 1;
