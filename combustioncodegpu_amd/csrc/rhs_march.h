@@ -294,8 +294,8 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(WPE, WP
       const int i3 = isz ? s2 + el : iR + da;
       const int i0 = isz ? P::COL + tid : iL - da;
       // the face-point data of the viscous flux; issued ahead of AUSM+ where
-      // the registers hold it (FP64: 256 of them; at the 128 of FP32 it spills)
-      constexpr bool EARLY = sizeof(R) == 8;
+      // the registers hold it (256 of them at 2 waves per SIMD; at 128 it spills)
+      constexpr bool EARLY = WPE <= 2;
       R rB[3][2], rC[3][2], rV[4];
       auto face_point = [&] {
 #pragma unroll
