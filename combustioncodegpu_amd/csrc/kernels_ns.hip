@@ -61,13 +61,31 @@ __device__ __forceinline__ PointWork point_work(const int *__restrict__ off, int
 // update_physical_properties (Field.cu:178-210): mixture cp, gamma and speed
 // of sound at temperature t and mass fractions Y; cp_l and sum Y_l/W_l are
 // returned for the transport.
+// FP64: cpl holds a copy of the cp coefficients in LDS (kCpRec per species, the
+// low ranges first), from which each lane reads those of its own range (the
+// same values).  species_cp reads them from memory behind a branch instead, one
+// species after the other: 256x128x128 cells with 9 species 0.30 -> 0.23 ms,
+// with the roots of all species at once (floor of its traffic: 0.17).
+constexpr int kCpRec = 6;  // 5 coefficients, 16-byte aligned
 template <typename R>
-__device__ __forceinline__ void mixture_gamma_c(SpeciesPtrT<R> sp, R t, const R *Y, R *cp, R &winv, R *out) {
+__device__ __forceinline__ void mixture_gamma_c(SpeciesPtrT<R> sp, const R *cpl, R t, const R *Y, R *cp, R &winv,
+                                                R *out) {
   R cpt = 0;
   winv = 0;
+  const bool hi = t >= R(sp->hi_from);
+  if (cpl && __all(hi || (t >= R(sp->lo_from) && t < R(sp->lo_to)))) {
+    const R *c = cpl + (hi ? NS * kCpRec : 0);
+#pragma unroll
+    for (int l = 0; l < NS; ++l) {
+      const R *x = c + l * kCpRec;
+      cp[l] = x[0] + t * (x[1] + t * (x[2] + t * (x[3] + t * x[4])));
+    }
+  } else {
+#pragma unroll
+    for (int l = 0; l < NS; ++l) cp[l] = species_cp<R>(sp, l, t);
+  }
 #pragma unroll
   for (int l = 0; l < NS; ++l) {
-    cp[l] = species_cp<R>(sp, l, t);
     winv += Y[l] * R(sp->inv_mw[l]);
     cpt += Y[l] * cp[l];
   }
@@ -82,7 +100,9 @@ __device__ __forceinline__ void mixture_gamma_c(SpeciesPtrT<R> sp, R t, const R 
 // = s_m/s_n (NS square roots instead of NS^2), and T*^-0.145 =
 // T^-0.145 (k/eps_l)^-0.145: one exponential per point, the species factor
 // from the table.
-template <typename R>
+// ROOTS: the roots and their reciprocals of all species at once (within an ulp
+// of the others).
+template <typename R, bool ROOTS = false>
 __device__ __forceinline__ void wilke_point(SpeciesPtrT<R> sp, const SchemeDev &S, R t, const R *Y, const R *cp,
                                             R winv, R *out) {
   // Chapman-Enskog species viscosity (Transport.cu:52-57)
@@ -96,9 +116,12 @@ __device__ __forceinline__ void wilke_point(SpeciesPtrT<R> sp, const SchemeDev &
     const R a = tdl + R(0.5);
     const R omega = R(1.147) * (tm * R(sp->om145[l])) + frcp<R>(a * a);
     mu_s[l] = fdiv<R>(R(sp->vis_coeff[l]) * st, omega);
-    s[l] = fsqrt<R>(mu_s[l]);
-    rs[l] = frcp<R>(s[l]);
+    if constexpr (!ROOTS) {
+      s[l] = fsqrt<R>(mu_s[l]);
+      rs[l] = frcp<R>(s[l]);
+    }
   }
+  if constexpr (ROOTS) fsqrt_n<NSA, R>(mu_s, s, rs);
   // Wilke mixing and Mason-Saxena conductivity (Transport.cu:58-83)
   R mu = 0, kappa = 0;
 #pragma unroll
@@ -134,6 +157,11 @@ __global__ void __launch_bounds__(kTpb) props_kernel(const BlockView *__restrict
   const GView B = gview(views[pw.blk]);
   const long long np = B.np;
   constexpr bool f32 = sizeof(R) == 4;
+  __shared__ __attribute__((aligned(16))) R cpl[f32 || NS == 0 ? 1 : 2 * NSA * kCpRec];
+  if constexpr (!f32 && NS > 0) {
+    for (int n = threadIdx.x; n < 10 * NS; n += kTpb) cpl[n / 5 * kCpRec + n % 5] = sp->cpc[n / (5 * NSA)][n / 5 % NSA][n % 5];
+    __syncthreads();
+  }
   const long long q = pw.base + threadIdx.x;
   if (q >= (PLANE ? B.sz : np)) return;
   const long long p = PLANE ? kNgg * B.sz + q : q;
@@ -157,8 +185,8 @@ __global__ void __launch_bounds__(kTpb) props_kernel(const BlockView *__restrict
 #pragma unroll
       for (int l = 0; l < NS; ++l) Y[l] = R(B.yk[l * np + p]);
     }
-    mixture_gamma_c<R>(sp, t, Y, cp, winv, out);
-    wilke_point<R>(sp, S, t, Y, cp, winv, out + 2);
+    mixture_gamma_c<R>(sp, f32 ? nullptr : cpl, t, Y, cp, winv, out);
+    wilke_point<R, !f32>(sp, S, t, Y, cp, winv, out + 2);
   }
   if constexpr (f32) {
     // loads first (T and Y are already held), then the stores
@@ -1242,7 +1270,7 @@ __global__ void __launch_bounds__(256) mlp_samples_kernel(const SpeciesDev *__re
 #pragma unroll
   for (int l = 0; l < NS; ++l) Y[l] = sum > 0.0 ? Y[l] * inv : 1.0 / NS;
   double cp[NSA], winv, gc[2], out[2 + NSA];
-  mixture_gamma_c<double>(sp, t, Y, cp, winv, gc);
+  mixture_gamma_c<double>(sp, nullptr, t, Y, cp, winv, gc);
   wilke_point<double>(sp, S, t, Y, cp, winv, out);
   double *xr = x + s * (NS + 2), *yr = y + s * (NS + 2);
   xr[0] = t;
@@ -1315,7 +1343,7 @@ __device__ __forceinline__ bool mlp_phase1(const GView &B, SpeciesPtrT<float> sp
   const int lane = threadIdx.x & 63;
   const long long np = B.np;
   float cp[NSA], winv, gc[2], x[kMlpIO];
-  mixture_gamma_c<float>(sp, b32[5], Y, cp, winv, gc);
+  mixture_gamma_c<float>(sp, nullptr, b32[5], Y, cp, winv, gc);
   float ymax = 0.0f;  // largest Y_l / W_l: the largest mole fraction times winv
 #pragma unroll
   for (int l = 0; l < NS; ++l) ymax = fmaxf(ymax, Y[l] * sp->inv_mw[l]);
@@ -1375,7 +1403,7 @@ __device__ __forceinline__ void mlp_phase23(const GView &B, SpeciesPtrT<float> s
     const double ir = 1.0 / ldg<double>(cvb, o8);
 #pragma unroll
     for (int l = 0; l < NS; ++l) Y[l] = float(ldg<double>(cvb + (5 + l) * npl, o8) * ir);
-    mixture_gamma_c<float>(sp, t, Y, cp, winv, gc);
+    mixture_gamma_c<float>(sp, nullptr, t, Y, cp, winv, gc);
     wilke_point<float>(sp, S, t, Y, cp, winv, w);
     if (check) {
 #pragma unroll
