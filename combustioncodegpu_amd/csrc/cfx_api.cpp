@@ -643,7 +643,7 @@ bool split_ops(const std::vector<FaceOp> &ops, int first, int dim, std::vector<F
 
 // The strips as components of linked points; false if one holds too many.
 bool build_strips(const cfx_ctx *ctx, const std::vector<std::vector<FaceOp>> &rest, std::vector<ExSlot> &slots,
-                  std::vector<ExOp> &ops, std::vector<int> &slot_off, std::vector<int> &op_off) {
+                  std::vector<ExOp> &ops, std::vector<int> &slot_off, std::vector<int> &op_off, int end[3]) {
   struct PointOp {
     int a, b;  // point ids: written (and averaged) / read
     bool average;
@@ -711,8 +711,18 @@ bool build_strips(const cfx_ctx *ctx, const std::vector<std::vector<FaceOp>> &re
     local[x] = count[comp[x]]++;
     if (local[x] >= kMaxSlots) return false;
   }
+  // ... then by their slots, as many as fit each form of the kernel
   const int nc = (int)count.size();
-  for (int c = 0; c < nc; ++c) slot_off.push_back(slot_off[c] + count[c]);
+  std::vector<int> rank(nc);
+  for (int q = 0, r = 0; q < 3; ++q) {
+    for (int c = 0; c < nc; ++c) {
+      if (count[c] > kStripSlots[q] || (q > 0 && count[c] <= kStripSlots[q - 1])) continue;
+      rank[c] = r++;
+      slot_off.push_back(slot_off.back() + count[c]);
+    }
+    end[q] = r;
+  }
+  for (int x = 0; x < np; ++x) comp[x] = rank[comp[x]];
   slots.resize(np);
   for (int x = 0; x < np; ++x) slots[slot_off[comp[x]] + local[x]] = pts[x];
   op_off.assign(nc + 1, 0);
@@ -748,14 +758,13 @@ int split_exchange(cfx_ctx *ctx) {
   std::vector<ExOp> ops;
   std::vector<int> slot_off, op_off;
   if (!split_ops(ctx->ops, ctx->n_bc_ops, ctx->dim, mid, rest)) return 0;
-  if (!build_strips(ctx, rest, slots, ops, slot_off, op_off)) return 0;
+  if (!build_strips(ctx, rest, slots, ops, slot_off, op_off, ctx->strips.end)) return 0;
   int rc;
   std::vector<int> one(mid.size(), 0);
   if ((rc = build_schedule(ctx, mid, ctx->sched_mid, 0, (int)mid.size(), false, &one)) ||
       (rc = upload(ctx, slots, ctx->strips.slots)) || (rc = upload(ctx, ops, ctx->strips.ops)) ||
       (rc = upload(ctx, slot_off, ctx->strips.slot_off)) || (rc = upload(ctx, op_off, ctx->strips.op_off)))
     return rc;
-  ctx->strips.n = (int)slot_off.size() - 1;
   ctx->ex_split = true;
   return 0;
 }

@@ -249,8 +249,9 @@ struct ExStrips {
   const ExSlot *slots;
   const ExOp *ops;
   const int *slot_off, *op_off;
-  int n;  // components
+  int end[3];  // components of at most kStripSlots[q] slots end at end[q]
 };
+constexpr int kStripSlots[3] = {4, 8, kMaxSlots};
 
 // Work segments: workgroup w (counted from off[0]) belongs to segment s with
 // off[s] <= w < off[s+1], s in [0, n).  The search is uniform per workgroup.
