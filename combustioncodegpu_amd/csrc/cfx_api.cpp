@@ -208,11 +208,21 @@ int build_tables(cfx_ctx *ctx) {
     const HostBlock &H = ctx->hb[b];
     pad[b] = chunks(H.np, kTpb);
     in1[b] = chunks(H.ni, kTpb);
-    dtc[b] = chunks(H.ni, kTpb * kDtIter);
-    last[b] = chunks(H.ni, kTpb * kLastIter);
     res[b] = chunks(H.ni, kTpb * kResIter);
   }
   int rc;
+  // small contexts spread the points over the chip instead (128x64 points: time
+  // step 10.5 -> 4.4 us, snapshot 7.1 -> 4.6); the time step ends in an atomic
+  // per workgroup, and takes few of them (1021x509 points: 2031 workgroups 29 us,
+  // 508 16 us)
+  long long all = 0;
+  for (const HostBlock &H : ctx->hb) all += H.ni;
+  ctx->dt_iter = (int)std::min<long long>(kDtIter, 1 + all / (kTpb * 512));
+  ctx->last_iter = (int)std::min<long long>(kLastIter, 1 + all / (kTpb * 2048));
+  for (int b = 0; b < nb; ++b) {
+    dtc[b] = chunks(ctx->hb[b].ni, kTpb * ctx->dt_iter);
+    last[b] = chunks(ctx->hb[b].ni, kTpb * ctx->last_iter);
+  }
   if ((rc = upload_table(ctx, ctx->t_pad, pad)) || (rc = upload_table(ctx, ctx->t_int, in1)) ||
       (rc = upload_table(ctx, ctx->t_dt, dtc)) || (rc = upload_table(ctx, ctx->t_last, last)) ||
       (rc = upload_table(ctx, ctx->t_res, res)))
@@ -891,12 +901,13 @@ int per_batch(cfx_ctx *ctx, const Table &t, F &&f) {
   return 0;
 }
 
-int do_dt(cfx_ctx *ctx, int global, int store_local) {
+// reset: whether the reduction's target needs it (not after do_store_last with reset)
+int do_dt(cfx_ctx *ctx, int global, int store_local, bool reset = true) {
   auto *bits = reinterpret_cast<unsigned long long *>(ctx->d_dt);
-  if (global) CFX_TRY(ctx->timed_launch(K_DT, [&] { return launch_dt_reset(bits, ctx->stream); }));
+  if (global && reset) CFX_TRY(ctx->timed_launch(K_DT, [&] { return launch_dt_reset(bits, ctx->stream); }));
   CFX_TRY(per_batch(ctx, ctx->t_dt, [&](const Batch &b) {
     return ctx->timed_launch(K_DT, [&] {
-      return launch_dt(b, ctx->S, ctx->ns, store_local, global ? bits : ctx->d_minscratch, ctx->stream);
+      return launch_dt(b, ctx->S, ctx->ns, ctx->dt_iter, store_local, global ? bits : ctx->d_minscratch, ctx->stream);
     });
   }));
   return 0;
@@ -975,15 +986,15 @@ int do_ghosts(cfx_ctx *ctx, bool after_update) {
   return run_levels(ctx, seq, 0, seq.levels());
 }
 
-int do_elim(cfx_ctx *ctx, bool ring = false) {
+int do_elim(cfx_ctx *ctx) {
   if (ctx->dim != 2) return 0;
   for (auto &B : ctx->views)
-    CFX_TRY(ctx->timed_launch(K_OTHER, [&] { return launch_eliminate_k(B, ctx->ns, ring ? 1 : 0, ctx->stream); }));
+    CFX_TRY(ctx->timed_launch(K_OTHER, [&] { return launch_eliminate_k(B, ctx->ns, ctx->stream); }));
   return 0;
 }
 
-// plane: the plane k = 0 of 2-D blocks alone (not with the surrogate)
-int do_props(cfx_ctx *ctx, bool plane = false) {
+// mode: kProps... (the 2-D ones not with the surrogate)
+int do_props(cfx_ctx *ctx, int mode = kPropsPadded) {
   if (ctx->transport == CFX_TRANSPORT_MLP) {
     if (!ctx->mlp_ready) return ctx->fail(CFX_E_SURROGATE, "surrogate transport selected but not trained or loaded");
     auto fn = g_kernels32[ctx->ns].props_mlp;
@@ -996,15 +1007,17 @@ int do_props(cfx_ctx *ctx, bool plane = false) {
     return 0;
   }
   auto fn = ctx->mixed ? g_kernels32[ctx->ns].props : g_kernels64[ctx->ns].props;
-  CFX_TRY(per_batch(ctx, plane ? ctx->t_plane : ctx->t_pad, [&](const Batch &b) {
-    return ctx->timed_launch(K_PROPS, [&] { return fn(b, plane ? 1 : 0, ctx->sp_dev, ctx->S, ctx->stream); });
+  CFX_TRY(per_batch(ctx, mode == kPropsPadded ? ctx->t_pad : ctx->t_plane, [&](const Batch &b) {
+    return ctx->timed_launch(K_PROPS, [&] { return fn(b, mode, ctx->sp_dev, ctx->S, ctx->stream); });
   }));
   return 0;
 }
 
-int do_store_last(cfx_ctx *ctx) {
+// reset_dt: also resets the target of the global time step's reduction
+int do_store_last(cfx_ctx *ctx, bool reset_dt = false) {
+  auto *bits = reset_dt ? reinterpret_cast<unsigned long long *>(ctx->d_dt) : nullptr;
   CFX_TRY(per_batch(ctx, ctx->t_last, [&](const Batch &b) {
-    return ctx->timed_launch(K_OTHER, [&] { return launch_store_last(b, ctx->stream); });
+    return ctx->timed_launch(K_OTHER, [&] { return launch_store_last(b, ctx->last_iter, bits, ctx->stream); });
   }));
   return 0;
 }
@@ -1017,28 +1030,29 @@ int do_store_last(cfx_ctx *ctx) {
 // ghost fills, which cover their tangential rows too.  The stages within the
 // step therefore work on the plane alone (RHS without k differences, copies of
 // the ring near the faces, properties of the plane); the full copies and the
-// properties of all planes are made once, for the state the step leaves.
-// 1021x509 air, per stage: copies 40 -> 5 us, properties 28 -> 9 us.  (The
+// properties of all planes are made once, for the state the step leaves.  The
+// properties kernel makes the copies: 1021x509 air, copies and properties
+// together 68 us per stage -> 11 us within a step, 34 us at its end.  (The
 // surrogate counts the points it falls back on, over all planes, and keeps the
 // full stages.)
 int do_step(cfx_ctx *ctx) {
   int rc;
-  if ((rc = do_store_last(ctx))) return rc;
+  if ((rc = do_store_last(ctx, ctx->rk == 3))) return rc;
   const int stages = ctx->rk == 3 ? 3 : 1;
   const bool planar = ctx->plane_only && ctx->transport != CFX_TRANSPORT_MLP;
   for (int s = 0; s < stages; ++s) {
     const bool last = s == stages - 1;
     if ((rc = do_rhs(ctx, -1, planar && s > 0))) return rc;
     if (ctx->rk == 3) {
-      if (s == 0 && (rc = do_dt(ctx, 1, 0))) return rc;
+      if (s == 0 && (rc = do_dt(ctx, 1, 0, /*reset=*/false))) return rc;
     } else {
       if ((rc = do_dt(ctx, 0, 1))) return rc;
     }
     if (ctx->lusgs && (rc = do_lusgs(ctx))) return rc;
     if ((rc = do_update(ctx, s))) return rc;
     if ((rc = do_ghosts(ctx, true))) return rc;
-    if ((rc = do_elim(ctx, planar && !last))) return rc;
-    if ((rc = do_props(ctx, planar && !last))) return rc;
+    if (!planar && (rc = do_elim(ctx))) return rc;
+    if ((rc = do_props(ctx, !planar ? kPropsPadded : (last ? kPropsPlanes : kPropsRing)))) return rc;
   }
   return 0;
 }

@@ -101,6 +101,7 @@ struct cfx_ctx {
   Schedule sched_mid, sched_bc_step;
   ExStrips strips{};
   int n_fused = 0;
+  int dt_iter = kDtIter, last_iter = kLastIter;  // points per thread of these kernels
   bool plane_only = false;  // 2-D: no ghost fill reads more of the planes along k than the ring near the faces
   bool batched = true, use_graph = false;
   hipGraph_t graph = nullptr;

@@ -16,8 +16,8 @@ namespace cfx {
 
 // ------------------------------------------------------------ work units ---
 constexpr int kTpb = 256;        // threads per workgroup of the point kernels
-constexpr int kDtIter = 8;       // points per thread of the time-step reduction
-constexpr int kLastIter = 4;     // points per thread of the last-step snapshot
+constexpr int kDtIter = 8;       // most points per thread of the time-step reduction
+constexpr int kLastIter = 4;     // most points per thread of the last-step snapshot
 constexpr int kResIter = 8;      // points per thread of the residual partials
 
 // A batch of blocks: views[0..nb) with workgroup prefix off[0..nb] (device
@@ -65,12 +65,17 @@ inline int plane_groups(const int m[3], const PlaneTile &t) {
 // planar: the ghost planes along k equal the plane, and are not read
 using PlaneFn = int (*)(const Batch &b, int planar, const SpeciesDev *sp, const SchemeDev &S, hipStream_t st);
 
+// Properties over the padded range; or of the plane k = 0 alone with the copies
+// of the ring near the faces to the ghost planes along k; or of all planes, with
+// the copies of the whole plane.
+constexpr int kPropsPadded = 0, kPropsRing = 1, kPropsPlanes = 2;
+
 inline int rhs_variants(int dim) { return dim == 3 ? kNVar3 : kNVar2; }
 
 struct KernelSet64 {
   int present;
-  // plane: only the plane k = 0 of 2-D blocks (a batch of their planes)
-  int (*props)(const Batch &b, int plane, const SpeciesDev *sp, const SchemeDev &S, hipStream_t st);
+  // mode: kPropsPadded, or (2-D, a batch of the blocks' planes) kPropsRing, kPropsPlanes
+  int (*props)(const Batch &b, int mode, const SpeciesDev *sp, const SchemeDev &S, hipStream_t st);
   int (*cv_from_bv)(const Batch &b, const SpeciesDev *sp, const SchemeDev &S, hipStream_t st);
   int (*update)(const Batch &b, const SpeciesDev *sp, const SchemeDev &S, int mixed, int stage, const double *dt,
                 int *flags, unsigned long long *newton_fail, hipStream_t st);
@@ -96,7 +101,7 @@ struct KernelSet64 {
 struct MlpDev;
 struct KernelSet32 {
   int present;
-  int (*props)(const Batch &b, int plane, const SpeciesDev *sp, const SchemeDev &S, hipStream_t st);
+  int (*props)(const Batch &b, int mode, const SpeciesDev *sp, const SchemeDev &S, hipStream_t st);
   // properties with the surrogate transport (mixed precision)
   int (*props_mlp)(const Batch &b, const SpeciesDev *sp, const SchemeDev &S, const MlpDev *mlp, const void *ops,
                    const float *bias, unsigned long long *counters, hipStream_t st);
@@ -110,9 +115,11 @@ extern KernelSet32 g_kernels32[kMaxSp + 1];
 
 // ------------------------------------------------ species-independent ones ---
 int launch_dt_reset(unsigned long long *dt_bits, hipStream_t st);
-int launch_dt(const Batch &b, const SchemeDev &S, int ns, int store_local, unsigned long long *dt_bits,
+// iter: points per thread (as in the batch's prefix)
+int launch_dt(const Batch &b, const SchemeDev &S, int ns, int iter, int store_local, unsigned long long *dt_bits,
               hipStream_t st);
-int launch_store_last(const Batch &b, hipStream_t st);
+// reset (may be null): also resets the target of the reduction to follow
+int launch_store_last(const Batch &b, int iter, unsigned long long *reset, hipStream_t st);
 // metrics and Jacobian of one block from its coordinates over ngg+1 ghost
 // layers (3 planes of (mx+2ngg+2)(my+2ngg+2)(mz+2ngg+2)); FP32 copies when
 // metric32 is non-null; *bad counts points with a non-positive Jacobian
@@ -134,7 +141,6 @@ int launch_residual_partial(const Batch &b, double *partial, hipStream_t st);
 int launch_residual_final(const double *partial, int n, double *out, hipStream_t st);
 // every component of the strips, one lane per component, the fields over the wavefronts
 int launch_exchange_strips(const BlockView *views, const ExStrips &x, int ns, int mixed, hipStream_t st);
-// ring: only the points that a ghost fill reads
-int launch_eliminate_k(const BlockView &B, int ns, int ring, hipStream_t st);
+int launch_eliminate_k(const BlockView &B, int ns, hipStream_t st);
 
 }  // namespace cfx

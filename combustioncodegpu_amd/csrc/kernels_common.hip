@@ -39,20 +39,20 @@ __device__ __forceinline__ double wave_sum(double v) {
 
 // ------------------------------------------------------------- time step ---
 // SteadyTemporalScheme::compute_time_step (TemporalScheme.cu:10-43) over
-// kDtIter chunks of the block's interior points, then a wavefront
+// `iter` chunks of the block's interior points, then a wavefront
 // min-reduction of the CFL time step into *dt_bits (positive doubles order
 // like their bit patterns).
 __global__ void __launch_bounds__(kTpb) dt_kernel(const BlockView *__restrict__ views, const int *__restrict__ off,
-                                                  int nb, SchemeDev S, int ns, int store_local,
+                                                  int nb, SchemeDev S, int ns, int iter, int store_local,
                                                   unsigned long long *dt_bits) {
   __shared__ double red[kTpb / 64];
   const int w = blockIdx.x + off[0];
   const int blk = find_seg(off, nb, w);
   const GView B = gview(views[blk]);
   const long long np = B.np;
-  const long long base = (long long)(w - off[blk]) * (kTpb * kDtIter);
+  const long long base = (long long)(w - off[blk]) * (kTpb * iter);
   double dmin = 1e300;
-  for (int it = 0; it < kDtIter; ++it) {
+  for (int it = 0; it < iter; ++it) {
     const long long q = base + it * kTpb + threadIdx.x;
     if (q >= B.ni) break;
     const long long p = interior_pidx(B, q);
@@ -91,17 +91,21 @@ __global__ void __launch_bounds__(kTpb) dt_kernel(const BlockView *__restrict__ 
   }
 }
 
+constexpr unsigned long long kInfBits = 0x7FF0000000000000ull;
 __global__ void set_u64_kernel(unsigned long long *dst, unsigned long long v) { *dst = v; }
 
-// store_last_step (TimeAdvanceFunc.cu:13-24)
+// store_last_step (TimeAdvanceFunc.cu:13-24); reset (may be null): the target of
+// the time step's reduction that follows, set to +infinity
 __global__ void __launch_bounds__(kTpb) store_last_kernel(const BlockView *__restrict__ views,
-                                                          const int *__restrict__ off, int nb) {
+                                                          const int *__restrict__ off, int nb, int iter,
+                                                          unsigned long long *reset) {
+  if (reset && blockIdx.x == 0 && threadIdx.x == 0) *reset = kInfBits;
   const int w = blockIdx.x + off[0];
   const int blk = find_seg(off, nb, w);
   const GView B = gview(views[blk]);
   const long long np = B.np, ni = B.ni;
-  const long long base = (long long)(w - off[blk]) * (kTpb * kLastIter);
-  for (int it = 0; it < kLastIter; ++it) {
+  const long long base = (long long)(w - off[blk]) * (kTpb * iter);
+  for (int it = 0; it < iter; ++it) {
     const long long q = base + it * kTpb + threadIdx.x;
     if (q >= ni) break;
     const long long p = interior_pidx(B, q);
@@ -256,14 +260,12 @@ __global__ void __launch_bounds__(kStripTpb) exchange_strip_kernel(const BlockVi
   }
 }
 
-// eliminate_k_gradient (Field.cu:268-292), 2-D only; ring: only for the points
-// that a ghost fill reads, the ghosts and ngg + 1 layers behind every face
-__global__ void eliminate_k_kernel(BlockView view, int ns, int ring) {
+// eliminate_k_gradient (Field.cu:268-292), 2-D only
+__global__ void eliminate_k_kernel(BlockView view, int ns) {
   const GView B = gview(view);
   const int i = (int)(blockIdx.x * blockDim.x + threadIdx.x) - kNgg;
   const int j = (int)(blockIdx.y * blockDim.y + threadIdx.y) - kNgg;
   if (i >= B.mx + kNgg || j >= B.my + kNgg) return;
-  if (ring && i > kNgg && i < B.mx - 1 - kNgg && j > kNgg && j < B.my - 1 - kNgg) return;
   const long long np = B.np;
   const long long p0 = pidx(B, i, j, 0);
   for (int k = 1; k <= kNgg; ++k) {
@@ -290,14 +292,14 @@ __global__ void eliminate_k_kernel(BlockView view, int ns, int ring) {
 }  // namespace
 
 int launch_dt_reset(unsigned long long *dt_bits, hipStream_t st) {
-  set_u64_kernel<<<1, 1, 0, st>>>(dt_bits, 0x7FF0000000000000ull);
+  set_u64_kernel<<<1, 1, 0, st>>>(dt_bits, kInfBits);
   return (int)hipGetLastError();
 }
 
-int launch_dt(const Batch &b, const SchemeDev &S, int ns, int store_local, unsigned long long *dt_bits,
+int launch_dt(const Batch &b, const SchemeDev &S, int ns, int iter, int store_local, unsigned long long *dt_bits,
               hipStream_t st) {
   if (b.total <= 0) return 0;
-  dt_kernel<<<b.total, kTpb, 0, st>>>(b.views, b.off, b.nb, S, ns, store_local, dt_bits);
+  dt_kernel<<<b.total, kTpb, 0, st>>>(b.views, b.off, b.nb, S, ns, iter, store_local, dt_bits);
   return (int)hipGetLastError();
 }
 
@@ -544,9 +546,9 @@ int launch_metrics(const double *xyz, int mx, int my, int mz, double *metric, do
   return (int)hipGetLastError();
 }
 
-int launch_store_last(const Batch &b, hipStream_t st) {
+int launch_store_last(const Batch &b, int iter, unsigned long long *reset, hipStream_t st) {
   if (b.total <= 0) return 0;
-  store_last_kernel<<<b.total, kTpb, 0, st>>>(b.views, b.off, b.nb);
+  store_last_kernel<<<b.total, kTpb, 0, st>>>(b.views, b.off, b.nb, iter, reset);
   return (int)hipGetLastError();
 }
 
@@ -576,10 +578,10 @@ int launch_exchange_strips(const BlockView *views, const ExStrips &x, int ns, in
   return (int)hipGetLastError();
 }
 
-int launch_eliminate_k(const BlockView &B, int ns, int ring, hipStream_t st) {
+int launch_eliminate_k(const BlockView &B, int ns, hipStream_t st) {
   const dim3 tpb(16, 16, 1);
   const dim3 g((B.px + 15) / 16, (B.py + 15) / 16, 1);
-  eliminate_k_kernel<<<g, tpb, 0, st>>>(B, ns, ring);
+  eliminate_k_kernel<<<g, tpb, 0, st>>>(B, ns);
   return (int)hipGetLastError();
 }
 

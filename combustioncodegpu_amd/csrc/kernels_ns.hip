@@ -146,10 +146,13 @@ __device__ __forceinline__ void wilke_point(SpeciesPtrT<R> sp, const SchemeDev &
     out[2 + l] = fabs(X[l] - R(1)) < R(1e-3) ? mus : fdiv<R>((R(1) - Y[l]) * mu, (R(1) - X[l]) * R(S.sc));
 }
 
-// Properties over the padded range, or the plane k = 0 of it alone (PLANE, 2-D:
-// its rows are contiguous).  In R = float (mixed precision) the
+// Properties over the padded range, or (2-D) by the points of the plane k = 0,
+// whose rows are contiguous: MODE kPropsRing, its properties, and near the faces
+// the copies to the ghost planes along k (eliminate_k_gradient, Field.cu:268-292)
+// that the ghost fills read; kPropsPlanes, the properties of all planes (those of
+// equal points) and every copy.  In R = float (mixed precision) the
 // kernel also writes the FP32 copies of the primitives the FP32 RHS reads.
-template <typename R, bool PLANE>
+template <typename R, int MODE>
 __global__ void __launch_bounds__(kTpb) props_kernel(const BlockView *__restrict__ views, const int *__restrict__ off,
                                                      int nb, const SpeciesDev *__restrict__ spg, SchemeDev S) {
   const SpeciesPtrT<R> sp = const_table<R>(spg);
@@ -163,8 +166,8 @@ __global__ void __launch_bounds__(kTpb) props_kernel(const BlockView *__restrict
     __syncthreads();
   }
   const long long q = pw.base + threadIdx.x;
-  if (q >= (PLANE ? B.sz : np)) return;
-  const long long p = PLANE ? kNgg * B.sz + q : q;
+  if (q >= (MODE ? B.sz : np)) return;
+  const long long p = MODE ? kNgg * B.sz + q : q;
   const R t = R(B.bv[5 * np + p]);
   R out[4 + (NS > 0 ? NS : 0)];
   R Y[NSA];
@@ -188,32 +191,65 @@ __global__ void __launch_bounds__(kTpb) props_kernel(const BlockView *__restrict
     mixture_gamma_c<R>(sp, f32 ? nullptr : cpl, t, Y, cp, winv, out);
     wilke_point<R, !f32>(sp, S, t, Y, cp, winv, out + 2);
   }
-  if constexpr (f32) {
-    // loads first (T and Y are already held), then the stores
-    float b32[6];
+  // loads first (T and Y are already held), then the stores
+  double b64[6], c0 = 0;
+  if constexpr (f32 || MODE) {
 #pragma unroll
-    for (int v = 0; v < 6; ++v) b32[v] = float(B.bv[v * np + p]);
+    for (int v = 0; v < 6; ++v) b64[v] = B.bv[v * np + p];
+  }
+  double cvY[NSA];
+  if constexpr (MODE && f32) c0 = B.cv[p];
+  if constexpr (MODE && NS > 0) {
 #pragma unroll
-    for (int v = 0; v < 4 + NS; ++v) B.props32[v * np + p] = out[v];
+    for (int l = 0; l < NS; ++l) cvY[l] = f32 ? B.cv[(5 + l) * np + p] : double(Y[l]);
+  }
+  auto put = [&](long long x) {
+    if constexpr (f32) {
 #pragma unroll
-    for (int v = 0; v < 6; ++v) B.bv32[v * np + p] = b32[v];
-    if constexpr (NS > 0) {
+      for (int v = 0; v < 4 + NS; ++v) B.props32[v * np + x] = out[v];
 #pragma unroll
-      for (int l = 0; l < NS; ++l) B.yk32[l * np + p] = float(Y[l]);
+      for (int v = 0; v < 6; ++v) B.bv32[v * np + x] = float(b64[v]);
+      if constexpr (NS > 0) {
+#pragma unroll
+        for (int l = 0; l < NS; ++l) B.yk32[l * np + x] = float(Y[l]);
+      }
+    } else {
+#pragma unroll
+      for (int v = 0; v < 4 + NS; ++v) B.props[v * np + x] = out[v];
     }
-  } else {
+  };
+  put(p);
+  if constexpr (MODE) {
+    const int px = B.px, i = (int)q % px - kNgg, j = (int)q / px - kNgg;
+    if (MODE == kPropsRing && i > kNgg && i < B.mx - 1 - kNgg && j > kNgg && j < B.my - 1 - kNgg) return;
 #pragma unroll
-    for (int v = 0; v < 4 + NS; ++v) B.props[v * np + p] = out[v];
+    for (int g = -kNgg; g <= kNgg; ++g) {
+      if (g == 0) continue;
+      const long long x = p + g * B.sz;
+#pragma unroll
+      for (int v = 0; v < 6; ++v) B.bv[v * np + x] = b64[v];
+      if constexpr (f32) {  // the mixed path derives Y from cv: rho and rho*Y instead
+        B.cv[x] = c0;
+#pragma unroll
+        for (int l = 0; l < NS; ++l) B.cv[(5 + l) * np + x] = cvY[l];
+      } else {
+#pragma unroll
+        for (int l = 0; l < NS; ++l) B.yk[l * np + x] = cvY[l];
+      }
+      if (MODE == kPropsPlanes) put(x);
+    }
   }
 }
 
 template <typename R>
-int launch_props(const Batch &b, int plane, const SpeciesDev *sp, const SchemeDev &S, hipStream_t st) {
+int launch_props(const Batch &b, int mode, const SpeciesDev *sp, const SchemeDev &S, hipStream_t st) {
   if (b.total <= 0) return 0;
-  if (plane)
-    props_kernel<R, true><<<b.total, kTpb, 0, st>>>(b.views, b.off, b.nb, sp, S);
+  if (mode == kPropsRing)
+    props_kernel<R, kPropsRing><<<b.total, kTpb, 0, st>>>(b.views, b.off, b.nb, sp, S);
+  else if (mode == kPropsPlanes)
+    props_kernel<R, kPropsPlanes><<<b.total, kTpb, 0, st>>>(b.views, b.off, b.nb, sp, S);
   else
-    props_kernel<R, false><<<b.total, kTpb, 0, st>>>(b.views, b.off, b.nb, sp, S);
+    props_kernel<R, kPropsPadded><<<b.total, kTpb, 0, st>>>(b.views, b.off, b.nb, sp, S);
   return (int)hipGetLastError();
 }
 
