@@ -100,28 +100,34 @@ __device__ __forceinline__ void mixture_gamma_c(SpeciesPtrT<R> sp, const R *cpl,
 // = s_m/s_n (NS square roots instead of NS^2), and T*^-0.145 =
 // T^-0.145 (k/eps_l)^-0.145: one exponential per point, the species factor
 // from the table.
-// ROOTS: the roots and their reciprocals of all species at once (within an ulp
-// of the others).
-template <typename R, bool ROOTS = false>
+// FAST: the roots and their reciprocals of all species at once, and the quotients
+// of fdiv_n (within an ulp of the others).
+template <typename R, bool FAST = false>
 __device__ __forceinline__ void wilke_point(SpeciesPtrT<R> sp, const SchemeDev &S, R t, const R *Y, const R *cp,
                                             R winv, R *out) {
   // Chapman-Enskog species viscosity (Transport.cu:52-57)
   const R tm = fexp<R>(R(-0.145) * flog<R>(t)), st = fsqrt<R>(t);
   R mu_s[NSA], X[NSA], s[NSA], rs[NSA];
   const R imw = frcp<R>(winv);
+  auto div = [](R a, R b) {
+    R q;
+    if constexpr (FAST) fdiv_n<1, R>(&a, &b, &q);
+    else q = fdiv<R>(a, b);
+    return q;
+  };
 #pragma unroll
   for (int l = 0; l < NS; ++l) {
     X[l] = Y[l] * imw * R(sp->inv_mw[l]);
     const R tdl = t * R(sp->lj_inv[l]);
     const R a = tdl + R(0.5);
     const R omega = R(1.147) * (tm * R(sp->om145[l])) + frcp<R>(a * a);
-    mu_s[l] = fdiv<R>(R(sp->vis_coeff[l]) * st, omega);
-    if constexpr (!ROOTS) {
+    mu_s[l] = div(R(sp->vis_coeff[l]) * st, omega);
+    if constexpr (!FAST) {
       s[l] = fsqrt<R>(mu_s[l]);
       rs[l] = frcp<R>(s[l]);
     }
   }
-  if constexpr (ROOTS) fsqrt_n<NSA, R>(mu_s, s, rs);
+  if constexpr (FAST) fsqrt_n<NSA, R>(mu_s, s, rs);
   // Wilke mixing and Mason-Saxena conductivity (Transport.cu:58-83)
   R mu = 0, kappa = 0;
 #pragma unroll
@@ -134,8 +140,8 @@ __device__ __forceinline__ void wilke_point(SpeciesPtrT<R> sp, const SchemeDev &
       vt += q * q * R(sp->sqw8[m][n]) * X[n];
     }
     const R lam = mu_s[m] * (cp[m] + R(sp->cond_add[m]));
-    mu += fdiv<R>(mu_s[m] * X[m], vt);
-    kappa += fdiv<R>(lam * X[m], R(1.065) * vt - R(0.065) * X[m]);
+    mu += div(mu_s[m] * X[m], vt);
+    kappa += div(lam * X[m], R(1.065) * vt - R(0.065) * X[m]);
   }
   out[0] = mu;
   out[1] = kappa;
@@ -143,7 +149,7 @@ __device__ __forceinline__ void wilke_point(SpeciesPtrT<R> sp, const SchemeDev &
   const R mus = mu * R(S.inv_sc);
 #pragma unroll
   for (int l = 0; l < NS; ++l)
-    out[2 + l] = fabs(X[l] - R(1)) < R(1e-3) ? mus : fdiv<R>((R(1) - Y[l]) * mu, (R(1) - X[l]) * R(S.sc));
+    out[2 + l] = fabs(X[l] - R(1)) < R(1e-3) ? mus : div((R(1) - Y[l]) * mu, (R(1) - X[l]) * R(S.sc));
 }
 
 // Properties over the padded range, or (2-D) by the points of the plane k = 0,
