@@ -18,7 +18,6 @@ HostCopy::~HostCopy() {
 
 bool HostCopy::ready() {
   if (n_ > 0) return true;
-  if (hipGetDevice(&device_) != hipSuccess) return false;
   const int want = std::min<int>(kThreads, std::max(1u, std::thread::hardware_concurrency()));
   for (int t = 0; t < want; ++t) {
     if (!piece_[t] && hipHostMalloc(&piece_[t], kPiece, hipHostMallocDefault) != hipSuccess) {
@@ -39,13 +38,25 @@ bool HostCopy::ready() {
 int HostCopy::to_host(void *dst, const void *src, size_t n, hipStream_t st) {
   if (hipError_t e = hipStreamSynchronize(st)) return (int)e;
   std::unique_lock<std::mutex> lock(busy_, std::defer_lock);
-  if (n < kLeast || !lock.try_lock() || !ready()) return (int)hipMemcpy(dst, src, n, hipMemcpyDeviceToHost);
+  if (n < kLeast || !lock.try_lock()) return (int)hipMemcpy(dst, src, n, hipMemcpyDeviceToHost);
+  // events and transfers belong to the stream's device, which need not be the
+  // caller's current one
+  int device = 0, current = 0;
+  if (hipStreamGetDevice(st, &device) != hipSuccess || hipGetDevice(&current) != hipSuccess ||
+      hipSetDevice(device) != hipSuccess) {
+    (void)hipGetLastError();
+    return (int)hipMemcpy(dst, src, n, hipMemcpyDeviceToHost);
+  }
+  if (!ready()) {
+    (void)hipSetDevice(current);
+    return (int)hipMemcpy(dst, src, n, hipMemcpyDeviceToHost);
+  }
   // about two pieces per thread at least, of 512 KiB or more
   const size_t piece = std::min(kPiece, std::max<size_t>(n / (2 * kThreads) / 4096 * 4096, 512u << 10));
   std::atomic<size_t> next{0};
   std::atomic<int> error{0};
   auto work = [&](int t) {
-    int e = (int)hipSetDevice(device_);
+    int e = (int)hipSetDevice(device);
     while (e == 0 && error.load(std::memory_order_relaxed) == 0) {
       const size_t at = next.fetch_add(piece);
       if (at >= n) break;
@@ -69,6 +80,7 @@ int HostCopy::to_host(void *dst, const void *src, size_t n, hipStream_t st) {
   work(0);
   for (std::thread &m : more)
     if (m.joinable()) m.join();
+  (void)hipSetDevice(current);
   return error.load();
 }
 

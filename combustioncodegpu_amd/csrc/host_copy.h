@@ -35,7 +35,7 @@ class HostCopy {
  private:
   bool ready();
   std::mutex busy_;
-  int device_ = 0, n_ = 0;  // n_: threads that have a piece
+  int n_ = 0;  // threads that have a piece
   void *piece_[kThreads] = {};
   hipEvent_t done_[kThreads] = {};
 };
