@@ -421,9 +421,14 @@ int build_schedule(cfx_ctx *ctx, const std::vector<FaceOp> &all, Schedule &sc, i
   const int nlev = n ? *std::max_element(level.begin(), level.end()) + 1 : 0;
   std::vector<FaceOp> ordered;
   sc.lvl.assign(1, 0);
+  sc.copies.clear();
   for (int L = 0; L < nlev; ++L) {
     for (int i = 0; i < n; ++i)
       if (level[i] == L) ordered.push_back(all[first + i]);
+    bool copies = true;
+    for (int i = sc.lvl.back(); i < (int)ordered.size(); ++i)
+      copies = copies && (ordered[i].kind == CFX_BC_OUTFLOW || ordered[i].kind == kOpExchange);
+    sc.copies.push_back(copies ? 1 : 0);
     sc.lvl.push_back((int)ordered.size());
   }
   sc.off_host.assign(ordered.size() + 1, 0);
@@ -855,6 +860,8 @@ int run_levels(cfx_ctx *ctx, const Schedule &sc, int l0, int l1) {
     const int a = sc.lvl[L], b = sc.lvl[L + 1];
     const int total = sc.off_host[b] - sc.off_host[a];
     CFX_TRY(ctx->timed_launch(K_BC, [&] {
+      if (sc.copies[L])
+        return k.copy_ops(ctx->views_dev, sc.ops + a, sc.off + a, b - a, total, ctx->mixed ? 1 : 0, ctx->stream);
       return k.face_ops(ctx->views_dev, sc.ops + a, sc.off + a, b - a, total, ctx->sp_dev, ctx->S, ctx->inflow_dev,
                         ctx->stream);
     }));

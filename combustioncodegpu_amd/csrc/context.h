@@ -40,6 +40,7 @@ struct Schedule {
   int *off = nullptr;
   std::vector<int> off_host;
   std::vector<int> lvl;
+  std::vector<char> copies;  // per level: it only copies and averages
   int levels() const { return lvl.empty() ? 0 : (int)lvl.size() - 1; }
 };
 

@@ -82,6 +82,9 @@ struct KernelSet64 {
   // ops[0..nops) with workgroup prefix off[0..nops], total workgroups
   int (*face_ops)(const BlockView *views, const FaceOp *ops, const int *off, int nops, int total,
                   const SpeciesDev *sp, const SchemeDev &S, const InflowDev *inflow, hipStream_t st);
+  // the same for ops that only copy and average (outflow, exchange)
+  int (*copy_ops)(const BlockView *views, const FaceOp *ops, const int *off, int nops, int total, int mixed,
+                  hipStream_t st);
   PlaneFn plane[kNVar2];
   MarchFn march;
   OccFn march_occ;

@@ -724,25 +724,33 @@ __device__ __forceinline__ void bc_symmetry_point(const GView &B, const FaceRang
   }
 }
 
-// inner_communication (Field.cu:213-266) with the face loop of
-// Mesh.cpp:905-917 at loop point n: shared-face points are averaged between
-// the two blocks, ghost layers take the neighbour's values.
-__device__ __forceinline__ void exchange_point(const GView &B, const GView &T, const InnerDev &f,
-                                               const int n[3], bool ghosts_only) {
+// loop point n of an exchange: the point p of the block and t of the target, and
+// whether they are on the shared layer
+__device__ __forceinline__ bool exchange_pair(const GView &B, const GView &T, const InnerDev &f, const int n[3],
+                                              long long &p, long long &t) {
   int idx[3], d_idx[3], it[3];
   for (int q = 0; q < 3; ++q) {
     d_idx[q] = f.loop_dir[q] * n[q];
     idx[q] = f.rs[q] + d_idx[q];
   }
   for (int q = 0; q < 3; ++q) it[q] = f.ts[q] + f.target_loop_dir[q] * d_idx[f.src_tar[q]];
-  const long long p = pidx(B, idx[0], idx[1], idx[2]);
-  const long long t = pidx(T, it[0], it[1], it[2]);
+  p = pidx(B, idx[0], idx[1], idx[2]);
+  t = pidx(T, it[0], it[1], it[2]);
+  return idx[f.face] == (f.direction > 0 ? f.rs[f.face] : f.re[f.face]);
+}
+
+// inner_communication (Field.cu:213-266) with the face loop of
+// Mesh.cpp:905-917 at loop point n: shared-face points are averaged between
+// the two blocks, ghost layers take the neighbour's values.
+__device__ __forceinline__ void exchange_point(const GView &B, const GView &T, const InnerDev &f,
+                                               const int n[3], bool ghosts_only) {
+  long long p, t;
+  const bool shared = exchange_pair(B, T, f, n, p, t);
   const long long np = B.np, tnp = T.np;
-  const int face_layer = f.direction > 0 ? f.rs[f.face] : f.re[f.face];
   // Loads are grouped ahead of the stores (the two blocks' arrays may alias
   // as far as the compiler knows, so it keeps every store before any later
   // load: field by field, each would cost a memory round trip).
-  if (idx[f.face] == face_layer) {
+  if (shared) {
     if (ghosts_only) return;
     // the shared layer: both sides of a group of fields, then the averages
     auto average = [&](gptr<double> bb, gptr<double> tt, auto kc) {
@@ -812,6 +820,66 @@ __global__ void __launch_bounds__(kTpb) face_ops_kernel(const BlockView *__restr
     }
     default: break;
   }
+}
+
+// The same for a level that only copies and averages (outflow conditions,
+// exchanges): blockIdx.y takes one of the arrays bv, cv, yk, whose fields do not
+// depend on each other.  A third of the chain per thread, and of the registers
+// that hold a point's fields: the middles of 27 blocks of 20..90 points 424 -> 339
+// us FP64, of 64 blocks of 12..44 mixed 125 -> 96, the edges of one block 13 -> 8.
+__global__ void __launch_bounds__(kTpb) copy_ops_kernel(const BlockView *__restrict__ views,
+                                                        const FaceOp *__restrict__ ops, const int *__restrict__ off,
+                                                        int nops) {
+  const int w = blockIdx.x + off[0];
+  const int s = find_seg(off, nops, w);
+  const FaceOp &op = ops[s];
+  const long long n = (long long)(w - off[s]) * kTpb + threadIdx.x;
+  if (n >= op.npts) return;
+  const int e0 = op.ext[0], e1 = op.ext[1];
+  const int nn[3] = {(int)(n % e0), (int)((n / e0) % e1), (int)(n / ((long long)e0 * e1))};
+  const GView B = gview(views[op.blk]);
+  const long long np = B.np;
+  auto by_array = [&](auto f) {
+    if (blockIdx.y == 0) f(B.bv, std::integral_constant<int, 6>{}, 0);
+    else if (blockIdx.y == 1) f(B.cv, std::integral_constant<int, 5 + NS>{}, 1);
+    else if constexpr (NS > 0) f(B.yk, std::integral_constant<int, NS>{}, 2);
+  };
+  if (op.kind == CFX_BC_OUTFLOW) {
+    const long long p = pidx(B, op.r.rs[0] + nn[0], op.r.rs[1] + nn[1], op.r.rs[2] + nn[2]);
+    const long long stride[3] = {1, B.sy, B.sz}, step = op.r.direction * stride[op.r.face];
+    by_array([&](gptr<double> a, auto kc, int) {
+      constexpr int K = decltype(kc)::value;
+      double x[K];
+#pragma unroll
+      for (int l = 0; l < K; ++l) x[l] = a[l * np + p];
+#pragma unroll
+      for (int g = 1; g <= kNgg; ++g)
+#pragma unroll
+        for (int l = 0; l < K; ++l) a[l * np + p + g * step] = x[l];
+    });
+    return;
+  }
+  const GView T = gview(views[op.tgt]);
+  const long long tnp = T.np;
+  long long p, t;
+  const bool shared = exchange_pair(B, T, op.f, nn, p, t);
+  if (shared && op.ghosts_only) return;
+  by_array([&](gptr<double> a, auto kc, int which) {
+    constexpr int K = decltype(kc)::value;
+    const gptr<double> b = which == 0 ? T.bv : (which == 1 ? T.cv : T.yk);
+    double x[K];
+#pragma unroll
+    for (int l = 0; l < K; ++l) x[l] = b[l * tnp + t];
+    if (shared) {  // both sides take the average
+      double y[K];
+#pragma unroll
+      for (int l = 0; l < K; ++l) y[l] = a[l * np + p];
+#pragma unroll
+      for (int l = 0; l < K; ++l) b[l * tnp + t] = x[l] = 0.5 * (x[l] + y[l]);
+    }
+#pragma unroll
+    for (int l = 0; l < K; ++l) a[l * np + p] = x[l];
+  });
 }
 
 int launch_update(const Batch &b, const SpeciesDev *sp, const SchemeDev &S, int mixed, int stage, const double *dt,
@@ -1255,6 +1323,13 @@ int launch_face_ops(const BlockView *views, const FaceOp *ops, const int *off, i
   return (int)hipGetLastError();
 }
 
+int launch_copy_ops(const BlockView *views, const FaceOp *ops, const int *off, int nops, int total, int mixed,
+                    hipStream_t st) {
+  if (total <= 0) return 0;
+  copy_ops_kernel<<<dim3(total, NS > 0 && !mixed ? 3 : 2, 1), kTpb, 0, st>>>(views, ops, off, nops);
+  return (int)hipGetLastError();
+}
+
 // ------------------------------------------------- surrogate training set ---
 // Counter-based uniform in [0, 1): SplitMix64 finaliser of (seed, sample, k);
 // each sample owns 4096 counters (a sample draws at most 2 + ns (3*32 + 1)).
@@ -1343,6 +1418,7 @@ struct Register64 {
     k.cv_from_bv = launch_cv_from_bv;
     k.update = launch_update;
     k.face_ops = launch_face_ops;
+    k.copy_ops = launch_copy_ops;
     k.lusgs_coef = launch_lusgs_coef;
     k.lusgs_reset = launch_lusgs_reset;
     k.lusgs_sweep = launch_lusgs_sweep;
