@@ -43,7 +43,7 @@ def test_training_trajectory(ns, batch, epochs):
     the normalisation with the envelope, and the losses of the form with one
     wavefront per 32 samples and the operands packed anew for each step.  The
     same products and sums in the same order: equal up to 1e-6 of the largest."""
-    ref = np.load(os.path.join(os.path.dirname(__file__), "golden", "mlp_training.npz"))
+    ref = np.load(os.path.join(os.path.dirname(__file__), "trajectories", "mlp_training.npz"))
     g = solver(ns)
     rep = g.mlp_train(n_samples=40960, epochs=epochs, batch=batch, holdout=0.1)
     params, norm = g.mlp_get_params()
