@@ -80,8 +80,8 @@ def cpu_baseline(case, threads, steps=5):
 
 
 def measure_traffic(precision="fp64", timeout_s=240):
-    """HBM bytes of one RHS evaluation (three direction launches, default
-    tiles) measured in this run: two rocprofv3 counter passes over a child
+    """HBM bytes of one RHS evaluation (one launch, default chunk length)
+    measured in this run: two rocprofv3 counter passes over a child
     `bench.py --rhs-only 2` (FETCH_SIZE, then WRITE_SIZE, KiB per dispatch),
     each scaled by the factor the same counter reads for a plain device copy
     of known size (profiles/rhs_c1_<precision>_traffic.json: a 2 GiB float64
@@ -217,7 +217,7 @@ def measure_group(case, args, specs, rounds=5, traffic=None):
             out["rhs_tiles"] = info["tiles"]
         if "mlp_report" in info:
             out["mlp"] = {"training": info["mlp_report"], "counters": g.mlp_stats()}
-        # one timed RHS event per direction launch (batched: all blocks at once)
+        # one timed RHS event per launch (batched: all blocks at once)
         rhs_ms, rhs_n = kt["rhs"]
         stages = 3 * 3
         rhs_stage_s = rhs_ms / stages / 1e3
@@ -225,7 +225,7 @@ def measure_group(case, args, specs, rounds=5, traffic=None):
             bpc = BYTES_PER_CELL_STAGE_FP64 if precision == "fp64" else BYTES_PER_CELL_STAGE_MIXED
             achieved = bpc * case.n_cells / rhs_stage_s / 1e9
             # HBM bytes per RHS evaluation measured in this run with the
-            # default tiles (None for autotuned tiles, whose traffic differs)
+            # default chunk length (None for autotuned ones, whose traffic differs)
             tr = (traffic or {}).get(precision) if "tiles" not in info else None
             out["roofline"] = {
                 "bound": "hbm", "achieved": round(achieved, 2), "peak": HBM_PEAK_GBS, "unit": "GB/s",
@@ -235,7 +235,7 @@ def measure_group(case, args, specs, rounds=5, traffic=None):
                 "kernel_avg_ms_per_stage": round(rhs_stage_s * 1e3, 4),
                 "launches_per_stage": round(rhs_n / stages, 2), "bytes_per_cell_stage": round(bpc, 2)}
             # the same kernel against the vector ALU: FP64 / FP32 flops per stage
-            # counted with rocprofv3 VALU instruction counters on the default tiles
+            # counted with rocprofv3 VALU instruction counters, default chunk length
             fpath = os.path.join(ROOT, "profiles", f"rhs_c1_{precision}_flops.json")
             if os.path.exists(fpath) and "tiles" not in info and case.n_cells == 256 * 128 * 128:
                 with open(fpath) as f:
@@ -256,7 +256,7 @@ def measure_group(case, args, specs, rounds=5, traffic=None):
 def lusgs_form(case, args, cfl=5.0, steps=10):
     """The implicit LU-SGS step (local time step, CFL 5) on the same block,
     FP64, batched and graph-captured: time per step (one stage: RHS, local
-    dt, coefficient kernel, forward and backward hyperplane sweeps, update,
+    dt, coefficient kernel, forward and backward sweeps, update,
     ghost fill, properties) and per-kernel times; Mcell-updates/s counts
     interior cells x steps."""
     import copy

@@ -157,8 +157,10 @@ class Solver(StepContext):
         return list(v), list(p)
 
     def autotune(self, reps=3):
-        """Pick the fastest RHS tile shape and persistence per direction on
-        this context's blocks; returns (variants, persistence, ms per direction)."""
+        """Pick the fastest RHS variant (3-D: the planes a workgroup marches
+        through, 2-D: the tile shape) on this context's blocks; returns
+        (variants, persistence, ms), the choice and its time in the last
+        direction's place."""
         ms = (C.c_double * 3)()
         self._call("autotune", int(reps), ms)
         v, p = self.rhs_tiles()
