@@ -960,11 +960,11 @@ __global__ void __launch_bounds__(kTpb) lusgs_coef_kernel(const BlockView *__res
 // us, and the hand-overs, 3 us each beyond the steps.  The form before it ran
 // tiles of 4 x 8 x 8 cells, one launch per tile hyperplane, with two barriers per
 // step and the neighbours' terms formed by the consumer: 96x80x64 cells with 9
-// species took 80 launches of 39 us per solve, now two of 0.39 ms.  Measured on
+// species took 80 launches of 39 us per solve, now two of 0.36 ms.  Measured on
 // the way: one wavefront that also moves the cells 1.1 us per step; hand-over
 // records by cell instead of by step (scattered stores) 0.47 ms per sweep;
 // chunks of 4 steps, with three workgroups per CU, 0.42 (the workgroups of a CU
-// meet on one SIMD), with one 0.35, and 7% slower than 8 on larger blocks.
+// meet on one SIMD), with one 0.35, but 7% slower than 8 on larger blocks.
 constexpr int kLuCols = kLuP * kLuP, kLuG = 8;
 constexpr int kLuHeld = kLuCols * kLuG / 64;  // cells of a chunk per lane of the second wavefront
 static_assert(kLuCols == 16, "the columns of a variable group are one DPP row");
