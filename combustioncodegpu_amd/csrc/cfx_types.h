@@ -48,7 +48,7 @@ struct alignas(8 * sizeof(T)) MixRec {
 template <typename T>
 struct SpeciesT {
   ThermoRec<T> th[kMaxSp];   // the thermo arrays below, regrouped per species
-  MixRec<T> mix[2][kMaxSp];  // range 0 low, 1 high
+  MixRec<T> mix[3][kMaxSp];  // range 0 low, 1 high, 2 below t_low (linear in T)
   int ns;
   T mw[kMaxSp], inv_mw[kMaxSp], r_sp[kMaxSp];  // W, 1/W, R_u/W
   T t_low[kMaxSp], t_mid[kMaxSp];

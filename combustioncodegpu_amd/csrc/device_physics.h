@@ -207,12 +207,14 @@ __device__ __forceinline__ R on_all_lanes(R v) {
   return v;
 }
 
-// The NASA-7 range every lane of the wavefront is in, for every species:
-// kRangeHi (all in the high set), kRangeLo (all in the low set, above
-// t_low), kRangeEach (each lane in one of the two), or kRangeMixed.  Smooth fields put most wavefronts on one side of t_mid; those
-// evaluate one polynomial set instead of both (the value is the same bit for
-// bit: the general path selects the same expression).
-constexpr int kRangeMixed = 0, kRangeLo = 1, kRangeHi = 2, kRangeEach = 3;
+// The NASA-7 ranges of a wavefront's temperatures t0, t1: kRangeHi (every species
+// in its high set), kRangeLo (every one in its low set, above t_low), kRangeEach
+// (each temperature in one of the two), or kRangeAny (some below a t_low, or
+// between the species' t_mid).  It chooses where the coefficients are read, never
+// the value: the sums are the same ones in the same order, whatever the other
+// lanes hold.  (A face on the seam of two tiles is formed in both, next to other
+// faces, and its two fluxes have to be the same bits.)
+constexpr int kRangeAny = 0, kRangeLo = 1, kRangeHi = 2, kRangeEach = 3;
 template <typename R>
 __device__ __forceinline__ int thermo_range(SpeciesPtrT<R> sp, R t0, R t1) {
   const R hf = R(sp->hi_from), lf = R(sp->lo_from), lt = R(sp->lo_to);
@@ -220,7 +222,7 @@ __device__ __forceinline__ int thermo_range(SpeciesPtrT<R> sp, R t0, R t1) {
   if (__all(h0 && h1)) return kRangeHi;
   if (__all(l0 && l1)) return kRangeLo;
   if (__all((h0 || l0) && (h1 || l1))) return kRangeEach;
-  return kRangeMixed;
+  return kRangeAny;
 }
 
 // h and cp of one species from its thermo record c, each lane in its own range
@@ -244,45 +246,47 @@ __device__ __forceinline__ void species_h_cp(SpeciesPtrT<R> sp, int l, R t, R &h
   thermo_h_cp<R>(sp->th[l].v, t, h, cp);
 }
 
-// h_l(T) alone (the same value as thermo_h_cp's h), for loops that need no
-// cp: the marker on the selected cp would otherwise keep both cp
-// polynomials alive.
-template <typename R>
-__device__ __forceinline__ R species_h(SpeciesPtrT<R> sp, int l, R t) {
-  const auto &c = sp->th[l].v;
-  auto p5 = [&](int o) { return R(c[o]) + t * (R(c[o + 1]) + t * (R(c[o + 2]) + t * (R(c[o + 3]) + t * R(c[o + 4])))); };
-  const R h_lo = t * p5(kThH) + R(c[kThH + 5]);
-  const R h_hi = t * p5(kThH + 6) + R(c[kThH + 11]);
-  const R hp = on_all_lanes<R>(t >= R(c[kThTmid]) ? h_hi : h_lo);
-  const R tl = R(c[kThTlow]);
-  return t < tl ? R(c[kThHtlow]) + R(c[kThCptlow]) * (t - tl) : hp;
-}
-
-// The mixture coefficients of a kernel: a copy of the table in LDS (2 x NS
-// records of 8, range 0 first).  Read as constant memory only a few records
-// fit the scalar registers, so that every one or two species wait for a scalar
-// load; the LDS copy (broadcast reads) keeps many reads in flight, and lets
+// The mixture coefficients of a kernel: a copy of the table in LDS (3 x NS
+// records of 8: low sets, high sets, below t_low).  Read as constant memory only a
+// few records fit the scalar registers, so that every one or two species wait for a
+// scalar load; the LDS copy (broadcast reads) keeps many reads in flight, and lets
 // each lane have a range of its own: an FP64 RHS wavefront's AUSM+ phase took
 // 3.4k cycles with scalar loads, of which it issued 1.6k.
 template <int NS, typename R>
 struct ThermoLds {
   SpeciesPtrT<R> sp;
   const R *lds;
-  __device__ auto rec(int l) const { return sp->th[l].v; }
   __device__ const R *mix(bool hi) const { return lds + (hi ? NS * 8 : 0); }
+  // species l's record at temperature t
+  __device__ const R *rec(int l, R t) const {
+    return lds + 8 * l + (t < R(sp->t_low[l]) ? 2 * NS * 8 : (t >= R(sp->t_mid[l]) ? NS * 8 : 0));
+  }
 };
 
 // H_k = sum_l w_l h_{l,k}, k = 0..5, with the coefficients of range rg at
-// temperature t (kRangeLo, kRangeHi, or by lane with kRangeEach), N sums at
-// once over the weights w(n, l).
+// temperature t (by lane with kRangeEach, by lane and species with kRangeAny), N
+// sums at once over the weights w(n, l).  The fused products are written out: left
+// to the compiler, a branch may round x0 c0 + x1 c1 the other way round.
 template <int NS, int N, typename R, typename TH, typename W>
 __device__ __forceinline__ void mixture_sum(const TH &th, int rg, const R *t, W w, R (*H)[6]) {
   auto add = [&](const R *c, int n, int l) {
     const R x = w(n, l);
 #pragma unroll
-    for (int k = 0; k < 6; ++k) H[n][k] = l == 0 ? x * c[k] : H[n][k] + x * c[k];
+    for (int k = 0; k < 6; ++k) H[n][k] = l == 0 ? x * c[k] : fma(x, c[k], H[n][k]);
   };
   const R hf = R(th.sp->hi_from);
+  if (rg == kRangeAny) {
+#pragma unroll
+    for (int l = 0; l < NS; ++l) {
+#pragma unroll
+      for (int n = 0; n < N; ++n) {
+        add(th.rec(l, t[n]), n, l);
+        // (else the branches' sums are merged into one with every record in registers)
+        asm volatile("" : "+v"(H[n][0]), "+v"(H[n][1]), "+v"(H[n][2]), "+v"(H[n][3]), "+v"(H[n][4]), "+v"(H[n][5]));
+      }
+    }
+    return;
+  }
   if (N > 1 && rg == kRangeEach) {
 #pragma unroll
     for (int n = 0; n < N; ++n) {
@@ -300,8 +304,8 @@ __device__ __forceinline__ void mixture_sum(const TH &th, int rg, const R *t, W 
 }
 
 // h(T) and cp(T) = dh/dT of a mixture from its summed enthalpy coefficients
-// H_k = sum_l Y_l h_{l,k} (k = 0..5, in the layout of the thermo records, all
-// species in one range): cp's coefficients are (k + 1) H_k.
+// H_k = sum_l Y_l h_{l,k} (k = 0..5, in the layout of the thermo records): cp's
+// coefficients are (k + 1) H_k.
 // N mixtures in lockstep.
 template <int N, typename R>
 __device__ __forceinline__ void mixture_h_cp(const R (*C)[6], const R *t, R *h, R *cp) {
@@ -313,6 +317,15 @@ __device__ __forceinline__ void mixture_h_cp(const R (*C)[6], const R *t, R *h, 
     for (int n = 0; n < N; ++n) h[n] = C[n][k] + t[n] * h[n], cp[n] = R(k + 1) * C[n][k] + t[n] * cp[n];
 #pragma unroll
   for (int n = 0; n < N; ++n) h[n] = C[n][5] + t[n] * h[n];
+}
+
+// sum_l w_l h_l(t), the enthalpy that the diffusive fluxes w_l carry
+template <int NS, typename R, typename TH>
+__device__ __forceinline__ R carried_enthalpy(const TH &th, R t, const R *w) {
+  R H1[1][6];
+  mixture_sum<NS, 1, R>(th, thermo_range<R>(th.sp, t, t), &t, [&](int, int l) { return w[l]; }, H1);
+  const R *H = H1[0];
+  return H[5] + t * (H[0] + t * (H[1] + t * (H[2] + t * (H[3] + t * H[4]))));
 }
 
 // cp_l(T) only, frozen below t_low (Thermo.cu:49-63).  Loops over species
@@ -402,7 +415,7 @@ __device__ __forceinline__ void ausm_from_states(SpeciesPtrT<R> sp, const TH &th
 #pragma unroll
   for (int n = 0; n < 2; ++n) H[n] = R(0.5) * (P[n][1] * P[n][1] + P[n][2] * P[n][2] + P[n][3] * P[n][3]);
   if constexpr (NS > 0) {
-    R w[2] = {R(0), R(0)}, t[2], cp[2] = {R(0), R(0)};
+    R w[2] = {R(0), R(0)}, t[2], cp[2];
 #pragma unroll
     for (int l = 0; l < NS; ++l)
 #pragma unroll
@@ -413,26 +426,14 @@ __device__ __forceinline__ void ausm_from_states(SpeciesPtrT<R> sp, const TH &th
     for (int n = 0; n < 2; ++n) x[n] = P[n][4], y[n] = P[n][0] * w[n];
     fdiv_n<2, R>(x, y, t);
     const int rg = thermo_range<R>(sp, t[0], t[1]);
-    if (rg != kRangeMixed) {
-      // every lane in one range: the mixture's polynomial first
-      // (six coefficients, each summed over the species), evaluated once, in
-      // place of one enthalpy and one cp polynomial per species
-      R C[2][6], h[2];
-      mixture_sum<NS, 2, R>(th, rg, t, [&](int n, int l) { return P[n][5 + l]; }, C);
-      mixture_h_cp<2, R>(C, t, h, cp);
+    // the mixture's polynomial first (six coefficients, each summed over the
+    // species), evaluated once, in place of one enthalpy and one cp polynomial per
+    // species
+    R C[2][6], h[2];
+    mixture_sum<NS, 2, R>(th, rg, t, [&](int n, int l) { return P[n][5 + l]; }, C);
+    mixture_h_cp<2, R>(C, t, h, cp);
 #pragma unroll
-      for (int n = 0; n < 2; ++n) H[n] += h[n];
-    } else {
-#pragma unroll
-      for (int l = 0; l < NS; ++l)
-#pragma unroll
-        for (int n = 0; n < 2; ++n) {
-          R h, c;
-          thermo_h_cp<R>(th.rec(l), t[n], h, c);
-          H[n] += h * P[n][5 + l];
-          cp[n] += c * P[n][5 + l];
-        }
-    }
+    for (int n = 0; n < 2; ++n) H[n] += h[n];
 #pragma unroll
     for (int n = 0; n < 2; ++n) x[n] = cp[n] * (w[n] * t[n]), y[n] = cp[n] - w[n];
     fdiv_n<2, R>(x, y, c2);  // gamma R T

@@ -47,7 +47,7 @@ struct MarchShape {
   static constexpr int KVG = (NVS + GRP - 1) / GRP;    // variables per thread
   static constexpr int SLOT = NVS * PL;                // one resident plane
   static constexpr int COL = 3 * SLOT, FB = COL + NV * NFZ, ACC = FB + NV * NF;
-  static constexpr int MIX = (ACC + NV * NFZ + 3) / 4 * 4, TOTAL = MIX + 16 * NS;  // mixture coefficients (16-byte reads)
+  static constexpr int MIX = (ACC + NV * NFZ + 3) / 4 * 4, TOTAL = MIX + 24 * NS;  // mixture coefficients (16-byte reads)
   static_assert(NFZ % 64 == 0, "a wavefront of the dq pass works on one variable");
   static_assert(NF <= NT - 64 && PLP <= NT, "one face per thread, the last wavefront moves the data");
   static_assert(MIX % 4 == 0 && TOTAL * sizeof(R) <= 163840, "the planes and fluxes fit in LDS");
@@ -89,9 +89,9 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(WPE, WP
   const int tid = threadIdx.x;
   const unsigned syb = (unsigned)B.sy * sizeof(R), szb = (unsigned)B.sz * sizeof(R);
 
-  // the mixture coefficients of both ranges
+  // the mixture coefficients of all ranges
   if constexpr (NS > 0) {
-    for (int n = tid; n < 16 * NS; n += NT) sm[P::MIX + n] = sp->mix[n / (8 * NS)][n / 8 % NS].v[n % 8];
+    for (int n = tid; n < 24 * NS; n += NT) sm[P::MIX + n] = sp->mix[n / (8 * NS)][n / 8 % NS].v[n % 8];
   }
   const ThermoLds<NS, R> th{sp, sm + P::MIX};
 
@@ -474,17 +474,7 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(WPE, WP
             asm volatile("" : "+v"(dp[s]), "+v"(uc));
             __builtin_amdgcn_sched_barrier(0);
           });
-          // sum_l dp_l h_l(Ta): as the mixture polynomial where every lane is in one range
-          const int vrg = thermo_range<R>(sp, Ta, Ta);
-          if (vrg != kRangeMixed) {
-            R H2[1][6];
-            mixture_sum<NS, 1, R>(th, vrg, &Ta, [&](int, int s) { return dp[s]; }, H2);
-            const R *H = H2[0];
-            G4 += H[5] + Ta * (H[0] + Ta * (H[1] + Ta * (H[2] + Ta * (H[3] + Ta * H[4]))));
-          } else {
-#pragma unroll
-            for (int s = 0; s < NS; ++s) G4 += dp[s] * species_h<R>(sp, s, Ta);
-          }
+          G4 += carried_enthalpy<NS, R>(th, Ta, dp);
 #pragma unroll
           for (int s = 0; s < NS; ++s) sm[fb + (5 + s) * NF] -= dp[s] - yb[s] * (R(0.5) * uc);
         }

@@ -32,7 +32,7 @@ struct PlaneShape {
   static constexpr int NT = 512, NV = 5 + NS, NVS = 6 + NS;  // threads; fluxes; staged variables (with T)
   static constexpr int W0 = TX + 4, PL = W0 * (TY + 4);
   static constexpr int FB = NVS * PL;                            // flux slots, one per thread and variable
-  static constexpr int MIX = (FB + NV * NT + 3) / 4 * 4, TOTAL = MIX + 16 * NS;  // mixture coefficients (16-byte reads)
+  static constexpr int MIX = (FB + NV * NT + 3) / 4 * 4, TOTAL = MIX + 24 * NS;  // mixture coefficients (16-byte reads)
   static_assert((TX + 1) * TY <= 256 && TX * (TY + 1) <= 256 && PL <= NT, "one face and one staged point per thread");
   static_assert(TOTAL * sizeof(R) <= 163840, "the plane and the fluxes fit in LDS");
 };
@@ -107,7 +107,7 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(WPE, W
         rV[2 * v] = ldg<R>(PR_ + (2 + v) * np, pl_b), rV[2 * v + 1] = ldg<R>(PR_ + (2 + v) * np, pr_b);
     }
     if constexpr (NS > 0) {
-      for (int n = tid; n < 16 * NS; n += NT) sm[P::MIX + n] = sp->mix[n / (8 * NS)][n / 8 % NS].v[n % 8];
+      for (int n = tid; n < 24 * NS; n += NT) sm[P::MIX + n] = sp->mix[n / (8 * NS)][n / 8 % NS].v[n % 8];
     }
     if (tid < PL) {
 #pragma unroll
@@ -217,17 +217,7 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(WPE, W
           dp[s] = (rD[s][0] + rD[s][1]) * along(4 + s, yb[s]);
           uc += dp[s];
         }
-        // sum_l dp_l h_l(Ta): as the mixture polynomial where every lane is in one range
-        const int rg = thermo_range<R>(sp, Ta, Ta);
-        if (rg != kRangeMixed) {
-          R H2[1][6];
-          mixture_sum<NS, 1, R>(th, rg, &Ta, [&](int, int s) { return dp[s]; }, H2);
-          const R *H = H2[0];
-          G4 += H[5] + Ta * (H[0] + Ta * (H[1] + Ta * (H[2] + Ta * (H[3] + Ta * H[4]))));
-        } else {
-#pragma unroll
-          for (int s = 0; s < NS; ++s) G4 += dp[s] * species_h<R>(sp, s, Ta);
-        }
+        G4 += carried_enthalpy<NS, R>(th, Ta, dp);
 #pragma unroll
         for (int s = 0; s < NS; ++s) sm[fb + (5 + s) * NT] -= dp[s] - yb[s] * (R(0.5) * uc);
       }
