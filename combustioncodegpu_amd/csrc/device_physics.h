@@ -148,11 +148,11 @@ __device__ __forceinline__ void fdiv_n(const R *a, const R *b, R *q) {
     for (int n = 0; n < N; ++n) q[n] = fma(r[n], e[n], q[n]);
   }
 }
-// sqrt(a) and 1/sqrt(a) of positive, normal operands well inside the exponent
-// range.  FP64: one hardware reciprocal square root, g -> sqrt(a), h ->
-// 1/(2 sqrt(a)) by the coupled Newton iteration e = 1/2 - g h, g += g e,
-// h += h e, and two residual corrections of g (no scaling and special-value
-// steps, as for fdiv).
+// sqrt(a) and 1/sqrt(a) of operands well inside the exponent range.  FP64: one
+// hardware reciprocal square root, g -> sqrt(a), h -> 1/(2 sqrt(a)) by the coupled
+// Newton iteration e = 1/2 - g h, g += g e, h += h e, and two residual corrections
+// of g (no scaling and special-value steps, as for fdiv: the root of 0 or infinity
+// is NaN, and the caller's to replace where it can occur).
 template <int N, typename R>
 __device__ __forceinline__ void fsqrt_n(const R *a, R *g, R *rs) {
   if constexpr (sizeof(R) == 8) {
@@ -455,6 +455,10 @@ __device__ __forceinline__ void ausm_from_states(SpeciesPtrT<R> sp, const TH &th
   c2[2] = k1 * k1 + k2 * k2 + k3 * k3;
   R g[3], rs[3];
   fsqrt_n<3, R>(c2, g, rs);
+  if constexpr (sizeof(R) == 8) {  // the sound speed of a vacuum
+#pragma unroll
+    for (int n = 0; n < 2; ++n) g[n] = c2[n] == R(0) ? R(0) : g[n];
+  }
   const R gk = g[2], c = R(0.5) * (g[0] + g[1]);
   const R ic = frcp<R>(c) * rs[2];  // 1 / (c |k|)
   R m[2], a[2], b[2];

@@ -4,6 +4,7 @@ import numpy as np
 import pytest
 
 from combustioncodegpu_amd import abi, cases
+from tests.helpers import assert_close_sel
 
 pytestmark = pytest.mark.gpu
 
@@ -87,3 +88,21 @@ def test_infinite_density_or_pressure(n_spec, size, limiter, mixed):
         got = dq_with(Solver(make(size, n_spec, limiter, mixed)), var, INF, at)
         print(f"[broken] {size} ns={n_spec} limiter {limiter} mixed={mixed} bv[{var}]=inf", flush=True)
         assert np.array_equal(np.isfinite(got), np.isfinite(ref))
+
+
+@pytest.mark.parametrize("mixed", [False, True])
+@pytest.mark.parametrize("limiter", [0, 1])
+@pytest.mark.parametrize("size", SIZES)
+@pytest.mark.parametrize("n_spec", [0, 2, 9])
+def test_zero_pressure(n_spec, size, limiter, mixed):
+    """A vacuum's sound speed is 0: finite everywhere, and in FP64 the oracle's dq
+    at the step bar of 1e-12."""
+    from combustioncodegpu_amd.lib import Solver
+    from oracle.pyoracle import Oracle
+    at = (18, 9, size[2] // 2)
+    got = dq_with(Solver(make(size, n_spec, limiter, mixed)), 4, 0.0, at)
+    print(f"[broken] {size} ns={n_spec} limiter {limiter} mixed={mixed} p=0", flush=True)
+    assert np.isfinite(got).all()
+    if not mixed:
+        ref = dq_with(Oracle(make(size, n_spec, limiter)), 4, 0.0, at)
+        assert_close_sel(abi.DQ, got, ref, 1e-12, f"{size}")
