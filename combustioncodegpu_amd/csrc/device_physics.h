@@ -466,7 +466,8 @@ __device__ __forceinline__ void ausm_from_states(SpeciesPtrT<R> sp, const TH &th
   for (int n = 0; n < 2; ++n) m[n] = (k1 * P[n][1] + k2 * P[n][2] + k3 * P[n][3]) * ic;
   constexpr double alpha = 3 / 16.0;
   // split Mach numbers and pressures; beyond |M| = 1 the pressure split
-  // M+-/M is 1 or 0 by the sign of M
+  // M+-/M is 1 or 0 by the sign of M.  (M +- |M|, and not a maximum: of an infinite
+  // M it leaves NaN, so that an infinite velocity reaches the flux on every side)
 #pragma unroll
   for (int n = 0; n < 2; ++n) {
     const R o = n == 0 ? R(1) : R(-1);
@@ -474,8 +475,8 @@ __device__ __forceinline__ void ausm_from_states(SpeciesPtrT<R> sp, const TH &th
     b[n] = (m[n] * m[n] - R(1)) * (m[n] * m[n] - R(1));
   }
   const bool sl = fabs(m[0]) > R(1), sr = fabs(m[1]) > R(1);
-  const R mlp = sl ? fmax(m[0], R(0)) : a[0] + R(0.125) * b[0];
-  const R mrn = sr ? fmin(m[1], R(0)) : -a[1] - R(0.125) * b[1];
+  const R mlp = sl ? R(0.5) * (m[0] + fabs(m[0])) : a[0] + R(0.125) * b[0];
+  const R mrn = sr ? R(0.5) * (m[1] - fabs(m[1])) : -a[1] - R(0.125) * b[1];
   const R plp = sl ? (m[0] > R(0) ? R(1) : R(0)) : a[0] * (R(2) - m[0]) + R(alpha) * m[0] * b[0];
   const R prn = sr ? (m[1] < R(0) ? R(1) : R(0)) : a[1] * (R(2) + m[1]) - R(alpha) * m[1] * b[1];
   const R p_coeff = plp * pl[4] + prn * pr[4];
