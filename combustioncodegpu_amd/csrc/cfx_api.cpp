@@ -265,7 +265,7 @@ int plan_sweeps(cfx_ctx *ctx) {
   all.insert(all.end(), own.begin(), own.end());
   int rc = 0;
   ctx->lu_order = ctx->dalloc<LuPatch>(all.size(), rc);
-  ctx->lu_ticket = ctx->dalloc<int>(1, rc);
+  ctx->lu_ticket = ctx->dalloc<int>(2, rc);
   if (rc) return rc;
   return (int)hipMemcpy(ctx->lu_order, all.data(), sizeof(LuPatch) * all.size(), hipMemcpyHostToDevice);
 }

@@ -78,7 +78,7 @@ struct cfx_ctx {
   // block (index 0), in the order of their tickets
   LuPatch *lu_order = nullptr;
   std::vector<int> lu_off;                     // first entry of each block's own list, and the end
-  int *lu_ticket = nullptr;
+  int *lu_ticket = nullptr;                    // a sweep's ticket counter and its abort word
   bool lusgs = false;
   Table t_rhs[kNVar2];                         // 2-D: RHS tiles per variant
   Table t_plane;                               // 2-D: the points of the plane k = 0 with its ghosts

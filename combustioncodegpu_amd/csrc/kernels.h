@@ -93,8 +93,9 @@ struct KernelSet64 {
   int (*mlp_samples)(const SpeciesDev *sp, const SchemeDev &S, long long n, unsigned long long seed,
                      const double lim[4], double alpha, double *x, double *y, hipStream_t st);
   // LU-SGS: the diagonal and neighbour coefficients over the interior (point
-  // batch); what a sweep expects of its hand-over and its ticket counter (point
-  // batch); and the forward (fwd = 1) or backward sweep of n patches
+  // batch); what a sweep expects of its hand-over and of ticket[0..1], its ticket
+  // counter and abort word (point batch); and the forward (fwd = 1) or backward
+  // sweep of n patches
   int (*lusgs_coef)(const Batch &b, const SchemeDev &S, hipStream_t st);
   int (*lusgs_reset)(const Batch &b, int *ticket, hipStream_t st);
   int (*lusgs_sweep)(const BlockView *views, const LuPatch *order, int n, int *ticket, const SchemeDev &S, int fwd,

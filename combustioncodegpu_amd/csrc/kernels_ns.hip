@@ -9,6 +9,7 @@
 
 #include "device_physics.h"
 #include "kernels.h"
+#include "lusgs_plan.h"
 #include "mlp.h"
 #include "rhs_march.h"
 #include "rhs_plane.h"
@@ -951,7 +952,7 @@ __global__ void __launch_bounds__(kTpb) lusgs_coef_kernel(const BlockView *__res
 // last: a workgroup takes its patch from a ticket counter whose order holds
 // every patch behind the two that it waits for, so these are done or running.
 // (A wait beyond kLuWait, which none of this allows, is given up with an error
-// flag that ends every other wait as well.)
+// flag, and raises an abort word that ends the sweep's other waits: ticket[1].)
 //
 // The backward sweep is the forward one in mirrored indices, with the other
 // sign of dG.
@@ -991,13 +992,13 @@ __device__ __forceinline__ double first_row(double v) {
   return __hiloint2double((int)word((unsigned)__double2hiint(v)), (int)word((unsigned)__double2loint(v)));
 }
 
-// every place of a hand-over empty, the ticket counter back to 0
+// every place of a hand-over empty, the ticket counter and the abort word back to 0
 __global__ void __launch_bounds__(kTpb) lusgs_reset_kernel(const BlockView *__restrict__ views,
                                                            const int *__restrict__ off, int nb, int *ticket) {
   const PointWork pw = point_work(off, nb);
   const GView B = gview(views[pw.blk]);
   const long long q = pw.base + threadIdx.x;
-  if (blockIdx.x == 0 && threadIdx.x == 0) *ticket = 0;
+  if (blockIdx.x == 0 && threadIdx.x == 0) ticket[0] = ticket[1] = 0;
   if (q >= B.ni) return;
   const int m[3] = {B.mx, B.my, B.mz};
   const long long n = lu_hand_over(m, NS);
@@ -1225,20 +1226,20 @@ __global__ void __launch_bounds__(128, 1) lusgs_sweep_kernel(const BlockView *__
       const Cell &x = cell[t & 1];
       read(chunk, min(t + 1, kLuG - 1), cell[(t + 1) & 1]);
       u64 *aj = ij[t & 1], *ak = ik[t & 1];
-      if (__any(missing(aj, ak))) {
-        // (a patch that waits for its first terms leaves the memory to the others)
-        const long long until = (long long)wall_clock64() + kLuWait;
-        for (int spin = 1; __any(missing(aj, ak)); ++spin) {
-          if (s < kLuP) __builtin_amdgcn_s_sleep(16);
-          if (missing(aj, ak)) {
-            fetch(now(need_j, s), in_j, aj);
-            fetch(now(need_k, s), in_k, ak);
-          }
-          if (spin % 256) continue;
-          if ((long long)wall_clock64() > until) atomicOr(flags, kLuFlag);
-          if (__hip_atomic_load(flags, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & kLuFlag) break;
-        }
-      }
+      lu_wait([&] { return __any(missing(aj, ak)) != 0; },
+              [&] {  // (a patch that waits for its first terms leaves the memory to the others)
+                if (s < kLuP) __builtin_amdgcn_s_sleep(16);
+                if (missing(aj, ak)) {
+                  fetch(now(need_j, s), in_j, aj);
+                  fetch(now(need_k, s), in_k, ak);
+                }
+              },
+              [] { return (long long)wall_clock64(); }, kLuWait,
+              [&] {
+                atomicOr(flags, kLuFlag);
+                __hip_atomic_store(ticket + 1, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+              },
+              [&] { return __hip_atomic_load(ticket + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0; });
       double dn[NSL];
 #pragma unroll
       for (int q = 0; q < NSL; ++q) {

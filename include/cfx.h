@@ -262,7 +262,10 @@ int cfx_get_dt(cfx_ctx *ctx, double *dt);
 /* Set the device dt (fixed-dt runs). */
 int cfx_set_dt(cfx_ctx *ctx, double dt);
 /* Health check: synchronises and reports non-finite state (CFX_E_NONFINITE)
- * and Newton failures (CFX_E_NEWTON, count in *n_newton_fail if non-NULL). */
+ * and Newton failures (CFX_E_NEWTON, count in *n_newton_fail if non-NULL); an
+ * LU-SGS sweep that gave up waiting (hipErrorLaunchTimeOut; the increments of that
+ * sweep are not valid, later sweeps are not affected).  What has been found stays
+ * reported as long as the context lives. */
 int cfx_check(cfx_ctx *ctx, long long *n_newton_fail);
 /* Synchronise the context's stream. */
 int cfx_sync(cfx_ctx *ctx);
