@@ -248,21 +248,10 @@ int build_tables(cfx_ctx *ctx) {
 // the two patches a patch waits for stand before it.
 int plan_sweeps(cfx_ctx *ctx) {
   if (!ctx->lusgs) return 0;
-  std::vector<LuPatch> all, own;
-  std::vector<int> count;
-  for (size_t b = 0; b < ctx->hb.size(); ++b) {
-    const int nj = chunks(ctx->hb[b].my, kLuP), nk = chunks(ctx->hb[b].mz, kLuP);
-    for (int d = 0; d <= nj + nk - 2; ++d)
-      for (int K = std::max(0, d - nj + 1); K <= std::min(d, nk - 1); ++K) {
-        all.push_back(LuPatch{(int)b, d - K, K});
-        own.push_back(LuPatch{0, d - K, K});
-      }
-    count.push_back(nj * nk);
-  }
-  std::stable_sort(all.begin(), all.end(), [](const LuPatch &x, const LuPatch &y) { return x.J + x.K < y.J + y.K; });
-  ctx->lu_off.assign(1, (int)all.size());
-  for (int c : count) ctx->lu_off.push_back(ctx->lu_off.back() + c);
-  all.insert(all.end(), own.begin(), own.end());
+  std::vector<LuPatch> all;
+  std::vector<int> my, mz;
+  for (const HostBlock &H : ctx->hb) my.push_back(H.my), mz.push_back(H.mz);
+  lu_plan(my, mz, all, ctx->lu_off);
   int rc = 0;
   ctx->lu_order = ctx->dalloc<LuPatch>(all.size(), rc);
   ctx->lu_ticket = ctx->dalloc<int>(2, rc);

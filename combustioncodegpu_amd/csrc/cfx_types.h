@@ -9,6 +9,7 @@
 #include <cstdint>
 
 #include "../../include/cfx.h"
+#include "lusgs_plan.h"
 
 namespace cfx {
 
@@ -102,23 +103,6 @@ struct BlockView {
   int fuse[6];
   int fuse_any;
 };
-
-// LU-SGS sweeps: patches of kLuP x kLuP columns along i; the patch (J, K) of a
-// block, in the order in which wavefronts take them (any patch behind (J-1, K)
-// and (J, K-1)); and the values a sweep hands from patch to patch.
-constexpr int kLuP = 4;
-struct LuPatch {
-  int blk, J, K;
-};
-// a third of the species, and the places of a cell's variables: (rho, rho V, E)
-// and three groups of species
-__host__ __device__ constexpr int lu_third(int ns) { return (ns + 2) / 3; }
-__host__ __device__ constexpr int lu_places(int ns) { return 5 + 3 * lu_third(ns); }
-__host__ __device__ inline long long lu_hand_over(const int m[3], int ns) {
-  const long long nj = (m[1] + kLuP - 1) / kLuP, nk = (m[2] + kLuP - 1) / kLuP;
-  const long long wj = m[1] < kLuP ? m[1] : kLuP, wk = m[2] < kLuP ? m[2] : kLuP;
-  return nj * nk * (m[0] + wj + wk - 2) * lu_places(ns) * kLuP * ((nj > 1 ? 1 : 0) + (nk > 1 ? 1 : 0));
-}
 
 // Pointers in the global address space.  A view loaded from device memory
 // (the block table) hands out generic pointers, for which the compiler emits

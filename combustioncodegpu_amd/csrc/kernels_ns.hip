@@ -1037,25 +1037,18 @@ __global__ void __launch_bounds__(128, 1) lusgs_sweep_kernel(const BlockView *__
   const int jj = pt.J * kLuP + jl, kk = pt.K * kLuP + kl;
   const bool col = jj < my && kk < mz;
   const int h0 = vg == 0 ? 0 : 5 + (vg - 1) * N3;  // this lane's places
-  // hand-over to the next patch along j (then along k): [patch][step][variable of
-  // a group][group][kl], so that a step's values are a few whole lines
-  const int nJ = (my + kLuP - 1) / kLuP, nK = (mz + kLuP - 1) / kLuP, wj = min(kLuP, my), wk = min(kLuP, mz);
-  const int steps = mx + wj + wk - 2, n_chunk = (steps + kLuG - 1) / kLuG;
-  constexpr int ST = kLuP * NP;
-  const long long fs = (long long)steps * ST;
+  const int nJ = (my + kLuP - 1) / kLuP, steps = lu_steps(mx, my, mz), n_chunk = (steps + kLuG - 1) / kLuG;
+  constexpr int ST = lu_record(NS);
   const long long at = (long long)pt.K * nJ + pt.J;
   typedef unsigned long long u64;
   const gptr<u64> F = (gptr<u64>)B.luf;
-  const gptr<u64> FK = F + (nJ > 1 ? (long long)nJ * nK * fs : 0);
+  const gptr<u64> FK = F + lu_along_k(NS, mx, my, mz);
   const bool need_j = col && jl == 0 && jj > 0, need_k = col && kl == 0 && kk > 0;
   const bool give_j = col && jl == kLuP - 1 && jj + 1 < my, give_k = col && kl == kLuP - 1 && kk + 1 < mz;
-  // a cell that the patch before updates in its step s + kLuP - 1 is the upstream
-  // neighbour of one of step s here
-  gptr<u64> in_j = F + (at - 1) * fs + (kLuP - 1) * ST + kLuP * vg + kl;
-  gptr<u64> in_k = FK + (at - nJ) * fs + (kLuP - 1) * ST + kLuP * vg + jl;
-  gptr<u64> out_j = F + at * fs + kLuP * vg + kl, out_k = FK + at * fs + kLuP * vg + jl;
-  // this lane's value q in a step's record (from N3 on group 0's alone)
-  auto place = [](int q) { return q < N3 ? 4 * kLuP * q : (3 * N3 + q) * kLuP; };
+  gptr<u64> in_j = F + lu_at(NS, steps, at - 1, kLuAhead, vg, kl);
+  gptr<u64> in_k = FK + lu_at(NS, steps, at - nJ, kLuAhead, vg, jl);
+  gptr<u64> out_j = F + lu_at(NS, steps, at, 0, vg, kl), out_k = FK + lu_at(NS, steps, at, 0, vg, jl);
+  auto place = [](int q) { return lu_place(NS, q); };  // this lane's value q in a step's record
 
   if (mover) {
     // ---- the second wavefront moves the cells: lane e + kLuG (column % 8) holds
@@ -1208,7 +1201,7 @@ __global__ void __launch_bounds__(128, 1) lusgs_sweep_kernel(const BlockView *__
   double T0[NSL], T1[NSL], T2[NSL];
 #pragma unroll
   for (int q = 0; q < NSL; ++q) T0[q] = T1[q] = T2[q] = 0.0;
-  auto now = [&](bool need, int s) { return need && s >= jl + kl && s < mx + jl + kl; };
+  auto now = [&](bool need, int s) { return need && lu_active(mx, jl, kl, s); };
 #pragma unroll
   for (int s = 0; s < 2; ++s) {
     fetch(now(need_j, s), in_j + s * ST, ij[s]);
@@ -1222,7 +1215,7 @@ __global__ void __launch_bounds__(128, 1) lusgs_sweep_kernel(const BlockView *__
 #pragma unroll 2
     for (int t = 0; t < kLuG; ++t) {
       const int s = n * kLuG + t;
-      const bool act = col && s >= jl + kl && s < mx + jl + kl;
+      const bool act = col && lu_active(mx, jl, kl, s);
       const Cell &x = cell[t & 1];
       read(chunk, min(t + 1, kLuG - 1), cell[(t + 1) & 1]);
       u64 *aj = ij[t & 1], *ak = ik[t & 1];
