@@ -39,6 +39,13 @@ int HostCopy::to_host(void *dst, const void *src, size_t n, hipStream_t st) {
   if (hipError_t e = hipStreamSynchronize(st)) return (int)e;
   std::unique_lock<std::mutex> lock(busy_, std::defer_lock);
   if (n < kLeast || !lock.try_lock()) return (int)hipMemcpy(dst, src, n, hipMemcpyDeviceToHost);
+  if (n_ == 0) {
+    asked_ += n;
+    if (asked_ < kWorth) {
+      lock.unlock();
+      return (int)hipMemcpy(dst, src, n, hipMemcpyDeviceToHost);
+    }
+  }
   // events and transfers belong to the stream's device, which need not be the
   // caller's current one
   int device = 0, current = 0;

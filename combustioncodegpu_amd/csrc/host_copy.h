@@ -23,6 +23,13 @@ class HostCopy {
   // smaller copies go through hipMemcpy: 3.4 MB 0.22 ms there; with the threads
   // 5 MB 0.34, 9 MB 0.52, 17 MB 0.70, 68 MB 2.0 ms (hipMemcpy 6.5)
   static constexpr size_t kLeast = 8u << 20;
+  // The pinned pieces and their events take 1 to 3 ms to set up, 7 for the first
+  // context of a process, and what they save adds up to that over about this many
+  // bytes (a process's first copy, hipMemcpy and new pieces: 17 MB 2.2 and 7.9 ms,
+  // 56 MB 5.7 and 9.5, 86 MB 9.0 and 10.0, 112 MB 11.0 and 10.5).  So they are set
+  // up for a copy of this size, or once the copies so far add up to it: a program
+  // that fetches a field or two does not pay for them.
+  static constexpr size_t kWorth = 96u << 20;
   HostCopy() = default;
   HostCopy(const HostCopy &) = delete;
   HostCopy &operator=(const HostCopy &) = delete;
@@ -35,7 +42,8 @@ class HostCopy {
  private:
   bool ready();
   std::mutex busy_;
-  int n_ = 0;  // threads that have a piece
+  size_t asked_ = 0;  // bytes asked for before the pieces were set up
+  int n_ = 0;         // threads that have a piece
   void *piece_[kThreads] = {};
   hipEvent_t done_[kThreads] = {};
 };
