@@ -35,10 +35,19 @@ bool HostCopy::ready() {
   return n_ > 0;
 }
 
+// Whether p is ordinary host memory.  The runtime itself copies at the link's rate
+// into pinned memory, and the processor need not reach device memory at all.
+static bool pageable(const void *p) {
+  hipPointerAttribute_t a{};
+  if (hipPointerGetAttributes(&a, p) == hipSuccess) return a.type == hipMemoryTypeUnregistered;
+  (void)hipGetLastError();
+  return true;
+}
+
 int HostCopy::to_host(void *dst, const void *src, size_t n, hipStream_t st) {
   if (hipError_t e = hipStreamSynchronize(st)) return (int)e;
   std::unique_lock<std::mutex> lock(busy_, std::defer_lock);
-  if (n < kLeast || !lock.try_lock()) return (int)hipMemcpy(dst, src, n, hipMemcpyDeviceToHost);
+  if (n < kLeast || !pageable(dst) || !lock.try_lock()) return (int)hipMemcpy(dst, src, n, hipMemcpyDeviceToHost);
   if (n_ == 0) {
     asked_ += n;
     if (asked_ < kWorth) {

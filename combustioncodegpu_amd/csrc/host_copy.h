@@ -34,9 +34,9 @@ class HostCopy {
   HostCopy(const HostCopy &) = delete;
   HostCopy &operator=(const HostCopy &) = delete;
   ~HostCopy();
-  // n bytes of device memory src to host memory dst, after the work on stream
-  // st; returns a hipError_t.  Callers that find the pieces in use by another
-  // thread, or no pinned memory, copy with hipMemcpy.
+  // n bytes of device memory src to dst, after the work on stream st; returns a
+  // hipError_t.  Callers that find the pieces in use by another thread, or no
+  // pinned memory, or whose dst is pinned or device memory, copy with hipMemcpy.
   int to_host(void *dst, const void *src, size_t n, hipStream_t st);
 
  private:

@@ -31,6 +31,14 @@ inline int hipStreamGetDevice(hipStream_t, int *d) { *d = 0; return 0; }
 inline int hipGetDevice(int *d) { *d = 0; return 0; }
 inline int hipSetDevice(int) { return 0; }
 inline int hipGetLastError() { return 0; }
+enum hipMemoryType { hipMemoryTypeUnregistered = 0, hipMemoryTypeHost = 1, hipMemoryTypeDevice = 2 };
+struct hipPointerAttribute_t { hipMemoryType type; };
+inline int memory_type = 0;  // of every destination; -1: the runtime does not know the pointer
+inline int hipPointerGetAttributes(hipPointerAttribute_t *a, const void *) {
+  if (memory_type < 0) return hipErrorInvalidValue;
+  a->type = (hipMemoryType)memory_type;
+  return 0;
+}
 inline int hipMemcpy(void *d, const void *s, size_t n, int) { ++n_plain; std::memcpy(d, s, n); return 0; }
 inline int hipMemcpyAsync(void *d, const void *s, size_t n, int, hipStream_t) { ++n_async; std::memcpy(d, s, n); return 0; }
 """
@@ -39,12 +47,13 @@ HARNESS = r"""
 #include <cstdio>
 #include <vector>
 #include "host_copy.h"
-// argv: copies in MiB; prints for each whether it went through hipMemcpy, the pinned pieces there are, and
+// argv: the destinations' memory type, copies in MiB; prints for each whether it went through hipMemcpy, the pinned pieces there are, and
 // whether every byte arrived
 int main(int argc, char **argv) {
   {
     cfx::HostCopy c;
-    for (int a = 1; a < argc; ++a) {
+    memory_type = std::atoi(argv[1]);
+    for (int a = 2; a < argc; ++a) {
       const size_t n = (size_t)(std::atof(argv[a]) * 1048576) + 13;
       std::vector<unsigned char> src(n), dst(n + 8, 77);
       for (size_t i = 0; i < n; ++i) src[i] = (unsigned char)(i * 2654435761u >> 13);
@@ -69,8 +78,8 @@ def exe(tmp_path_factory):
     subprocess.run(["g++", "-std=c++17", "-O1", "-pthread", "-I", str(d), "-I", CSRC, str(d / "main.cpp"),
                     os.path.join(CSRC, "host_copy.cpp"), "-o", str(d / "main")], check=True)
 
-    def run(*mib):
-        r = subprocess.run([str(d / "main")] + [str(m) for m in mib], capture_output=True, text=True, check=True)
+    def run(*mib, memory=0):
+        r = subprocess.run([str(d / "main"), str(memory)] + [str(m) for m in mib], capture_output=True, text=True, check=True)
         rows = r.stdout.split("\n")[:-1]
         assert rows[-1] == "left 0"
         return [tuple(map(int, x.split())) for x in rows[:-1]]
@@ -93,3 +102,14 @@ def test_pieces_where_they_are_worth_it(exe, before, last):
     pinned = rows[len(before)][1]
     assert 1 <= pinned <= 8
     assert rows[len(before):] == [(0, pinned, 1), (0, pinned, 1), (1, pinned, 1), (0, pinned, 1)]
+
+
+@pytest.mark.parametrize("memory", [1, 2])
+def test_pinned_or_device_destination(exe, memory):
+    """The runtime copies there by itself: no pieces, no store by the processor."""
+    assert exe(130.3, 100, memory=memory) == [(1, 0, 1)] * 2
+
+
+def test_unknown_pointer_is_ordinary_memory(exe):
+    rows = exe(130.3, memory=-1)
+    assert rows[0][0] == 0 and rows[0][2] == 1
