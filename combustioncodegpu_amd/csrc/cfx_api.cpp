@@ -1034,11 +1034,15 @@ int do_store_last(cfx_ctx *ctx, bool reset_dt = false) {
 // together 68 us per stage -> 11 us within a step, 34 us at its end.  (The
 // surrogate counts the points it falls back on, over all planes, and keeps the
 // full stages.)
+bool works_on_plane(const cfx_ctx *ctx) { return ctx->plane_only && ctx->transport != CFX_TRANSPORT_MLP; }
+// whether a step has stages after the first that do
+bool stages_on_plane(const cfx_ctx *ctx) { return ctx->rk == 3 && works_on_plane(ctx); }
+
 int do_step(cfx_ctx *ctx) {
   int rc;
   if ((rc = do_store_last(ctx, ctx->rk == 3))) return rc;
   const int stages = ctx->rk == 3 ? 3 : 1;
-  const bool planar = ctx->plane_only && ctx->transport != CFX_TRANSPORT_MLP;
+  const bool planar = works_on_plane(ctx);
   for (int s = 0; s < stages; ++s) {
     const bool last = s == stages - 1;
     if ((rc = do_rhs(ctx, -1, planar && s > 0))) return rc;
@@ -1663,7 +1667,9 @@ int cfx_get_rhs_tiles(cfx_ctx *ctx, int variant[3], int persist[3]) {
 
 // Times every variant on this context's blocks (reps launches each, after one
 // warm-up launch) and keeps the fastest: in 2-D every tile shape, in 3-D every
-// chunk length of the march; the choice is the last direction's.  dq holds no
+// chunk length of the march; the choice is the last direction's.  What is timed is
+// what a step runs: where the later stages of RK3 work on the plane alone (see
+// do_step), one RHS with the differences along k and two without.  dq holds no
 // result afterwards; the next RHS rewrites it.
 int cfx_autotune(cfx_ctx *ctx, int reps, double *best_ms) {
   if (!ctx || reps <= 0) return CFX_E_ARG;
@@ -1675,19 +1681,25 @@ int cfx_autotune(cfx_ctx *ctx, int reps, double *best_ms) {
   int rc = 0;
   if (best_ms)
     for (int d = 0; d < ctx->dim; ++d) best_ms[d] = 0;
-  const int d = ctx->dim - 1;
+  const int d = ctx->dim - 1, n = stages_on_plane(ctx) ? 3 : 1;
   double best = 1e30;
   int bv = 0;
+  auto evaluate = [&] {
+    for (int s = 0; s < n; ++s)
+      if (int e = do_rhs(ctx, -1, /*planar=*/s > 0)) return e;
+    return 0;
+  };
   for (int v = 0; v < rhs_variants(ctx->dim) && !rc; ++v) {
     ctx->rhs_var[d] = v;
-    if ((rc = do_rhs(ctx, -1))) break;
+    if ((rc = evaluate())) break;
     (void)hipEventRecord(a, ctx->stream);
-    for (int r = 0; r < reps && !rc; ++r) rc = do_rhs(ctx, -1);
+    for (int r = 0; r < reps && !rc; ++r) rc = evaluate();
     (void)hipEventRecord(b, ctx->stream);
     (void)hipEventSynchronize(b);
     float ms = 0;
     (void)hipEventElapsedTime(&ms, a, b);
-    if (ms / reps < best) best = ms / reps, bv = v;
+    const double each = ms / ((double)reps * n);
+    if (each < best) best = each, bv = v;
   }
   ctx->rhs_var[d] = bv;
   if (best_ms) best_ms[d] = best;

@@ -317,9 +317,10 @@ int cfx_rhs_variants(cfx_ctx *ctx);
 int cfx_set_rhs_variant(cfx_ctx *ctx, int variant);
 int cfx_set_rhs_tiles(cfx_ctx *ctx, const int variant[3], const int persist[3]);
 int cfx_get_rhs_tiles(cfx_ctx *ctx, int variant[3], int persist[3]);
-/* Times every variant on the context's blocks, reps launches each, and keeps
- * the fastest; best_ms[3] (may be NULL) receives the launch's time in the last
- * direction's place and 0 in the others.  Leaves dq undefined. */
+/* Times every variant on the context's blocks, reps launches each (2-D with
+ * rk_stages 3: reps times the three launches of a step), and keeps the fastest;
+ * best_ms[3] (may be NULL) receives the time of a launch in the last direction's
+ * place and 0 in the others.  Leaves dq undefined. */
 int cfx_autotune(cfx_ctx *ctx, int reps, double *best_ms);
 
 /* ------------------------------------------------ transport surrogate ---
