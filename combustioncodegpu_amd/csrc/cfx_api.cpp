@@ -60,13 +60,10 @@ void fill_thermo(SpeciesT<T> &s) {
       for (int k = 0; k < 5; ++k) v[kThCp + 5 * g + k] = s.cpc[g][l][k];
       for (int k = 0; k < 6; ++k) v[kThH + 6 * g + k] = s.hc[g][l][k];
     }
-    for (int g = 0; g < 2; ++g) {
+    for (int g = 0; g < 2; ++g)
       for (int k = 0; k < 6; ++k) s.mix[g][l].v[k] = s.hc[g][l][k];
-      s.mix[g][l].v[6] = s.inv_mw[l];
-    }
     s.mix[2][l].v[0] = s.cp_tlow[l];
     s.mix[2][l].v[5] = (T)((double)s.h_tlow[l] - (double)s.cp_tlow[l] * (double)s.t_low[l]);
-    s.mix[2][l].v[6] = s.inv_mw[l];
     v[kThTmid] = s.t_mid[l];
     v[kThTlow] = s.t_low[l];
     v[kThHtlow] = s.h_tlow[l];

@@ -38,9 +38,9 @@ struct alignas(64) ThermoRec {
 };
 
 
-// The enthalpy coefficients of one species in one range alone, for the sums
-// over species that form a mixture's polynomial: [0..5] as kThH, [6] 1/W.
-// One record is one scalar load (16 dwords in FP64, 8 in FP32).
+// The enthalpy coefficients of one species in one range, for the sums over species
+// that form a mixture's polynomial: [0..5] as kThH, then two places of padding, so
+// that the copy in LDS is read in 16-byte pieces.
 template <typename T>
 struct alignas(8 * sizeof(T)) MixRec {
   T v[8];

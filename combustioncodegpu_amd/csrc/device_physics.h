@@ -101,31 +101,12 @@ __device__ __forceinline__ R flog(R a) { return log(a); }
 template <>
 __device__ __forceinline__ float flog<float>(float a) { return __builtin_amdgcn_logf(a) * 0.6931471805599453f; }
 
-// N reciprocals, quotients or square roots at once, each step over all of
-// them before the next: an FP64 chain of dependent operations leaves most
-// issue slots of a wavefront empty (two wavefronts share a SIMD in the FP64
-// kernels), and the compiler keeps the order in which chains are written.
-// The reciprocals are those of the single form.  The quotients take one Newton
-// step less: with r within 2^-40 of 1/b the residual correction q + r (a - b q)
-// leaves nothing but its own rounding (2^-80 of q), whatever the second step adds.
-template <int N, typename R>
-__device__ __forceinline__ void frcp_n(const R *b, R *r) {
-  if constexpr (sizeof(R) == 8) {
-    R e[N];
-#pragma unroll
-    for (int n = 0; n < N; ++n) r[n] = __builtin_amdgcn_rcp(b[n]);
-#pragma unroll
-    for (int it = 0; it < 2; ++it) {
-#pragma unroll
-      for (int n = 0; n < N; ++n) e[n] = fma(-b[n], r[n], R(1));
-#pragma unroll
-      for (int n = 0; n < N; ++n) r[n] = fma(r[n], e[n], r[n]);
-    }
-  } else {
-#pragma unroll
-    for (int n = 0; n < N; ++n) r[n] = frcp<R>(b[n]);
-  }
-}
+// N quotients or square roots at once, each step over all of them before the next:
+// an FP64 chain of dependent operations leaves most issue slots of a wavefront empty
+// (two wavefronts share a SIMD in the FP64 kernels), and the compiler keeps the order
+// in which chains are written.  The quotients take one Newton step less than fdiv:
+// with r within 2^-40 of 1/b the residual correction q + r (a - b q) leaves nothing
+// but its own rounding (2^-80 of q), whatever the second step adds.
 template <int N, typename R>
 __device__ __forceinline__ void fdiv_n(const R *a, const R *b, R *q) {
   R r[N], e[N];
@@ -137,7 +118,8 @@ __device__ __forceinline__ void fdiv_n(const R *a, const R *b, R *q) {
 #pragma unroll
     for (int n = 0; n < N; ++n) r[n] = fma(r[n], e[n], r[n]);
   } else {
-    frcp_n<N, R>(b, r);
+#pragma unroll
+    for (int n = 0; n < N; ++n) r[n] = frcp<R>(b[n]);
   }
 #pragma unroll
   for (int n = 0; n < N; ++n) q[n] = a[n] * r[n];
@@ -380,9 +362,9 @@ __device__ __forceinline__ void limiter_n(const R *a, const R *b, R *s) {
 }
 
 // MUSCL kappa = 1/3 on one variable (Reconstruction.cu:26-44), or first
-// order.  Both limiters are symmetric, lim(a,b) == lim(b,a) bit for bit, so
-// the reference's four calls per face reduce to the two limited slopes of
-// the two cells: (1-kappa)/4 + (1+kappa)/4 = 1/2.
+// order.  Both limiters are symmetric (Van Albada up to the rounding of its
+// denominator), so the reference's four calls per face reduce to the two limited
+// slopes of the two cells: (1-kappa)/4 + (1+kappa)/4 = 1/2.
 // N variables in lockstep, q[n][0..3] the four points; MODE: 0 minmod, 1 Van
 // Albada, 2 first order.
 template <int MODE, int N, typename R>

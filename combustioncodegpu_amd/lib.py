@@ -146,6 +146,8 @@ class Solver(StepContext):
         self._call("set_rhs_variant", int(v))
 
     def set_rhs_tiles(self, variant, persist):
+        """The RHS variant is the last direction's; the other directions' and the
+        persistence factors are checked and kept, and have no effect."""
         v = (C.c_int * 3)(*variant)
         p = (C.c_int * 3)(*persist)
         self._call("set_rhs_tiles", v, p)
