@@ -195,7 +195,10 @@ __device__ __forceinline__ R on_all_lanes(R v) {
 // between the species' t_mid).  It chooses where the coefficients are read, never
 // the value: the sums are the same ones in the same order, whatever the other
 // lanes hold.  (A face on the seam of two tiles is formed in both, next to other
-// faces, and its two fluxes have to be the same bits.)
+// faces, and its two fluxes have to be the same bits.)  97x61x75 cells with 9
+// species and temperatures on both sides of t_low: 21.5 ms per 20 FP64 steps; with a
+// sum over the species for the temperatures outside the ranges, beside the
+// polynomial of the others, 22.9.
 constexpr int kRangeAny = 0, kRangeLo = 1, kRangeHi = 2, kRangeEach = 3;
 template <typename R>
 __device__ __forceinline__ int thermo_range(SpeciesPtrT<R> sp, R t0, R t1) {

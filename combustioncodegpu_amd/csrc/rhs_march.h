@@ -26,9 +26,9 @@
 // metric, transport and dq arrays were read or rewritten by every pass, and
 // the passes waited for their staged batches (VALU busy 45% of a SIMD's
 // cycles).  256x128x128 cells, 9 species, per evaluation: FP64 2.44 -> 1.12
-// ms, mixed 1.15 -> 0.57 ms; 11.1 -> 2.0 GB through HBM in FP64.
+// ms, mixed 1.15 -> 0.58 ms; 11.1 -> 2.0 GB through HBM in FP64.
 //
-// What bounds it now is the vector ALU: about 1300 instructions per face, and
+// What bounds it now is the vector ALU: about 1350 instructions per face, and
 // in FP64 seven wavefronts of faces on four SIMDs (the planes and fluxes of
 // 9 species fill the LDS, so a larger tile does not fit).
 #pragma once
